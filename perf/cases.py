@@ -1,0 +1,549 @@
+"""The work that programs built on this library spend their time in, as cases to be timed.
+
+The library serves quantised LLM inference: MXFP4 linears, a paged fp8 or bf16 KV cache, one token
+per sequence in decode and packed prompts in prefill.  The cases cover each of its paths from the
+smallest call to the largest, with the ragged lengths, odd batch sizes and block tables that a
+serving engine hands over:
+
+  * ``matvec``         one linear of a decode step, 1..16 rows (``ops.h4mv``);
+  * ``linear``         one linear of a larger batch or a prompt, 17 rows and more
+                       (``ops.mxfp4_linear``: activation quantiser and GEMM);
+  * ``decode``         paged decode attention over fp8 or bf16 caches (``ops.decode_attention``);
+  * ``prefill``        causal attention of one prompt or of several packed ones, after cached tokens
+                       or without (``ops.prefill_attention``, ``ops.prefill_attention_varlen``);
+  * ``lm_head``        draft logits with top-k, and the exact rerank of the candidates;
+  * ``decode_step``    layers and logits of a decode step, replayed from a HIP graph as an engine
+                       replays it;
+  * ``prefill_layer``  one layer of a prompt: norms, quantised linears, cache write, attention, SiLU.
+
+Caches have the engine's layout: one [blocks, kv heads, block size, 2 D] tensor with K and V side
+by side, read through strided views.  All sizes follow from the case alone, all values from the seed.
+"""
+import math
+import os
+import random
+import sys
+
+import torch
+
+_PKG = os.path.join(os.getcwd(), "gfx1201-tuning-log_amd")
+if _PKG not in sys.path:
+    sys.path.insert(0, _PKG)
+
+from fp8kv_amd import ops  # noqa: E402
+
+D = 128                       # head size
+E4M3_MAX = 448.0
+EPS = 1e-6
+VOCAB = 128167
+# one layer: hidden size, MLP width, query and kv heads, and its four linears (name: N, K)
+HIDDEN, MLP, HQ, HKV = 3584, 18944, 24, 4
+LAYER = {"qkv": ((HQ + 2 * HKV) * D, HIDDEN), "o": (HIDDEN, HQ * D), "gate_up": (2 * MLP, HIDDEN),
+         "down": (HIDDEN, MLP)}
+NORMS = ("norm1", "norm2")
+# what a residual stream carries is many times what one layer adds to it
+STREAM = 16
+MATVEC_MAX_M, SILU_MAX_M = 16, 8      # rows that ops.h4mv and ops.h4mv_silu_mul take
+
+
+# ------------------------------------------------------------------------------ the cases
+
+def listed():
+    return [
+        # the largest linear of a single-stream decode step
+        {"name": "matvec_m1", "op": "matvec", "N": 28672, "K": 4096, "M": 1},
+        # eight concurrent sequences through the MLP's down projection (long rows, few of them)
+        {"name": "matvec_m8_down", "op": "matvec", "N": 3584, "K": 18944, "M": 8},
+        # a busy server's decode batch through the qkv projection, per-token fp8 activations
+        {"name": "linear_m96_qkv", "op": "linear", "N": 4096, "K": 3584, "M": 96, "act": "token"},
+        # a whole prompt through the widest linear, MXFP8 activations
+        {"name": "linear_m2048_gate_up", "op": "linear", "N": 37888, "K": 3584, "M": 2048, "act": "mx"},
+        # the smallest call: one short conversation
+        {"name": "decode_b1_short", "op": "decode", "seqs": 1, "lo": 777, "hi": 777, "heads": 24,
+         "kv_heads": 4, "block": 16, "dtype": "fp8"},
+        # many sequences with long, unequal contexts over a bf16 cache
+        {"name": "decode_b32_bf16", "op": "decode", "seqs": 32, "lo": 512, "hi": 8192, "heads": 32,
+         "kv_heads": 8, "block": 16, "dtype": "bf16"},
+        # the second chunk of a long prompt
+        {"name": "prefill_2048_after_2048", "op": "prefill", "seqs": 1, "lo": 2048, "hi": 2048,
+         "cached": 2048, "heads": 24, "kv_heads": 4, "block": 16, "dtype": "fp8"},
+        # several prompts of unequal length that arrived together, sharing short cached prefixes
+        {"name": "prefill_varlen_6", "op": "prefill", "seqs": 6, "lo": 37, "hi": 900, "cached": 200,
+         "heads": 24, "kv_heads": 4, "block": 16, "dtype": "fp8"},
+        # a prompt over a bf16 cache
+        {"name": "prefill_1500_bf16", "op": "prefill", "seqs": 1, "lo": 1500, "hi": 1500, "cached": 0,
+         "heads": 24, "kv_heads": 4, "block": 16, "dtype": "bf16"},
+        # the end of a decode step: draft logits, top-k, exact rerank
+        {"name": "lm_head_m4", "op": "lm_head", "N": VOCAB, "K": HIDDEN, "M": 4, "k": 64},
+        # a decode step of eight sequences, cut to two layers, with its logits
+        {"name": "decode_step_b8", "op": "decode_step", "seqs": 8, "lo": 1024, "hi": 4096, "layers": 2},
+        # one layer of a prompt of odd length after a cached prefix
+        {"name": "prefill_layer_1000", "op": "prefill_layer", "new": 1000, "cached": 500},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def _heads(rng):
+    return rng.choice([(24, 4), (24, 4), (32, 8), (32, 8), (28, 4), (16, 2), (16, 16), (48, 8)])
+
+
+def draw(rng):
+    op = rng.choice(["matvec", "linear", "linear", "decode", "decode", "prefill", "prefill", "prefill",
+                     "lm_head", "decode_step", "prefill_layer"])
+    shapes = list(LAYER.values()) + [(28672, 4096)]
+    if op == "matvec":
+        n, k = rng.choice(shapes) if rng.random() < 0.5 else (_log_int(rng, 256, 40000), 32 * _log_int(rng, 16, 592))
+        return {"op": op, "N": n, "K": k, "M": rng.randint(1, 16)}
+    if op == "linear":
+        n, k = rng.choice(shapes) if rng.random() < 0.6 else (4 * _log_int(rng, 64, 9000), 128 * _log_int(rng, 4, 148))
+        most = min(4096, int(2.7e11 / (n * k)))
+        return {"op": op, "N": n, "K": k, "M": _log_int(rng, 17, max(most, 64)), "act": rng.choice(["mx", "token"])}
+    if op == "decode":
+        heads, kv = _heads(rng)
+        dtype = rng.choice(["fp8", "fp8", "bf16"])
+        seqs = _log_int(rng, 1, 64)
+        most = min(32768, int(2.5e8 / (2 * D * kv * (2 if dtype == "bf16" else 1)) / seqs))
+        hi = _log_int(rng, 64, most)
+        return {"op": op, "seqs": seqs, "lo": rng.randint(max(1, hi // 8), hi), "hi": hi, "heads": heads,
+                "kv_heads": kv, "block": rng.choice([16, 16, 32, 64, 128]), "dtype": dtype}
+    if op == "prefill":
+        heads, kv = _heads(rng)
+        seqs = rng.choice([1, 1, 2, 3, 5, 8, 12])
+        hi = _log_int(rng, 64, 2048 if seqs == 1 else 5000 // seqs)
+        cached = rng.choice([0, 0, _log_int(rng, 16, 4096 // seqs)])
+        return {"op": op, "seqs": seqs, "lo": rng.randint(max(1, hi // 8), hi) if seqs > 1 else hi, "hi": hi,
+                "cached": cached, "heads": heads, "kv_heads": kv, "block": rng.choice([16, 16, 32, 64]),
+                "dtype": rng.choice(["fp8", "fp8", "bf16"])}
+    if op == "lm_head":
+        return {"op": op, "N": rng.choice([VOCAB, 32000, _log_int(rng, 8000, 128000)]), "K": HIDDEN,
+                "M": rng.randint(1, 16), "k": rng.choice([1, 8, 20, 64])}
+    if op == "decode_step":
+        hi = _log_int(rng, 128, 8192)
+        return {"op": op, "seqs": rng.choice([1, 2, 3, 4, 6, 8, 11, 16, 24, 40]), "lo": max(1, hi // 3), "hi": hi,
+                "layers": rng.choice([1, 2])}
+    return {"op": op, "new": _log_int(rng, 65, 2048), "cached": rng.choice([0, _log_int(rng, 16, 2048)])}
+
+
+def _lengths(case):
+    """Sequence lengths from `lo` to `hi`, both of them present, in an order of no kind."""
+    n, lo, hi = case["seqs"], case["lo"], case["hi"]
+    if n == 1:
+        return [hi]
+    got = [lo + (hi - lo) * i // (n - 1) for i in range(n)]
+    random.Random(n * 1000003 + hi).shuffle(got)
+    return got
+
+
+# ------------------------------------------------------------------------------ inputs
+
+def _generator(seed):
+    return torch.Generator(device="cuda").manual_seed(seed)
+
+
+def _normal(g, *shape):
+    return torch.randn(*shape, device="cuda", generator=g).to(torch.bfloat16)
+
+
+def _weight(g, n, k, low=119):
+    """An MXFP4 checkpoint tensor: codes [N, K/2] over all values, scale bytes [K/32, N] from `low` up."""
+    return (torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device="cuda", generator=g),
+            torch.randint(low, low + 5, (k // 32, n), dtype=torch.uint8, device="cuda", generator=g))
+
+
+def _cache(g, ctx, kv_heads, block, dtype):
+    """Pool, K and V views, scales and block table of sequences of `ctx` tokens: blocks handed out in
+    no order, K and V ~ N(0, 1), fp8 caches quantised with one scale each."""
+    need = [-(-c // block) for c in ctx]
+    nb = sum(need)
+    shape = (nb, kv_heads, block, 2 * D)
+    if dtype == "bf16":
+        pool, scales = torch.empty(shape, dtype=torch.bfloat16, device="cuda"), []
+        for h in range(2):
+            pool[..., h * D:(h + 1) * D] = torch.randn(shape[:3] + (D,), device="cuda", generator=g)
+            scales.append(torch.ones(1, device="cuda"))
+    else:
+        pool, scales = torch.empty(shape, dtype=torch.uint8, device="cuda"), []
+        for h in range(2):
+            x = torch.randn(shape[:3] + (D,), device="cuda", generator=g)
+            s = (x.abs().max() / E4M3_MAX).reshape(1)
+            pool[..., h * D:(h + 1) * D] = (x / s).clamp(-E4M3_MAX, E4M3_MAX).to(torch.float8_e4m3fn).view(torch.uint8)
+            scales.append(s)
+    ids = torch.randperm(nb, device="cuda", generator=g).to(torch.int32)
+    table = torch.zeros(len(ctx), max(need), dtype=torch.int32, device="cuda")
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = ids[at:at + n]
+        at += n
+    return {"pool": pool, "k_scale": scales[0], "v_scale": scales[1], "table": table, "block": block}
+
+
+def _views(pool):
+    k, v = pool.transpose(1, 2).split(D, dim=-1)
+    return (k, v) if pool.dtype == torch.bfloat16 else (k.view(torch.float8_e4m3fn), v.view(torch.float8_e4m3fn))
+
+
+def _i32(values):
+    return torch.tensor(values, dtype=torch.int32, device="cuda")
+
+
+def _starts(lengths):
+    got = [0]
+    for n in lengths:
+        got.append(got[-1] + n)
+    return got
+
+
+def _slots(cache, positions):
+    """Slot of (sequence, position) pairs in the cache."""
+    seq, pos = (torch.tensor(v, dtype=torch.int64, device="cuda") for v in zip(*positions))
+    b = cache["block"]
+    return cache["table"].long()[seq, pos // b] * b + pos % b
+
+
+def _layer_weights(g):
+    w = {name: _weight(g, n, k, 117) for name, (n, k) in LAYER.items()}      # standard deviation about 0.02
+    for name in NORMS:
+        w[name] = (0.4 + 0.6 * torch.rand(HIDDEN, device="cuda", generator=g)).to(torch.bfloat16)
+    return w
+
+
+def _inputs(case, seed):
+    """Everything that the seed decides, made with torch alone."""
+    g, op = _generator(seed), case["op"]
+    if op in ("matvec", "linear"):
+        w = _weight(g, case["N"], case["K"])
+        return {"w": w, "x": _normal(g, case["M"], case["K"])}
+    if op == "decode":
+        ctx = _lengths(case)
+        return {"cache": _cache(g, ctx, case["kv_heads"], case["block"], case["dtype"]), "ctx": ctx,
+                "q": _normal(g, len(ctx), case["heads"], D)}
+    if op == "prefill":
+        new = _lengths(case)
+        ctx = [n + case["cached"] for n in new]
+        return {"cache": _cache(g, ctx, case["kv_heads"], case["block"], case["dtype"]), "ctx": ctx, "new": new,
+                "q": _normal(g, sum(new), case["heads"], D)}
+    if op == "lm_head":
+        return {"w": _weight(g, case["N"], case["K"]), "x": _normal(g, case["M"], case["K"]),
+                "embedding": _normal(g, case["N"], case["K"])}
+    if op == "decode_step":
+        ctx = _lengths(case)
+        return {"ctx": ctx, "layers": [(_layer_weights(g), _cache(g, ctx, HKV, 16, "fp8")) for _ in range(case["layers"])],
+                "norm": (0.5 + torch.rand(HIDDEN, device="cuda", generator=g)).to(torch.bfloat16),
+                "head": _weight(g, VOCAB, HIDDEN), "x": STREAM * _normal(g, len(ctx), HIDDEN)}
+    ctx = [case["new"] + case["cached"]]
+    return {"ctx": ctx, "layers": [(_layer_weights(g), _cache(g, ctx, HKV, 16, "fp8"))], "x": _normal(g, case["new"], HIDDEN),
+            "residual": STREAM * _normal(g, case["new"], HIDDEN),
+            "norm": (0.5 + torch.rand(HIDDEN, device="cuda", generator=g)).to(torch.bfloat16)}
+
+
+# ------------------------------------------------------------------------------ the library's work
+
+def _loaded(w):
+    """A checkpoint tensor as the matvec and the GEMM take it."""
+    return w[0], ops.repack_scales(w[1])
+
+
+def _linear(x, w):
+    """A linear as the engine routes it: the matvec for small batches, the GEMM for others."""
+    return ops.h4mv(x, *w) if x.shape[0] <= MATVEC_MAX_M else ops.mxfp4_linear(x, *w, act="token")
+
+
+def prepare(case, seed):
+    case = dict(case)
+    s = _inputs(case, seed)
+    s["op"], s["case"] = case["op"], case
+    op = case["op"]
+    if op in ("matvec", "linear", "lm_head"):
+        s["w"] = _loaded(s["w"])
+    if op == "matvec":
+        s["out"] = torch.empty(case["M"], case["N"], dtype=torch.bfloat16, device="cuda")
+    if op in ("decode", "prefill"):
+        s["k"], s["v"] = _views(s["cache"]["pool"])
+        s["out"] = torch.zeros_like(s["q"])
+        s["lens"] = _i32(s["ctx"])
+        s["starts"] = _i32(_starts(s["new"] if op == "prefill" else [1] * len(s["ctx"])))
+    if op in ("decode_step", "prefill_layer"):
+        loaded = []
+        for w, cache in s["layers"]:
+            lw = {n: _loaded(w[n]) for n in LAYER}
+            lw.update((n, w[n]) for n in NORMS)
+            if op == "decode_step" and len(s["ctx"]) <= SILU_MAX_M:
+                lw["gate_up"] = ops.interleave_gate_up(*lw["gate_up"])
+            loaded.append((lw, cache) + _views(cache["pool"]))
+        s["layers"] = loaded
+        s["lens"] = _i32(s["ctx"])
+        cache = loaded[0][1]
+        if op == "decode_step":
+            s["head"] = _loaded(s["head"])
+            s["starts"] = _i32(range(len(s["ctx"]) + 1))
+            s["residual"] = torch.zeros_like(s["x"])
+            s["slots"] = [_slots(layer[1], [(i, c - 1) for i, c in enumerate(s["ctx"])]) for layer in loaded]
+            _capture(s)
+        else:
+            s["slots"] = [_slots(cache, [(0, case["cached"] + i) for i in range(case["new"])])]
+    return s
+
+
+def _attend_and_mlp(s, i, x, residual, attention):
+    """One layer: both norms, the four linears, the cache write and `attention` of query and layer."""
+    lw, cache, k, v = s["layers"][i]
+    t = x.shape[0]
+    x = ops.fused_add_rmsnorm(x, residual, lw["norm1"], EPS)
+    qkv = _linear(x, lw["qkv"])
+    q, key, value = qkv.split([HQ * D, HKV * D, HKV * D], dim=1)
+    ops.cache_write(key.view(t, HKV, D), value.view(t, HKV, D), k, v, s["slots"][i], cache["k_scale"], cache["v_scale"])
+    o = attention(q.view(t, HQ, D), cache, k, v)
+    x = ops.fused_add_rmsnorm(_linear(o.view(t, HQ * D), lw["o"]), residual, lw["norm2"], EPS)
+    if s["op"] == "decode_step" and t <= SILU_MAX_M:
+        x = ops.h4mv_silu_mul(x, *lw["gate_up"])
+    else:
+        x = ops.silu_mul(_linear(x, lw["gate_up"]))
+    return _linear(x, lw["down"])
+
+
+def _decode_step(s):
+    residual = s["residual"]
+    residual.zero_()
+    x = s["x"]
+
+    def attention(q, cache, k, v):
+        return ops.decode_attention(q, k, v, torch.empty(q.shape, dtype=q.dtype, device=q.device), s["starts"],
+                                    s["lens"], cache["table"], cache["k_scale"], cache["v_scale"],
+                                    1 / math.sqrt(D), max_seq_len=max(s["ctx"]))
+
+    for i in range(len(s["layers"])):
+        x = _attend_and_mlp(s, i, x, residual, attention)
+    x = ops.fused_add_rmsnorm(x, residual, s["norm"], EPS)
+    if x.shape[0] <= MATVEC_MAX_M:
+        logits = ops.h4mv(x, *s["head"], out_dtype=torch.float32)
+    else:                                     # VOCAB is no multiple of 4, which the GEMM needs
+        logits = torch.cat([ops.h4mv(r, *s["head"], out_dtype=torch.float32) for r in x.split(MATVEC_MAX_M)])
+    return {"logits": logits, "residual": residual, "caches": [layer[1]["pool"] for layer in s["layers"]]}
+
+
+def _capture(s):
+    """The step recorded as an engine records it: once eagerly, then into a graph."""
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    s["graph"] = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        _decode_step(s)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(s["graph"], stream=stream):
+            s["result"] = _decode_step(s)
+    torch.cuda.current_stream().wait_stream(stream)
+
+
+def run(s):
+    op = s["op"]
+    if op == "matvec":
+        return ops.h4mv(s["x"], *s["w"], out=s["out"])
+    if op == "linear":
+        return ops.mxfp4_linear(s["x"], *s["w"], act=s["case"]["act"])
+    if op == "decode":
+        c = s["cache"]
+        return ops.decode_attention(s["q"], s["k"], s["v"], s["out"], s["starts"], s["lens"], c["table"],
+                                    c["k_scale"], c["v_scale"], 1 / math.sqrt(D), max_seq_len=max(s["ctx"]))
+    if op == "prefill":
+        c = s["cache"]
+        if len(s["new"]) == 1:
+            return ops.prefill_attention(s["q"], s["k"], s["v"], s["out"], c["table"], c["k_scale"], c["v_scale"],
+                                         1 / math.sqrt(D), s["case"]["cached"], s["new"][0])
+        return ops.prefill_attention_varlen(s["q"], s["k"], s["v"], s["out"], s["starts"], s["lens"], c["table"],
+                                            c["k_scale"], c["v_scale"], 1 / math.sqrt(D),
+                                            max_query_len=max(s["new"]))
+    if op == "lm_head":
+        draft, candidates = ops.lm_head_topk(s["x"], *s["w"], s["case"]["k"])
+        scores, order = ops.rerank_exact(s["embedding"], s["x"], candidates)
+        return {"draft": draft, "candidates": candidates, "scores": scores, "order": order}
+    if op == "decode_step":
+        s["graph"].replay()
+        return s["result"]
+    new, cached = s["case"]["new"], s["case"]["cached"]
+    residual = s["residual"].clone()
+
+    def attention(q, cache, k, v):
+        return ops.prefill_attention(q, k, v, torch.empty(q.shape, dtype=q.dtype, device=q.device), cache["table"],
+                                     cache["k_scale"], cache["v_scale"], 1 / math.sqrt(D), cached, new)
+
+    x = _attend_and_mlp(s, 0, s["x"], residual, attention)
+    x = ops.fused_add_rmsnorm(x, residual, s["norm"], EPS)        # what the next layer starts with
+    return {"x": x, "residual": residual, "cache": s["layers"][0][1]["pool"]}
+
+
+# ------------------------------------------------------------------------------ what it has to do
+
+def _linear_work(n, k, m, out=2):
+    return n * k // 2 + n * k // 32 + 2 * m * k + out * m * n, 2 * n * k * m
+
+
+def _decode_work(ctx, heads, kv_heads, block, size):
+    return (sum(ctx) * kv_heads * 2 * D * size + 4 * len(ctx) * heads * D + 4 * sum(-(-c // block) for c in ctx),
+            4 * sum(ctx) * heads * D)
+
+
+def _prefill_work(new, cached, heads, kv_heads, block, size):
+    pairs = sum(n * cached + n * (n + 1) // 2 for n in new)
+    return (sum(n + cached for n in new) * kv_heads * 2 * D * size + 4 * sum(new) * heads * D
+            + 4 * sum(-(-(n + cached) // block) for n in new), 4 * pairs * heads * D)
+
+
+def work(case):
+    op = case["op"]
+    if op in ("matvec", "linear"):
+        b, f = _linear_work(case["N"], case["K"], case["M"])
+    elif op == "decode":
+        b, f = _decode_work(_lengths(case), case["heads"], case["kv_heads"], case["block"], 2 if case["dtype"] == "bf16" else 1)
+    elif op == "prefill":
+        b, f = _prefill_work(_lengths(case), case["cached"], case["heads"], case["kv_heads"], case["block"],
+                             2 if case["dtype"] == "bf16" else 1)
+    elif op == "lm_head":
+        m, k, c = case["M"], case["K"], case["k"]
+        b, f = _linear_work(case["N"], k, m, 0)
+        b, f = b + 2 * m * c * k + 16 * m * c, f + 2 * m * c * k
+    else:
+        decode = op == "decode_step"
+        ctx = _lengths(case) if decode else [case["new"] + case["cached"]]
+        t = len(ctx) if decode else case["new"]
+        # a layer reads its weights and cache once and writes the new rows of the cache; what passes from
+        # one of its kernels to the next could stay on the chip
+        b = sum(n * k // 2 + n * k // 32 for n, k in LAYER.values()) + t * HKV * 2 * D
+        f = sum(2 * n * k * t for n, k in LAYER.values())
+        a = _decode_work(ctx, HQ, HKV, 16, 1) if decode else _prefill_work([t], case["cached"], HQ, HKV, 16, 1)
+        b, f = b + a[0] - 4 * t * HQ * D, f + a[1]
+        if decode:
+            h = _linear_work(VOCAB, HIDDEN, t, 4)
+            b, f = b * case["layers"] + h[0] + 2 * t * HIDDEN, f * case["layers"] + h[1]
+        else:
+            b += 4 * 2 * t * HIDDEN                    # x and residual in, both out
+    return {"bytes": b, "flops": f}
+
+
+def tolerance(case):
+    """About four times the error that each path shows against 64 bits."""
+    op = case["op"]
+    if op in ("matvec", "linear"):
+        return {"rel": 7e-3}                        # one rounding to bf16: 1.7e-3
+    if op in ("decode", "prefill"):
+        return {"rel": 9e-3}                        # probabilities and result in bf16: 2.3e-3
+    if op == "lm_head":
+        return {"rel": 4e-6, "differ": 0.01}        # logits in fp32: 9e-7; candidates closer than that may change places
+    return {"rel": 1.2e-2, "differ": 0.005}         # bf16 between the kernels, fp8 activations and cache: 3.2e-3
+
+
+# ------------------------------------------------------------------------------ the same in 64 bits
+
+_E2M1 = (0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0)
+
+
+def _dequantised(w):
+    codes, scales = w
+    table = torch.tensor(_E2M1 + tuple(-v for v in _E2M1), dtype=torch.float64, device="cuda")
+    n, half = codes.shape
+    x = torch.stack((table[(codes & 15).long()], table[(codes >> 4).long()]), dim=-1).view(n, half // 16, 32)
+    return (x * torch.exp2(scales.t().double() - 127).unsqueeze(-1)).view(n, 2 * half)
+
+
+def _product(x, w, rows=16384):
+    """x . dequant(w)^T, some rows of the weight at a time."""
+    return torch.cat([x @ _dequantised((w[0][i:i + rows], w[1][:, i:i + rows])).t() for i in range(0, w[0].shape[0], rows)], dim=1)
+
+
+def _quantised(x, act):
+    """bf16 activations after the quantiser of the GEMM path, as numbers."""
+    if act == "token":
+        scale = (x.float().abs().amax(dim=1, keepdim=True) / E4M3_MAX).clamp(min=1 / (E4M3_MAX * 512))
+        q = (x.float() / scale).clamp(-E4M3_MAX, E4M3_MAX).to(torch.float8_e4m3fn)
+        return q.double() * scale.double()
+    blocks = x.float().view(x.shape[0], -1, 32)
+    amax = blocks.abs().amax(dim=2, keepdim=True)
+    e = (torch.frexp(amax)[1] - 9).clamp(min=-127).double()
+    q = (blocks.double() / torch.exp2(e)).clamp(-E4M3_MAX, E4M3_MAX).float().to(torch.float8_e4m3fn)
+    return (q.double() * torch.exp2(e)).view(x.shape)
+
+
+def _rows(cache, i, n):
+    """K and V [n, kv heads, D] of sequence i."""
+    pool, b = cache["pool"], cache["block"]
+    t = torch.arange(n, device="cuda")
+    x = pool[cache["table"][i].long()[t // b], :, t % b]
+    k, v = x.split(D, dim=-1)
+    if pool.dtype == torch.bfloat16:
+        return k.double(), v.double()
+    return (k.view(torch.float8_e4m3fn).double() * cache["k_scale"].double(),
+            v.view(torch.float8_e4m3fn).double() * cache["v_scale"].double())
+
+
+def _attended(q, cache, new, ctx):
+    """Causal attention of packed queries (`new` of each sequence, its last tokens)."""
+    out, at = [], 0
+    for i, (n, c) in enumerate(zip(new, ctx)):
+        k, v = _rows(cache, i, c)
+        group = q.shape[1] // k.shape[1]
+        mask = torch.arange(c, device="cuda")[None, :] > torch.arange(c - n, c, device="cuda")[:, None]
+        heads = []
+        for h in range(q.shape[1]):
+            s = (q[at:at + n, h].double() @ k[:, h // group].t()) / math.sqrt(D)
+            heads.append(torch.softmax(s.masked_fill(mask, float("-inf")), dim=-1) @ v[:, h // group])
+        out.append(torch.stack(heads, dim=1))
+        at += n
+    return torch.cat(out)
+
+
+def _norm(x, residual, weight):
+    """(normed bf16, new residual bf16), both rounded where the library hands them on."""
+    z = x.double() + residual.double()
+    r = torch.rsqrt((z * z).mean(dim=1, keepdim=True) + EPS)
+    return ((z * r).to(torch.bfloat16).double() * weight.double()).to(torch.bfloat16), z.to(torch.bfloat16)
+
+
+def _exact_linear(x, w, rounded=True):
+    y = _product(x.double() if x.shape[0] <= MATVEC_MAX_M else _quantised(x, "token"), w)
+    return y.to(torch.bfloat16) if rounded else y
+
+
+def _exact_layer(s, i, x, residual, new):
+    w, cache = s["layers"][i]
+    x, residual = _norm(x, residual, w["norm1"])
+    q, key, value = _exact_linear(x, w["qkv"]).split([HQ * D, HKV * D, HKV * D], dim=1)
+    seqs = [(j, c - n + t) for j, (n, c) in enumerate(zip(new, s["ctx"])) for t in range(n)]
+    slots = _slots(cache, seqs)
+    for h, (y, scale) in enumerate(((key, cache["k_scale"]), (value, cache["v_scale"]))):
+        y = (y.float() / scale).clamp(-E4M3_MAX, E4M3_MAX).to(torch.float8_e4m3fn).view(torch.uint8)
+        b = cache["block"]
+        cache["pool"][slots // b, :, slots % b, h * D:(h + 1) * D] = y.view(-1, HKV, D)
+    o = _attended(q.reshape(-1, HQ, D), cache, new, s["ctx"]).to(torch.bfloat16)
+    x, residual = _norm(_exact_linear(o.view(-1, HQ * D), w["o"]), residual, w["norm2"])
+    gate, up = _exact_linear(x, w["gate_up"]).double().split(MLP, dim=1)
+    x = (gate / (1 + torch.exp(-gate)) * up).to(torch.bfloat16)
+    return _exact_linear(x, w["down"], rounded=False), residual
+
+
+def exact(case, seed):
+    s, op = _inputs(dict(case), seed), case["op"]
+    if op == "matvec":
+        return _product(s["x"].double(), s["w"])
+    if op == "linear":
+        return _product(_quantised(s["x"], case["act"]), s["w"])
+    if op == "decode":
+        return _attended(s["q"], s["cache"], [1] * len(s["ctx"]), s["ctx"])
+    if op == "prefill":
+        return _attended(s["q"], s["cache"], s["new"], s["ctx"])
+    if op == "lm_head":
+        x = s["x"].double()
+        draft, candidates = torch.topk(_product(x, s["w"]), case["k"])
+        scores = (s["embedding"][candidates].double() @ x.unsqueeze(-1)).squeeze(-1)
+        return {"draft": draft, "candidates": None, "scores": scores.sort(dim=1, descending=True)[0], "order": None}
+    x = s["x"]
+    if op == "prefill_layer":
+        x, residual = _exact_layer(s, 0, x, s["residual"], [case["new"]])
+        x, residual = _norm(x.to(torch.bfloat16), residual, s["norm"])
+        return {"x": x.double(), "residual": residual.double(), "cache": None}
+    residual = torch.zeros_like(x)
+    for i in range(case["layers"]):
+        x, residual = _exact_layer(s, i, x.to(torch.bfloat16), residual, [1] * len(s["ctx"]))
+    x, residual = _norm(x.to(torch.bfloat16), residual, s["norm"])
+    return {"logits": _product(x.double(), s["head"]), "residual": residual.double(), "caches": None}
