@@ -124,7 +124,7 @@ def draw(rng):
         hi = _log_int(rng, 128, 8192)
         return {"op": op, "seqs": rng.choice([1, 2, 3, 4, 6, 8, 11, 16, 24, 40]), "lo": max(1, hi // 3), "hi": hi,
                 "layers": rng.choice([1, 2])}
-    return {"op": op, "new": _log_int(rng, 65, 2048), "cached": rng.choice([0, _log_int(rng, 16, 2048)])}
+    return {"op": op, "new": _log_int(rng, 65, 1100), "cached": rng.choice([0, _log_int(rng, 16, 2048)])}
 
 
 def _lengths(case):
