@@ -190,46 +190,110 @@ merge_topk_kernel(const uint64_t* __restrict__ cand, int ncand, int k, float* __
     }
 }
 
-// grid (M): C candidate rows of E rescored against X[m] (fp32 dot products of bf16 rows, one wave
-// per candidate, lanes over 8-element pieces), then sorted in rank order.
-__global__ void __launch_bounds__(kThreads)
+// Dot product of a candidate's embedding row with the activation row over one wave (bf16 products
+// summed in fp32, 8-element piece p on lane p % 64, pieces in order, then a butterfly over the
+// lanes).  The loads of kRowBatch pieces per lane go out together - one row of 3584 is 7 - because a
+// row is a random 7 KB of a table far above the caches, and a load per iteration would pay its full
+// round trip every time.  Pieces past the row re-read its last one and count as zero.
+constexpr int kRowBatch = 8;
+
+__device__ __forceinline__ float row_score(const __bf16* x, const __bf16* e, int pieces, int lane)
+{
+    float acc = 0.f;
+    for (int p0 = 0; p0 < pieces; p0 += 64 * kRowBatch) {
+        u32x4_t a[kRowBatch], b[kRowBatch];
+#pragma unroll
+        for (int i = 0; i < kRowBatch; ++i) {
+            const int p = min(p0 + 64 * i + lane, pieces - 1);
+            b[i] = load_nt_16(e + 8 * p);
+            a[i] = load_16(x + 8 * p);
+        }
+#pragma unroll
+        for (int i = 0; i < kRowBatch; ++i) {
+            if (p0 + 64 * i + lane >= pieces) a[i] = b[i] = (u32x4_t){0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                acc = __builtin_fmaf(__uint_as_float(a[i][w] << 16), __uint_as_float(b[i][w] << 16), acc);
+                acc = __builtin_fmaf(__uint_as_float(a[i][w] & 0xffff0000u),
+                                     __uint_as_float(b[i][w] & 0xffff0000u), acc);
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s);
+    return acc;
+}
+
+// Writes row m's candidates at their positions in rank order; thread t holds candidate t's key
+// (0: invalid) in keys[t], published by a barrier.  A position is the number of keys ranked above
+// it, plus equal keys earlier in the list (repeated indices, and the zero keys of invalid
+// candidates, keep their candidate order).
+__device__ __forceinline__ void write_ranked(const uint64_t* keys, int C, int m, float* out_val, int32_t* out_idx)
+{
+    const int tid = threadIdx.x;
+    if (tid >= C) return;
+    const uint64_t mine = keys[tid];
+    int rank = 0;
+    for (int j = 0; j < C; ++j) rank += (keys[j] > mine || (keys[j] == mine && j < tid)) ? 1 : 0;
+    out_val[(size_t)m * C + rank] = mine ? key_value(mine) : -__builtin_inff();
+    out_idx[(size_t)m * C + rank] = mine ? key_index(mine) : -1;
+}
+
+// Exact rerank of C candidate rows of E against X[m].  The reads are M * C rows at random addresses,
+// so latency bounds it, and one workgroup per row of X leaves nearly all CUs idle.  Up to
+// kRerankOneMaxC candidates: one launch, grid (M), a wave per candidate.  More: rerank_score_kernel
+// gives every candidate of every row its own wave over the whole GPU (the scores wait in out_val),
+// and rerank_order_kernel sorts each row in place.  Measured in a graph, H = 3584, 128167 rows, us
+// per call at M = 1 / 4 / 16: 64 candidates 6.2 / 6.7 / 7.2 in two launches, 16.7 / 17.1 / 17.7 with
+// 16 waves in one, 45 / 63 / 67 with four waves and a load per iteration; 8 candidates at M = 4: 4.2
+// in one launch, 5.2 in two.
+constexpr int kRerankOneMaxC = 16;
+
+__global__ void __launch_bounds__(64 * kRerankOneMaxC)
 rerank_kernel(const __bf16* __restrict__ E, int64_t e_stride, int V, const __bf16* __restrict__ X,
               int64_t x_stride, const int32_t* __restrict__ cand, int C, int H,
               float* __restrict__ out_val, int32_t* __restrict__ out_idx)
 {
+    __shared__ uint64_t keys[kRerankOneMaxC];
+    const int m = blockIdx.x, lane = threadIdx.x & 63;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);        // the grid has a wave per candidate
+    const int32_t idx = cand[(size_t)m * C + c];
+    const bool ok = idx >= 0 && idx < V;
+    const float s = row_score(X + (int64_t)m * x_stride, E + (int64_t)(ok ? idx : 0) * e_stride, H / 8, lane);
+    if (lane == 0) keys[c] = ok ? rank_key(s, (uint32_t)idx) : 0;
+    __syncthreads();
+    write_ranked(keys, C, m, out_val, out_idx);
+}
+
+// grid (ceil(C / 4), min(M, 65535)): the candidates' scores, in candidate order, into out_val.
+__global__ void __launch_bounds__(kThreads)
+rerank_score_kernel(const __bf16* __restrict__ E, int64_t e_stride, int V, const __bf16* __restrict__ X,
+                    int64_t x_stride, const int32_t* __restrict__ cand, int C, int M, int H,
+                    float* __restrict__ out_val)
+{
+    const int lane = threadIdx.x & 63;
+    const int c = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (c >= C) return;
+    for (int m = blockIdx.y; m < M; m += gridDim.y) {
+        const int32_t idx = cand[(size_t)m * C + c];
+        const bool ok = idx >= 0 && idx < V;
+        const float s = row_score(X + (int64_t)m * x_stride, E + (int64_t)(ok ? idx : 0) * e_stride, H / 8, lane);
+        if (lane == 0) out_val[(size_t)m * C + c] = s;
+    }
+}
+
+// grid (M), one wave: row m's scores in out_val and its candidates, sorted in place.
+__global__ void __launch_bounds__(kMaxRerank)
+rerank_order_kernel(const int32_t* cand, int V, int C, float* out_val, int32_t* out_idx)
+{
     __shared__ uint64_t keys[kMaxRerank];
     const int m = blockIdx.x, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const __bf16* x = X + (int64_t)m * x_stride;
-    const int32_t* ci = cand + (size_t)m * C;
-    for (int c = wave; c < C; c += kThreads / 64) {
-        const int32_t idx = ci[c];
-        const bool ok = idx >= 0 && idx < V;
-        const __bf16* e = E + (int64_t)(ok ? idx : 0) * e_stride;
-        float acc = 0.f;
-        for (int p = lane; p < H / 8; p += 64) {
-            const u32x4_t a = *reinterpret_cast<const u32x4_t*>(x + 8 * p);
-            const u32x4_t b = *reinterpret_cast<const u32x4_t*>(e + 8 * p);
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                acc = __builtin_fmaf(__uint_as_float(a[w] << 16), __uint_as_float(b[w] << 16), acc);
-                acc = __builtin_fmaf(__uint_as_float(a[w] & 0xffff0000u), __uint_as_float(b[w] & 0xffff0000u), acc);
-            }
-        }
-#pragma unroll
-        for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s);
-        if (lane == 0) keys[c] = ok ? rank_key(acc, (uint32_t)idx) : 0;
+    if (tid < C) {
+        const int32_t idx = cand[(size_t)m * C + tid];
+        keys[tid] = idx >= 0 && idx < V ? rank_key(out_val[(size_t)m * C + tid], (uint32_t)idx) : 0;
     }
     __syncthreads();
-    if (tid < C) {
-        // Position = keys ranked above this one, plus equal keys earlier in the list (repeated
-        // indices, and the zero keys of invalid candidates, keep their candidate order).
-        const uint64_t mine = keys[tid];
-        int rank = 0;
-        for (int j = 0; j < C; ++j) rank += (keys[j] > mine || (keys[j] == mine && j < tid)) ? 1 : 0;
-        out_val[(size_t)m * C + rank] = mine ? key_value(mine) : -__builtin_inff();
-        out_idx[(size_t)m * C + rank] = mine ? key_index(mine) : -1;
-    }
+    write_ranked(keys, C, m, out_val, out_idx);
 }
 
 inline int nchunks(int N) { return (N + kChunk - 1) / kChunk; }
@@ -288,9 +352,20 @@ extern "C" int fp8kv_rerank_exact(const void* E, int64_t e_row_stride, int V, co
     if (V < 1 || C < 1 || M < 1 || H < 1) return FP8KV_ERR_ARG;
     if (C > kMaxRerank || H % 8 != 0) return FP8KV_ERR_SHAPE;
     if (!aligned(E, 16) || !aligned(X, 16) || (e_row_stride & 7) || (x_row_stride & 7)) return FP8KV_ERR_ALIGN;
+    const __bf16* e = static_cast<const __bf16*>(E);
+    const __bf16* x = static_cast<const __bf16*>(X);
+    const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     begin_launch();
-    launch_kernel(rerank_kernel, dim3((unsigned)M), dim3(kThreads), 0, reinterpret_cast<hipStream_t>(stream),
-                  static_cast<const __bf16*>(E), e_row_stride, V, static_cast<const __bf16*>(X), x_row_stride,
-                  cand_idx, C, H, out_val, out_idx);
+    if (C <= kRerankOneMaxC) {
+        launch_kernel(rerank_kernel, dim3((unsigned)M), dim3(64 * C), 0, st, e, e_row_stride, V, x, x_row_stride,
+                      cand_idx, C, H, out_val, out_idx);
+        return finish_launch();
+    }
+    launch_kernel(rerank_score_kernel, dim3((unsigned)((C + 3) / 4), (unsigned)(M < 65535 ? M : 65535)),
+                  dim3(kThreads), 0, st, e, e_row_stride, V, x, x_row_stride, cand_idx, C, M, H, out_val);
+    const int rc = finish_launch();
+    if (rc != FP8KV_OK) return rc;
+    begin_launch();
+    launch_kernel(rerank_order_kernel, dim3((unsigned)M), dim3(kMaxRerank), 0, st, cand_idx, V, C, out_val, out_idx);
     return finish_launch();
 }

@@ -122,6 +122,25 @@ def test_rerank_exact_against_oracle():
     assert idx[0, -2:].tolist() == [-1, -1]
 
 
+@pytest.mark.parametrize("M,C,H", [(1, 1, 8), (3, 15, 512), (2, 16, 4096), (2, 17, 4096), (1, 33, 4104),
+                                   (5, 64, 520), (65540, 18, 8)])
+def test_rerank_launch_forms(M, C, H):
+    """One launch (C <= 16) and two, a row of one piece, exactly one batch of loads per lane (4096), one
+    piece past it, partial batches, and more rows than a grid's second dimension holds.  The scores
+    are integers that fp32 holds exactly, so values and order are the oracle's."""
+    V = 300
+    g = torch.Generator().manual_seed(M + C + H)
+    E = torch.randint(-4, 5, (V, H), generator=g).to(torch.bfloat16)
+    X = torch.randint(-4, 5, (M, H), generator=g).to(torch.bfloat16)
+    cand = torch.randint(-1, V + 1, (M, C), generator=g, dtype=torch.int32)
+    vals, idx = ops.rerank_exact(E.to(DEV), X.to(DEV), cand.to(DEV))
+    torch.cuda.synchronize()
+    rows = range(M) if M < 100 else list(range(8)) + list(range(M - 8, M))
+    rv, ri = lm_head.rerank(E.float().numpy(), X[list(rows)].float().numpy(), cand[list(rows)].numpy())
+    assert np.array_equal(vals.cpu().numpy()[list(rows)].astype(np.float64), rv)
+    assert np.array_equal(idx.cpu().numpy()[list(rows)], ri)
+
+
 def test_draft_then_rerank_recovers_the_exact_argmax():
     """The chain the reference runs: an approximate head proposes candidates, the exact rows rank
     them.  W is a random MXFP4 head, E = dequant(W) + small bf16 noise: the draft's top 64 holds
