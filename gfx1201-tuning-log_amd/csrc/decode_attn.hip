@@ -470,32 +470,41 @@ constexpr Variant kVariants[] = {{8, 4, 1, false}, {8, 2, 1, false}, {4, 4, 1, f
                                  {8, 2, 2, true},  {8, 2, 2, false}, {8, 2, 1, true}};
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
-// Launch tunables (host state; fp8kv_decode_tune changes them for sweeps).  The default requests
-// each 16-token group's K and V bytes together: against all K of a chunk before its V (variant 4)
-// it runs 0.1-0.3 us shorter per launch on both clocks from b8@1k to b8@8k, and ties at b1@512.
-constexpr int kDefaultVariant = 5;
+// Launch tunables (host state; fp8kv_decode_tune changes them for sweeps).  The default is one
+// chunk of two 16-token groups in flight per wave: at 118 VGPRs two 8-wave workgroups share a CU,
+// and the second one's stream covers the first one's start and merge.  Against two chunks in
+// flight (variant 5, 149 VGPRs, one workgroup per CU; us in a graph, fp8): one sequence of 777 tokens
+// 5.96 / 6.15, of 16000 13.3 / 14.2, 8 of 1024..4096 10.15 / 10.25, 8 of 4096 equal (10.6), 16 of
+// 300..3000 11.1 / 12.8, 64 of 512..4096 36.8 / 37.9.
+constexpr int kDefaultVariant = 1;
 thread_local int g_variant = kDefaultVariant;
 thread_local int g_target_wgs = 256;
 
-// Splits per (sequence, kv head): enough workgroups to reach g_target_wgs (one per CU: at the
-// kernel's register use only one 8-wave workgroup fits on a CU, so a larger grid runs in two
-// rounds), never fewer than one chunk per workgroup, and at most kMaxPlannedSplits, since the
-// merging workgroup reads the split records kMergeBatch at a time.  A wave loops over as many
-// chunk pairs as its span holds.
+// Splits per (sequence, kv head).  Up to g_target_wgs workgroups, as many as fill the GPU (one per
+// CU: at b8@4k 8 splits take 10.6 us, 12 and 16 13.7 and 12.6), but no shorter than pays for the
+// merge: one split up to 256 tokens (200 tokens: 4.7 us in one, 5.4 in two), about 128 tokens each
+// up to 16 splits (777 tokens: 6.0 us in 8, 6.4 in 16), and above 16, where the merge holds 32
+// records, 512 tokens each (4000 tokens: 7.9 us in 16, 9.0 in 32; 16000: 13.3 and 12.1).
+// With a workgroup per CU or more from the pairs alone, the host knows only the longest context.
+// Long ones are split as often as kMaxPlannedRecords allows, because a ragged batch otherwise ends
+// with a few CUs walking its longest sequences (32 sequences of 512..8192, 8 kv heads, in three: 69.6
+// -> 62.0 us, bf16 126 -> 105); shorter ones are not (64 of 512..4096, 4 kv heads: 36.8 us in one,
+// 39.6 in three; 64 of 2048: 24.6 and 30.4).
 constexpr int kMaxPlannedSplits = 32;
+constexpr int kLongContext = 6144;
+// Every planned call fits the library's fixed 8 MiB of scratch at any GQA: 976 records of 16 heads.
+constexpr int kMaxPlannedRecords = 976;
 
 inline int plan_splits(int ns, int hkv, int max_seq_len)
 {
-    if (max_seq_len <= 0) return 1;
-    const Variant v = kVariants[g_variant];
-    const int chunk = 16 * v.ng;
+    if (max_seq_len <= 256) return 1;
     const int pairs = ns * hkv;
-    const int by_fill = (g_target_wgs + pairs - 1) / pairs;                  // fill the GPU
-    const int by_chunks = (max_seq_len + chunk - 1) / chunk;                 // >= 1 chunk per WG
-    int n = by_fill < by_chunks ? by_fill : by_chunks;
-    if (n > kMaxPlannedSplits) n = kMaxPlannedSplits;
-    if (n < 1) n = 1;
-    return n;
+    int n = max_seq_len <= 16 * 128 ? (max_seq_len + 127) / 128
+          : max_seq_len <= 16 * 512 ? 16
+          : max_seq_len / 512 < kMaxPlannedSplits ? (max_seq_len + 511) / 512 : kMaxPlannedSplits;
+    const int by_fill = (g_target_wgs + pairs - 1) / pairs;
+    if (by_fill > 1) return by_fill < n ? by_fill : n;
+    return max_seq_len >= kLongContext && pairs <= kMaxPlannedRecords ? kMaxPlannedRecords / pairs : 1;
 }
 
 // Zero-fill of a decode scratch region (ticket counters and records), a kernel rather than a

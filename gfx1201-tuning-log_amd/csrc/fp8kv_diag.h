@@ -64,8 +64,8 @@ void fp8kv_h4mv_mx_chunk_tune(int steps_log2);
 int fp8kv_h4mv_plan(int N, int K, int M, int* out);
 
 /* Tuning hook for sweeps of the decode attention launch: kernel variant index (0..6; any other
- * value, e.g. -1, selects the default, variant 5: 8 waves, chunks of 2 groups of 16 keys, 2 chunks
- * in flight per wave, each group's K and V bytes requested together) and the workgroup count its split planner
+ * value, e.g. -1, selects the default, variant 1: 8 waves, one chunk of 2 groups of 16 keys in
+ * flight per wave, each group's K and V bytes requested together) and the workgroup count its split planner
  * aims for (0 = default 256).  Affects later launches. */
 void fp8kv_decode_tune(int variant, int target_wgs);
 

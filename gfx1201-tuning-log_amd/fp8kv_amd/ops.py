@@ -74,9 +74,9 @@ _scratch_cache: dict = {}
 # one of them was current replays with its address, so freeing it would hand the graph's tickets
 # and records to whatever the allocator puts there next.
 _scratch_retired: list = []
-# First allocation per device.  The split planner's plans need at most
-# counters (256 KiB) + (2 * 256 - 1) records of 16 * 130 floats (4.25 MB at GQA 16), so a buffer of
-# this size never grows for planned splits; only explicit larger split counts grow it.
+# First allocation per device.  The split planner's plans need at most counters (256 KiB) + 976
+# records of 16 * 130 floats (8.12 MB at GQA 16), so a buffer of this size never grows for planned
+# splits; only explicit larger split counts grow it.
 DECODE_SCRATCH_MIN_BYTES = 8 << 20
 
 

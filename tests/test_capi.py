@@ -119,6 +119,19 @@ def test_decode_split_planner(lib):
         assert 1 <= n <= 256
 
 
+@pytest.mark.parametrize("ns,hkv,ctx,want", [
+    (1, 4, 256, 1), (1, 4, 257, 3), (1, 4, 2048, 16), (1, 4, 2049, 16), (1, 4, 8193, 17), (1, 4, 1 << 30, 32),
+    (8, 4, 300, 3), (63, 4, 4096, 2), (64, 4, 6143, 1), (64, 4, 6144, 3), (122, 8, 1 << 30, 1), (125, 8, 1 << 30, 1)])
+def test_decode_split_plan(lib, ns, hkv, ctx, want):
+    """Both sides of each line of the split rule, and every plan's records within the 8 MiB of the
+    call that takes no scratch, at the widest GQA."""
+    assert lib.fp8kv_decode_num_splits(ns, hkv, ctx) == want
+    for n in range(1, 400):
+        for kv in (1, 3, hkv):
+            splits = lib.fp8kv_decode_num_splits(n, kv, ctx)
+            assert 1 <= splits <= 32 and lib.fp8kv_decode_scratch_bytes(n, 16 * kv, kv, 128, splits) <= 8 << 20
+
+
 # fp8kv_cache_write: every call below is rejected before any HIP call (fake pointers).
 CW_OK = [A, 512, A, 512, A, A, 8192, 512, 128, 8192, 512, 128, A, A, A, 4, 4, 128, 16, None]
 
