@@ -31,13 +31,12 @@
 #include "fp8kv_common.h"
 #include "fp8kv_status.h"
 #include "fp8kv_diag.h"
-#include <utility>
+#include "w4a8_common.h"
 
 namespace fp8kv {
 namespace w4a8_detail {
 
-constexpr int kBN = 128, kBM = 128, kBK = 128;
-constexpr int kXcds = 8;
+constexpr int kBN = 128, kBM = 128;
 
 // 0: the LDS kernel, fragments double-buffered, 4-step ring, one workgroup per CU; 1: the
 // direct-to-register kernel; 2 / 3: as 0 with a 3 / 5-step ring; 4: single-buffered fragments,
@@ -46,8 +45,8 @@ constexpr int kXcds = 8;
 // 8: 8 waves of 8 x 4 tiles (256 x 256 per workgroup, 3-step ring, 150 KB of LDS).  Measured on
 // the configs[4] linears at M = 2048: 6 ~1.22-1.69 PFLOP/s, 5 ~1.27-1.41, 8 ~0.88-1.67 (only
 // gate/up fills the GPU), 7 ~1.05-1.27, 4 ~1.33, 0 ~1.01, 1 ~0.40.
-// Default (-1): variant 6 (the 8 x 4 wave tile, 256 x 128 per workgroup) when its grid has more
-// tiles than the GPU has CUs, else variant 5 (128 x 128, twice the workgroups).  With one
+// Default (-1): the K-splitting kernel where its tiles fit one round (slice_shape); else variant 6 (the
+// 8 x 4 wave tile, 256 x 128 per workgroup) when its grid has more tiles than the GPU has CUs, else variant 5 (128 x 128, twice the workgroups).  With one
 // workgroup per CU, variant 6 has one wave per SIMD and nothing hides its waits.  Measured at
 // M = 2048 (MXFP8, us per launch, variant 5 against 6): 224 tiles of 256 x 128 (down, K = 18944)
 // 150 against 184, 256 tiles (qkv) 36 against 45, 384 tiles 58-59 against 56-57, 512 tiles 68
@@ -55,20 +54,42 @@ constexpr int kXcds = 8;
 constexpr int kDefaultVariant = -1;
 thread_local int g_gemm_variant = kDefaultVariant;
 constexpr int64_t kGemmCus = 256;
+// 9 + s: the K-splitting kernel (w4a8_slice.hip) with tile shape s of kSliceShapes.
+constexpr int kSliceVariant = 9;
+
+// The first slice shape whose tiles all run at once, one per CU, or -1.  In one round the smallest
+// tile that fits is the fastest: its waves have the fewest bytes to fetch (in a graph, per-token
+// activations, us against the 128 x 128 or 256 x 128 kernel; N = 4096, K = 3584: 17 rows 5.2 / 20.1,
+// 64 6.7 / 20.4, 128 8.1 / 21.2, 256 10.7 / 21.4, 512 15.6 / 21.8; N = 3584, K = 18944: 17 rows 16.3 /
+// 104.5, 128 28.2 / 111.8, 512 55.9 / 113.4).  Past one round the larger tiles' smaller traffic wins (N = 37888,
+// K = 3584: 64 rows 38.0 / 32.2; N = 4096: 1000 rows 28.7 / 23.9).
+inline int slice_shape(int N, int K, int M)
+{
+    if (K < kSliceMinK) return -1;
+    for (int s = 0; s < kNumSliceShapes; ++s) {
+        const int bn = 16 * kSliceShapes[s].tn, bm = 16 * kSliceShapes[s].tm;
+        if ((int64_t)((N + bn - 1) / bn) * ((M + bm - 1) / bm) <= kGemmCus) return s;
+    }
+    return -1;
+}
 
 inline int default_variant(int N, int K, int M)
 {
-    (void)K;
+    const int s = slice_shape(N, K, M);
+    if (s >= 0) return kSliceVariant + s;
     const int64_t tiles6 = (int64_t)((N + 255) / 256) * ((M + 127) / 128);
     return tiles6 > kGemmCus ? 6 : 5;
 }
 
-inline int pick_variant(int N, int K, int M) { return g_gemm_variant >= 0 ? g_gemm_variant : default_variant(N, K, M); }
+// A forced slice shape needs kSliceMinK like a planned one.
+inline int pick_variant(int N, int K, int M)
+{
+    const bool forced = g_gemm_variant >= 0 && (g_gemm_variant < kSliceVariant || K >= kSliceMinK);
+    return forced ? g_gemm_variant : default_variant(N, K, M);
+}
 // 0: XCD split by the traffic model of pick_split (default); 1: XCDs split the weight blocks
 // only; 2: XCDs split the token blocks as far as their count allows.
 thread_local int g_gemm_order = 0;
-
-typedef int v8i __attribute__((ext_vector_type(8)));
 
 struct Frags {
     u32x4_t a[4];        // weight n-tile i: 16 bytes (32 e2m1 codes)
@@ -76,41 +97,6 @@ struct Frags {
     uint32_t sa[4];      // scale dword of (row, k step) per n-tile: 4 blocks, this lane's is byte j
     uint32_t sb[4];
 };
-
-__device__ __forceinline__ v8i concat8(u32x4_t lo, u32x4_t hi)
-{
-    return (v8i){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-}
-
-struct Params {
-    const uint8_t* W;
-    const uint8_t* St;
-    const uint8_t* Xq;
-    const uint8_t* Sx;
-    __bf16* Out;
-    const float* tok_scale;   // per-token mode: fp32 scale of each activation row (Sx unused)
-    int N, K, M;
-    int nblk, mblk;
-    int gm, gn;          // tile order: the 8 XCDs split the token blocks gm ways and the weight blocks gn ways
-};
-
-// Tile of workgroup L, or false when L has none.  Workgroup L runs on XCD L % 8 (round-robin
-// dispatch); XCD x = (xm, xn) takes token blocks xm, xm + gm, ... and the xn-th range of weight
-// blocks, weight-block major, so each XCD's L2 holds its share of the activations and the
-// weight tiles it streams are shared by the workgroups running it at the same time.
-__device__ __forceinline__ bool tile_of(const Params& P, int L, int& nb, int& mb)
-{
-    const int x = L % kXcds, slot = L / kXcds;
-    const int xm = x % P.gm, xn = x / P.gm;
-    const int my_m = (P.mblk - xm + P.gm - 1) / P.gm;
-    const int nper = (P.nblk + P.gn - 1) / P.gn;
-    const int n_lo = xn * nper;
-    const int n_hi = n_lo + nper < P.nblk ? n_lo + nper : P.nblk;
-    if (my_m <= 0 || n_lo >= n_hi || slot >= my_m * (n_hi - n_lo)) return false;
-    nb = n_lo + slot / my_m;
-    mb = xm + P.gm * (slot % my_m);
-    return true;
-}
 
 __device__ __forceinline__ uint32_t load_u32(const void* p) { return *reinterpret_cast<const uint32_t*>(p); }
 
@@ -925,7 +911,7 @@ quant_token_kernel(const uint16_t* __restrict__ X, int64_t x_stride, uint8_t* __
 
 // Variants the per-token entry point runs (the tuning hook's forced variant applies when it is
 // one of them).
-inline bool has_token_variant(int v) { return v == 5 || v == 6; }
+inline bool has_token_variant(int v) { return v == 5 || v == 6 || v >= kSliceVariant; }
 
 constexpr int64_t kL2Bytes = (int64_t)4 << 20;        // per XCD
 constexpr int kLdsPerCu = 160 * 1024;
@@ -969,6 +955,18 @@ int pick_split(const Params& P, int BM, int lds_bytes, bool act_scales)
 
 int launch_gemm(Params& P, int variant, bool tok, hipStream_t st)
 {
+    if (variant >= kSliceVariant) {
+        const SliceShape sh = kSliceShapes[variant - kSliceVariant];
+        P.nblk = (P.N + 16 * sh.tn - 1) / (16 * sh.tn);
+        P.mblk = (P.M + 16 * sh.tm - 1) / (16 * sh.tm);
+        if ((int64_t)P.nblk * P.mblk > 0x7FFFFFFF - kXcds) return FP8KV_ERR_SHAPE;
+        P.gm = pick_split(P, 16 * sh.tm, kLdsPerCu, !tok);
+        P.gn = kXcds / P.gm;
+        const int64_t per = (int64_t)((P.mblk + P.gm - 1) / P.gm) * ((P.nblk + P.gn - 1) / P.gn);
+        begin_launch();
+        launch_slice(variant - kSliceVariant, tok, dim3((unsigned)(per * kXcds)), st, P);
+        return finish_launch();
+    }
     const int BN = variant == 6 ? BigGeom<2, 2, 8, 4, 2>::BN : variant == 7 ? BigGeom<2, 2, 4, 8, 2>::BN
                  : variant == 8 ? BigGeom<2, 4, 8, 4, 3>::BN : 128;
     const int BM = variant == 6 ? BigGeom<2, 2, 8, 4, 2>::BM : variant == 7 ? BigGeom<2, 2, 4, 8, 2>::BM
@@ -1142,6 +1140,6 @@ extern "C" int h4a8_gemm_token(const void* W, const void* St, const void* Xq, co
 
 extern "C" void fp8kv_gemm_tune(int variant, int order)
 {
-    fp8kv::w4a8_detail::g_gemm_variant = (variant >= 0 && variant <= 8) ? variant : -1;
+    fp8kv::w4a8_detail::g_gemm_variant = (variant >= 0 && variant < kSliceVariant + kNumSliceShapes) ? variant : -1;
     fp8kv::w4a8_detail::g_gemm_order = (order == 1 || order == 2) ? order : 0;
 }

@@ -21,7 +21,7 @@ LIB_NAME = "libfp8kv_amd.so"
 LIB_PATH = os.path.join(PKG_ROOT, LIB_NAME)
 
 SOURCES = ["h4mv.hip", "h4mv_repack.hip", "decode_attn.hip", "prefill_attn.hip", "prefill_bf16kv.hip",
-           "cache_write.hip", "epilogues.hip", "w4a8_gemm.hip", "lm_head.hip"]
+           "cache_write.hip", "epilogues.hip", "w4a8_gemm.hip", "w4a8_slice.hip", "lm_head.hip"]
 # The benchmark's read-only reference launch (fp8kv_stream_read) is a measurement aid, not part of
 # the path: it is built into a library of its own that only bench.py loads.
 MEASURE_LIB_NAME = "libfp8kv_measure.so"
@@ -47,6 +47,7 @@ HIPCC_FLAGS = [
 # 12.85 -> 12.40 us).  Arguments passed as a struct are not preloaded.
 FILE_FLAGS = {
     "w4a8_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+    "w4a8_slice.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "h4mv.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "decode_attn.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "prefill_bf16kv.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],

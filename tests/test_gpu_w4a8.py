@@ -75,6 +75,28 @@ def test_gemm_parity(N, K, M, variant, order):
     assert matvec.bf16_excess_error(got, ref) < 1e-4
 
 
+@pytest.mark.parametrize("shape", range(10))
+@pytest.mark.parametrize("act", ["mx", "token"])
+@pytest.mark.parametrize("N,K,M", [(64, 512, 1), (36, 640, 17), (260, 1152, 129), (132, 3584, 65), (128, 8064, 40)])
+def test_slice_kernel_parity(shape, act, N, K, M):
+    """Every tile of the K-splitting kernel on partial tiles in both directions: fewer steps than
+    waves (K = 512: 4), slices of unequal length, whose last scale load is moved back inside the row
+    (640: 5 steps; 1152: 9; 8064: 63), and the repeat of a call, bit for bit (counted waits)."""
+    lib = _lib.load()
+    c, rc, rs = (_token_case if act == "token" else _gemm_case)(N, K, M, seed=N + M)
+    ref = (w4a8.gemm_token if act == "token" else w4a8.gemm)(c["W"].numpy(), c["St"].numpy(), rc, rs)
+    args = [torch.from_numpy(rc).to(DEV), torch.from_numpy(rs).to(DEV), c["W"].to(DEV), c["St"].to(DEV)]
+    gemm = ops.h4a8_gemm_token if act == "token" else ops.h4a8_gemm
+    try:
+        lib.fp8kv_gemm_tune(9 + shape, 0)
+        out, again = gemm(*args).clone(), gemm(*args)
+        torch.cuda.synchronize()
+    finally:
+        lib.fp8kv_gemm_tune(-1, 0)
+    assert torch.equal(out, again)
+    assert matvec.bf16_excess_error(out.float().cpu().numpy(), ref) < 1e-4
+
+
 @pytest.mark.parametrize("variant", [-1, 5, 6, 8])
 def test_gemm_scales_only_4_byte_aligned(variant):
     """Scale operands that start 4 bytes past a 16-byte boundary (the entry point requires 4): the
