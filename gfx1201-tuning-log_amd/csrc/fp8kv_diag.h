@@ -75,8 +75,9 @@ void fp8kv_decode_tune(int variant, int target_wgs);
  * token blocks (r, n16 - 1 - r) at any grid size, or -1 for the per-GQA default. */
 void fp8kv_prefill_tune(int shape);
 
-/* bf16-KV prefill: query heads per wave (1 or 2); any other value restores the default (two where
- * GQA > 1, else one). */
+/* bf16-KV prefill: query heads per wave of the register-direct kernel (1 or 2), or the key-split kernel
+ * (3; 4 with paired token blocks at any grid size); any other value restores the default (chosen from
+ * the shape; two heads per wave where GQA > 1, else one). */
 void fp8kv_prefill_bf16_tune(int heads_per_wave);
 
 /* Planner query of the prefill attention launch (host only, no GPU call): the plan the entry

@@ -36,6 +36,7 @@
 #include "fp8kv_status.h"
 #include "attn_common.h"
 #include "fp8kv_diag.h"
+#include "prefill_bf16kv.h"
 
 namespace fp8kv {
 namespace prefill_detail {
@@ -447,6 +448,7 @@ constexpr int kStageFloats = 8 * 64 * 4 + 64;        // one row-set: o [n][lane]
 // arithmetic (exp2(kMaxFloor - m) is 0 for any real row max m, and a row that has seen no key
 // keeps l = 0 and o = 0).
 constexpr float kMaxFloor = -1e30f;
+constexpr float kMaxFloor16 = -3e38f;      // bf16 caches are not bounded by a scale: below any finite score
 
 // max without the NaN-quieting canonicalisation the compiler adds to fmaxf of values that come
 // from MFMA results or lane swaps (the scores are never NaN: finite fp8 and bf16 inputs).
@@ -487,9 +489,8 @@ __device__ __forceinline__ float max_xor16_32_raw(float v)
 // alpha = exp2(0) = 1, exact), so the exponentials of row-set j and the P.V MFMAs of row-set
 // j - 1 sit in one basic block and interleave.
 template <int RS>
-__device__ __forceinline__ void softmax_pv_tile(const f32x4_t (&sc)[RS][2], float (&m_run)[RS],
-                                                float (&l_run)[RS], f32x4_t (&o)[RS][8],
-                                                const float (&qkr)[RS], const u32x4_t (&vf)[8])
+__device__ __forceinline__ void rescale_rows(const f32x4_t (&sc)[RS][2], float (&m_run)[RS], float (&l_run)[RS],
+                                             f32x4_t (&o)[RS][8], const float (&qkr)[RS])
 {
     float m8[RS];
     bool any_need = false;
@@ -514,22 +515,37 @@ __device__ __forceinline__ void softmax_pv_tile(const f32x4_t (&sc)[RS][2], floa
             m_run[j] = m_new;
         }
     }
+}
+
+// Probabilities of row-set j's tile in bf16 (the P^T operand), their fp32 sum added to l.  FUSED takes
+// score * qk - m in one fma: m is the rounded product of the row's largest score, so beyond |m| ~ 1e9
+// the difference is the rounding error, not 0.  e4m3 scores stay far below; bf16 ones are unbounded
+// and round the product like m.
+template <bool FUSED>
+__device__ __forceinline__ u32x4_t row_probs(const f32x4_t (&sc)[2], float qk, float m_run, float& l)
+{
+#pragma clang fp contract(off)
+    const float nm = -m_run;
+    float p[2][4];
+#pragma unroll
+    for (int kg = 0; kg < 2; ++kg)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            p[kg][e] = __builtin_amdgcn_exp2f(FUSED ? __builtin_fmaf(sc[kg][e], qk, nm) : sc[kg][e] * qk + nm);
+    l += ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) + ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
+    return (u32x4_t){pack_bf16x2(p[0][0], p[0][1]), pack_bf16x2(p[0][2], p[0][3]), pack_bf16x2(p[1][0], p[1][1]),
+                     pack_bf16x2(p[1][2], p[1][3])};
+}
+
+template <int RS>
+__device__ __forceinline__ void softmax_pv_tile(const f32x4_t (&sc)[RS][2], float (&m_run)[RS],
+                                                float (&l_run)[RS], f32x4_t (&o)[RS][8],
+                                                const float (&qkr)[RS], const u32x4_t (&vf)[8])
+{
+    rescale_rows<RS>(sc, m_run, l_run, o, qkr);
 #pragma unroll
     for (int j = 0; j < RS; ++j) {
-        const float qk = qkr[j];
-        const float nm = -m_run[j];
-        float p[2][4];
-#pragma unroll
-        for (int kg = 0; kg < 2; ++kg)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                p[kg][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][kg][e], qk, nm));
-        l_run[j] += ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) + ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
-        u32x4_t pb;
-        pb[0] = pack_bf16x2(p[0][0], p[0][1]);
-        pb[1] = pack_bf16x2(p[0][2], p[0][3]);
-        pb[2] = pack_bf16x2(p[1][0], p[1][1]);
-        pb[3] = pack_bf16x2(p[1][2], p[1][3]);
+        const u32x4_t pb = row_probs<true>(sc[j], qkr[j], m_run[j], l_run[j]);
 #pragma unroll
         for (int n = 0; n < 8; ++n) o[j][n] = mfma16x16x32_bf16(as_bf16x8(vf[n]), as_bf16x8(pb), o[j][n]);
     }
@@ -543,16 +559,29 @@ __device__ __forceinline__ void softmax_pv_tile(const f32x4_t (&sc)[RS][2], floa
     }
 }
 
-template <int RS, int NG, int TPW>
+// bf16 caches (B16): a tile is 16 KB, sixteen 1 KB copies of four 256-byte rows; wave w copies K rows and
+// V rows 4w .. 4w + 3, chunk c of row r at 16 (c ^ (r % 16)), so that the 16 rows one K fragment read
+// touches fall in 16 distinct bank groups.  K and Q go to the bf16 MFMA as they are, the scales do not
+// apply, and V needs only the register transpose.
+//
+// MB: the workgroup owns P.nb consecutive token blocks of a GQA below four, row-set r = (block r / gqa,
+// head r % gqa); otherwise one block, row-set r = head r.  Row-sets past the last repeat it and are not
+// stored.
+constexpr int kTileBytes16 = 16384;
+__device__ __forceinline__ int b16_slot(int row, int c) { return row * 256 + 16 * (c ^ (row & 15)); }
+
+template <int RS, int NG, int TPW, bool B16, bool MB>
 __global__ void __launch_bounds__(kSplitWaves * 64)
 prefill_split_kernel(Params P)
 {
     constexpr int W = kSplitWaves;
+    constexpr float floor_m = B16 ? kMaxFloor16 : kMaxFloor;
+    constexpr int TILE = B16 ? kTileBytes16 : kTileBytes;
     constexpr int RW = 2;                                  // ring windows
     constexpr int NR = W / NG;
     constexpr int NT = NR * TPW;                           // tiles per window
     static_assert(NG * NR == W && RS >= 1 && NT <= 64, "split shape");
-    constexpr int kWinBytes = NT * kTileBytes;
+    constexpr int kWinBytes = NT * TILE;
     constexpr int kRingBytes = RW * kWinBytes;
     constexpr int kStageBytes = NR > 1 ? NG * RS * kStageFloats * 4 : 0;
     // The merge stage reuses the ring: it is written only after every wave has finished its
@@ -589,59 +618,89 @@ prefill_split_kernel(Params P)
         qlen = P.qlen_host;
         q0 = P.q0_host;
     }
-    const int n16 = (qlen + 15) >> 4;
+    const int nbt = MB ? P.nb : 1;                                 // token blocks of 16 per workgroup
+    const int n16 = (qlen + 16 * nbt - 1) / (16 * nbt);
     const int tb = P.ntb_grid - 1 - rank;
     const int nwg = P.paired ? (n16 + 1) >> 1 : n16;              // workgroups this sequence needs
     if (tb < 0 || tb >= nwg || q0 < 0) return;                    // whole workgroup, before any barrier
     const int blk_a = tb, blk_b = P.paired ? n16 - 1 - tb : tb;
     const int nphase = blk_b > blk_a ? 2 : 1;
     const int32_t* btrow = P.bt + (int64_t)seq * P.bt_stride;
-    const float qk_signed = P.sm_scale * P.k_scale[0] * kLog2e;
+    const float qk_signed = B16 ? P.sm_scale * kLog2e : P.sm_scale * P.k_scale[0] * kLog2e;
     const float qk = fmaxf(fabsf(qk_signed), 1e-30f);         // > 0: -inf * qk stays -inf
-    const uint32_t qflip = qk_signed < 0.f ? 0x80808080u : 0u;   // negate Q (exact in e4m3)
-    const float vs = P.v_scale[0];
+    const uint32_t qflip = qk_signed < 0.f ? (B16 ? 0x80008000u : 0x80808080u) : 0u;   // negate Q (exact)
+    const float vs = B16 ? 1.f : P.v_scale[0];
 
-    // This wave's copy instruction of every tile: K rows (waves 0-3) or V rows (waves 4-7)
-    // 8 (wave & 3) .. +7, lane (row, chunk) as chosen by dma_lane_rc.
-    const bool dma_v = wave >= 4;
+    // This wave's copies of every tile, lane (row, chunk).  e4m3: one, of K rows (waves 0-3) or V rows
+    // (waves 4-7) 8 (wave & 3) .. +7, as chosen by dma_lane_rc; bf16: two, of K and V rows 4 wave .. +3.
+    const bool dma_v = !B16 && wave >= 4;
     int dma_r, dma_c;
-    dma_lane_rc(dma_v, lane, dma_r, dma_c);
-    const int dma_rk = 8 * (wave & 3) + dma_r;                     // key offset within a tile
+    if constexpr (B16) {
+        dma_r = lane >> 4;
+        dma_c = (lane & 15) ^ ((4 * wave + dma_r) & 15);
+    } else {
+        dma_lane_rc(dma_v, lane, dma_r, dma_c);
+    }
+    // The wave's rows lie in one aligned group of 8 (e4m3) or 4 and the block size is a power of two
+    // >= 16, so the slot of key 32 t + dma_row0 + dma_r is (32 t + dma_row0) mod block size
+    // (wave-uniform, folded into the scalar base) plus dma_r (this lane's fixed offset).
+    const int dma_row0 = B16 ? 4 * wave : 8 * (wave & 3);
+    const int dma_rk = dma_row0 + dma_r;                           // key offset within a tile
     const uint8_t* dma_base = dma_v ? P.v + (int64_t)kh * P.sv2 : P.k + (int64_t)kh * P.sk2;
     const int64_t dma_s0 = dma_v ? P.sv0 : P.sk0;
     const uint32_t dma_s1 = (uint32_t)(dma_v ? P.sv1 : P.sk1);    // < 2^32 / block size (host check)
     const uint32_t dma_chunk = 16u * (uint32_t)dma_c;
-    // The wave's 8 rows start at a multiple of 8 and the block size is a power of two >= 16, so
-    // the slot of key 32 t + dma_rk is (32 t + 8 (wave & 3)) mod block size (wave-uniform, folded
-    // into the scalar base) plus dma_r (this lane's fixed offset).
-    const int dma_row0 = 8 * __builtin_amdgcn_readfirstlane(wave & 3);
     const uint32_t voff_lane = (uint32_t)dma_r * dma_s1 + dma_chunk;
+    const uint8_t* const dma_base_v = P.v + (int64_t)kh * P.sv2;   // bf16: the second copy
+    const uint32_t voff_lane_v = (uint32_t)dma_r * (uint32_t)P.sv1 + dma_chunk;
+
+    // row-set j of this wave: its head, and the first token of its block in units of the launch's blocks
+    int rs_head[RS], rs_blk[RS];
+#pragma unroll
+    for (int j = 0; j < RS; ++j) {
+        const int rset = min(grp * RS + j, nbt * P.gqa - 1);
+        rs_blk[j] = MB ? rset / P.gqa : 0;
+        rs_head[j] = MB ? rset % P.gqa : rset;
+    }
 
     for (int ph = 0; ph < nphase; ++ph) {
         const int blk = ph == 0 ? blk_b : blk_a;
-        const int qpos0 = q0 + 16 * blk;
-        const int k_hi = q0 + min(16 * blk + 16, qlen);           // keys [0, k_hi)
+        const int tok0 = 16 * nbt * blk;                          // first token of the block(s)
+        const int qpos0 = q0 + tok0;
+        const int k_hi = q0 + min(tok0 + 16 * nbt, qlen);         // keys [0, k_hi)
         const int ntiles = (k_hi + kBN - 1) / kBN;
         const int nwin = (ntiles + NT - 1) / NT;
 
-        // Q as the fp8 B operand of S^T = K.Q^T (lane (n, p): d 16p .. 16p+15 and 64+16p .. +15
-        // of query row n), split exactly into e4m3 hi + lo parts (q_fp8_split), with the row's
-        // scale folded into this lane's softmax factor qkr.
+        // Q as the B operand of S^T = K.Q^T (lane (n, p): d 16p .. 16p+15 and 64+16p .. +15 of query
+        // row n).  e4m3 caches: split exactly into e4m3 hi + lo parts (q_fp8_split), the row's scale
+        // folded into this lane's softmax factor qkr.  bf16 caches: the four bf16 fragments.
         v8i qhi[RS], qlo[RS];
         float qkr[RS];
-        const int tok = 16 * blk + lr;
-        const bool tok_ok = tok < qlen;
+        auto token_of = [&](int j) { return MB ? tok0 + 16 * rs_blk[j] + lr : tok0 + lr; };
 #pragma unroll
         for (int j = 0; j < RS; ++j) {
             const u32x4_t zero = {0u, 0u, 0u, 0u};
+            const int tok = token_of(j);
+            const bool tok_ok = tok < qlen;
             const __bf16* qrow = P.q + (int64_t)(q_begin + (tok_ok ? tok : 0)) * P.q_stride +
-                                 (int64_t)(kh * P.gqa + grp * RS + j) * kD;
+                                 (int64_t)(kh * P.gqa + rs_head[j]) * kD;
             u32x4_t qf[4];
             qf[0] = tok_ok ? load_16(qrow + 16 * lp) : zero;
             qf[1] = tok_ok ? load_16(qrow + 16 * lp + 8) : zero;
             qf[2] = tok_ok ? load_16(qrow + 64 + 16 * lp) : zero;
             qf[3] = tok_ok ? load_16(qrow + 64 + 16 * lp + 8) : zero;
-            qkr[j] = qk * q_fp8_split(qf, qflip, qhi[j], qlo[j]);
+            if constexpr (B16) {
+                qkr[j] = qk;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    qhi[j][d] = (int)(qf[0][d] ^ qflip);
+                    qhi[j][4 + d] = (int)(qf[1][d] ^ qflip);
+                    qlo[j][d] = (int)(qf[2][d] ^ qflip);
+                    qlo[j][4 + d] = (int)(qf[3][d] ^ qflip);
+                }
+            } else {
+                qkr[j] = qk * q_fp8_split(qf, qflip, qhi[j], qlo[j]);
+            }
         }
 
         // Block ids for this wave's copy instruction of each tile of window wi (its 8 rows lie
@@ -650,7 +709,7 @@ prefill_split_kernel(Params P)
         // two windows the wait for window i's copies also covers this load (issued after them).
         int bids = 0;
         auto load_bids = [&](int wi) {
-            const int key0 = min((wi * NT + lane) * kBN + 8 * (wave & 3), k_hi - 1);
+            const int key0 = min((wi * NT + lane) * kBN + dma_row0, k_hi - 1);
             bids = lane < NT ? btrow[key0 >> P.pshift] : 0;
         };
         // Copies of tiles u0 .. u1 - 1 of window wi (keys >= k_hi fetch key k_hi - 1; the causal
@@ -662,14 +721,20 @@ prefill_split_kernel(Params P)
                 if (t < ntiles) {
                     const int64_t b = __builtin_amdgcn_readlane(bids, u);
                     const uint8_t* sb = dma_base + b * dma_s0;
-                    uint32_t voff = voff_lane;
+                    const uint8_t* sbv = dma_base_v + b * P.sv0;
+                    uint32_t voff = voff_lane, voff_v = voff_lane_v;
                     if (t * kBN + kBN > k_hi) {             // the tile holding the end of the keys
-                        const int key = min(t * kBN + dma_rk, k_hi - 1);
-                        voff = (uint32_t)(key & (P.pblk - 1)) * dma_s1 + dma_chunk;
+                        const uint32_t slot = (uint32_t)(min(t * kBN + dma_rk, k_hi - 1) & (P.pblk - 1));
+                        voff = slot * dma_s1 + dma_chunk;
+                        voff_v = slot * (uint32_t)P.sv1 + dma_chunk;
                     } else {
-                        sb += (uint32_t)((t * kBN + dma_row0) & (P.pblk - 1)) * dma_s1;
+                        const uint32_t slot = (uint32_t)((t * kBN + dma_row0) & (P.pblk - 1));
+                        sb += slot * dma_s1;
+                        sbv += slot * (uint32_t)P.sv1;
                     }
-                    dma16_saddr(sb, voff, ring + (wi % RW) * kWinBytes + u * kTileBytes + wave * 1024);
+                    unsigned char* dst = ring + (wi % RW) * kWinBytes + u * TILE + wave * 1024;
+                    dma16_saddr(sb, voff, dst);
+                    if constexpr (B16) dma16_saddr(sbv, voff_v, dst + TILE / 2);
                 }
             }
         };
@@ -685,7 +750,7 @@ prefill_split_kernel(Params P)
         f32x4_t o[RS][8];
 #pragma unroll
         for (int j = 0; j < RS; ++j) {
-            m_run[j] = kMaxFloor;
+            m_run[j] = floor_m;
             l_run[j] = 0.f;
 #pragma unroll
             for (int n = 0; n < 8; ++n) o[j][n] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -708,57 +773,118 @@ prefill_split_kernel(Params P)
                 const int t = i * NT + tw;
                 if (t >= ntiles) continue;
                 const int k0 = t * kBN;
-                const unsigned char* buf = ring + (i % RW) * kWinBytes + tw * kTileBytes;
-
-                // K as the fp8 A operand, straight from the ring: lane (r, p) = key 16 kg + r,
-                // d 16p .. 16p+15 (chunk p) and 64+16p .. +15 (chunk 4 + p).
-                v8i kf[2];
-#pragma unroll
-                for (int kg = 0; kg < 2; ++kg) {
-                    const int row = 16 * kg + lr;
-                    const unsigned char* kb = buf + (row >> 3) * 1024;
-                    const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(kb + 16 * k_slot(row & 7, lp));
-                    const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(kb + 16 * k_slot(row & 7, 4 + lp));
-                    kf[kg] = (v8i){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
-                                   (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-                }
-                // V^T raw rows (lane (c, p) transposes d = 8c .. 8c+7) and their widening go ahead
-                // of S^T = K.Q^T, so the VALU work can run between the MFMAs.
-                u32x2_t vr[8];
-#pragma unroll
-                for (int jj = 0; jj < 8; ++jj) {
-                    const int row = (jj < 4 ? 0 : 16) + 4 * lp + (jj & 3);
-                    const unsigned char* vb = buf + 4096 + (row >> 3) * 1024;
-                    vr[jj] = *reinterpret_cast<const u32x2_t*>(vb + 16 * v_slot(row & 7, lr >> 1) + 8 * (lr & 1));
-                }
-                u32x4_t vf[8];
-                v_fragments(vr, vf);
+                const unsigned char* buf = ring + (i % RW) * kWinBytes + tw * TILE;
                 f32x4_t sc[RS][2];
-#pragma unroll
-                for (int j = 0; j < RS; ++j)
+                u32x4_t vf[8];
+                if constexpr (B16) {
+                    // K fragments of 16 keys at a time: lane (r, p) = key 16 kg + r, d 16p .. 16p+15 (chunks
+                    // 2p, 2p + 1) and 64+16p .. +15 (chunks 8 + 2p, 9 + 2p)
 #pragma unroll
                     for (int kg = 0; kg < 2; ++kg) {
-                        const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-                        f32x4_t acc = mfma_fp8_16x16x128(kf[kg], qhi[j], zero);
-                        sc[j][kg] = mfma_fp8_16x16x128(kf[kg], qlo[j], acc);
-                    }
-                // Interleave: one MFMA, then up to four VALU (the V widening, 48 instructions).
+                        const int row = 16 * kg + lr;
+                        u32x4_t kf[4];
 #pragma unroll
-                for (int g = 0; g < 4 * RS; ++g) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-                }
-                if (k0 + kBN - 1 > qpos0) {                        // tile reaches past the first row
-                    const int qpos = qpos0 + lr;
+                        for (int f = 0; f < 4; ++f)
+                            kf[f] = *reinterpret_cast<const u32x4_t*>(buf + b16_slot(row, 8 * (f >> 1) + 2 * lp + (f & 1)));
+#pragma unroll
+                        for (int j = 0; j < RS; ++j) {
+                            f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                            for (int f = 0; f < 4; ++f) {
+                                const v8i& qq = f < 2 ? qhi[j] : qlo[j];
+                                const int h = 4 * (f & 1);
+                                const u32x4_t qv = {(uint32_t)qq[h], (uint32_t)qq[h + 1], (uint32_t)qq[h + 2],
+                                                    (uint32_t)qq[h + 3]};
+                                acc = mfma16x16x32_bf16(as_bf16x8(kf[f]), as_bf16x8(qv), acc);
+                            }
+                            sc[j][kg] = acc;
+                        }
+                    }
+                } else {
+                    // K as the fp8 A operand, straight from the ring: lane (r, p) = key 16 kg + r,
+                    // d 16p .. 16p+15 (chunk p) and 64+16p .. +15 (chunk 4 + p).
+                    v8i kf[2];
+#pragma unroll
+                    for (int kg = 0; kg < 2; ++kg) {
+                        const int row = 16 * kg + lr;
+                        const unsigned char* kb = buf + (row >> 3) * 1024;
+                        const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(kb + 16 * k_slot(row & 7, lp));
+                        const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(kb + 16 * k_slot(row & 7, 4 + lp));
+                        kf[kg] = (v8i){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
+                                       (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+                    }
+                    // V^T raw rows (lane (c, p) transposes d = 8c .. 8c+7) and their widening go ahead
+                    // of S^T = K.Q^T, so the VALU work can run between the MFMAs.
+                    u32x2_t vr[8];
+#pragma unroll
+                    for (int jj = 0; jj < 8; ++jj) {
+                        const int row = (jj < 4 ? 0 : 16) + 4 * lp + (jj & 3);
+                        const unsigned char* vb = buf + 4096 + (row >> 3) * 1024;
+                        vr[jj] = *reinterpret_cast<const u32x2_t*>(vb + 16 * v_slot(row & 7, lr >> 1) + 8 * (lr & 1));
+                    }
+                    v_fragments(vr, vf);
 #pragma unroll
                     for (int j = 0; j < RS; ++j)
+#pragma unroll
+                        for (int kg = 0; kg < 2; ++kg) {
+                            const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+                            f32x4_t acc = mfma_fp8_16x16x128(kf[kg], qhi[j], zero);
+                            sc[j][kg] = mfma_fp8_16x16x128(kf[kg], qlo[j], acc);
+                        }
+                    // Interleave: one MFMA, then up to four VALU (the V widening, 48 instructions).
+#pragma unroll
+                    for (int g = 0; g < 4 * RS; ++g) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                    }
+                }
+                if (k0 + kBN - 1 > qpos0) {                        // tile reaches past the first row
+#pragma unroll
+                    for (int j = 0; j < RS; ++j) {
+                        const int qpos = q0 + token_of(j);
 #pragma unroll
                         for (int kg = 0; kg < 2; ++kg)
 #pragma unroll
                             for (int e = 0; e < 4; ++e)
                                 if (k0 + 16 * kg + 4 * lp + e > qpos) sc[j][kg][e] = neg_inf();
+                    }
                 }
-                softmax_pv_tile<RS>(sc, m_run, l_run, o, qkr, vf);
+                if constexpr (!B16) {
+                    softmax_pv_tile<RS>(sc, m_run, l_run, o, qkr, vf);
+                } else {
+                    // Half of a V row's 16 bytes at a time, so that 16 registers hold the tile's V instead
+                    // of 32 (the RS = 3 kernel has none to spare): half h is d = 8c + 4h .. + 3.
+                    u32x2_t vr[8];
+                    auto read_half = [&](int h) {
+#pragma unroll
+                        for (int jj = 0; jj < 8; ++jj) {
+                            const int row = (jj < 4 ? 0 : 16) + 4 * lp + (jj & 3);
+                            vr[jj] = *reinterpret_cast<const u32x2_t*>(buf + TILE / 2 + b16_slot(row, lr) + 8 * h);
+                        }
+                    };
+                    read_half(0);
+                    rescale_rows<RS>(sc, m_run, l_run, o, qkr);
+                    u32x4_t pb[RS];
+#pragma unroll
+                    for (int j = 0; j < RS; ++j) pb[j] = row_probs<false>(sc[j], qkr[j], m_run[j], l_run[j]);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        u32x4_t va[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+#pragma unroll
+                            for (int w = 0; w < 2; ++w) {
+                                va[2 * w][k] = __builtin_amdgcn_perm(vr[2 * k + 1][w], vr[2 * k][w], 0x05040100u);
+                                va[2 * w + 1][k] = __builtin_amdgcn_perm(vr[2 * k + 1][w], vr[2 * k][w], 0x07060302u);
+                            }
+                        if (h == 0) read_half(1);
+#pragma unroll
+                        for (int n = 0; n < 4; ++n)
+#pragma unroll
+                            for (int j = 0; j < RS; ++j)
+                                o[j][4 * h + n] = mfma16x16x32_bf16(as_bf16x8(va[n]), as_bf16x8(pb[j]), o[j][4 * h + n]);
+                    }
+                }
             }
             // Block ids for the next window's copies, after this iteration's LDS reads so that
             // no LDS wait in the tile work has to cover the scalar loads.
@@ -775,7 +901,7 @@ prefill_split_kernel(Params P)
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < RS; ++j) {
-                float mg = kMaxFloor;
+                float mg = floor_m;
 #pragma unroll
                 for (int r = 0; r < NR; ++r) mg = fmaxf(mg, stage_m[((grp * NR + r) * RS + j) * 16 + lr]);
                 const float f = __builtin_amdgcn_exp2f(m_run[j] - mg);
@@ -814,10 +940,11 @@ prefill_split_kernel(Params P)
 #pragma unroll
             for (int j = 0; j < RS; ++j) {
                 const float l = sum_xor16_32(l_run[j]);
-                if (!tok_ok) continue;
+                const int tok = token_of(j);
+                if (tok >= qlen || grp * RS + j >= nbt * P.gqa) continue;
                 const float f = l > 0.f ? vs / l : 0.f;
                 __bf16* orow = P.out + (int64_t)(q_begin + tok) * P.o_stride +
-                               (int64_t)(kh * P.gqa + grp * RS + j) * kD + 32 * lp;
+                               (int64_t)(kh * P.gqa + rs_head[j]) * kD + 32 * lp;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     u32x4_t w;
@@ -970,11 +1097,11 @@ int launch(const Params& P0, int num_seqs, int max_query_len, int ctx_hint, hipS
     begin_launch();
     if (L.split >= 0) {
         switch (L.split) {
-            case 0: launch_kernel(prefill_split_kernel<3, 2, 2>, L.grid, L.block, 0, stream, P); break;
-            case 1: launch_kernel(prefill_split_kernel<3, 4, 2>, L.grid, L.block, 0, stream, P); break;
-            case 2: launch_kernel(prefill_split_kernel<2, 2, 2>, L.grid, L.block, 0, stream, P); break;
-            case 3: launch_kernel(prefill_split_kernel<2, 4, 2>, L.grid, L.block, 0, stream, P); break;
-            default: launch_kernel(prefill_split_kernel<2, 8, 2>, L.grid, L.block, 0, stream, P); break;
+            case 0: launch_kernel(prefill_split_kernel<3, 2, 2, false, false>, L.grid, L.block, 0, stream, P); break;
+            case 1: launch_kernel(prefill_split_kernel<3, 4, 2, false, false>, L.grid, L.block, 0, stream, P); break;
+            case 2: launch_kernel(prefill_split_kernel<2, 2, 2, false, false>, L.grid, L.block, 0, stream, P); break;
+            case 3: launch_kernel(prefill_split_kernel<2, 4, 2, false, false>, L.grid, L.block, 0, stream, P); break;
+            default: launch_kernel(prefill_split_kernel<2, 8, 2, false, false>, L.grid, L.block, 0, stream, P); break;
         }
         return finish_launch();
     }
@@ -988,6 +1115,33 @@ int launch(const Params& P0, int num_seqs, int max_query_len, int ctx_hint, hipS
         case 7: launch_kernel(prefill_kernel<8, 2, 4>, L.grid, L.block, 0, stream, P); break;
         default: launch_kernel(prefill_kernel<4, 1, 4>, L.grid, L.block, 0, stream, P); break;
     }
+    return finish_launch();
+}
+
+// bf16 caches: the same kernel for every GQA, row-sets spread over the smallest shape that holds them
+// (GQA 1 and 2 pack 4 / GQA token blocks into a workgroup).  Against one wave per two heads with
+// register-direct loads (prefill_bf16kv_kernel; us in a graph): 2048 tokens after 2048, 24 / 4 heads
+// 210 -> 104, 32 / 8 287 -> 170, 16 / 16 253 -> 89, 28 / 4 282 -> 125; 1500 alone, 24 / 4 70 -> 44;
+// 3 x 100..300 after 2000 107 -> 43.
+inline int bf16_split_blocks(int gqa) { return gqa <= 2 ? 4 / gqa : 1; }
+
+int launch_bf16(const Params& P0, int num_seqs, int max_query_len, bool force_paired, hipStream_t stream)
+{
+    Params P = P0;
+    const int g = P.gqa;
+    P.nb = bf16_split_blocks(g);
+    const int n = (max_query_len + 16 * P.nb - 1) / (16 * P.nb);
+    P.xcd_map = (P.hkv <= 8 && 8 % P.hkv == 0) ? 1 : 0;
+    P.paired = force_paired || !split_single_blocks_fit(n, P.hkv, num_seqs);
+    const int per = split_xcd_per(P.hkv), ranks = P.paired ? (n + 1) / 2 : n;
+    P.ntb_grid = (ranks + per - 1) / per * per;
+    const dim3 grid((unsigned)(P.ntb_grid * P.hkv), 1u, (unsigned)num_seqs), block(64 * kSplitWaves);
+    begin_launch();
+    if (g <= 2) launch_kernel(prefill_split_kernel<2, 2, 1, true, true>, grid, block, 0, stream, P);
+    else if (g <= 4) launch_kernel(prefill_split_kernel<2, 2, 1, true, false>, grid, block, 0, stream, P);
+    else if (g <= 6) launch_kernel(prefill_split_kernel<3, 2, 1, true, false>, grid, block, 0, stream, P);
+    else if (g <= 8) launch_kernel(prefill_split_kernel<2, 4, 2, true, false>, grid, block, 0, stream, P);
+    else launch_kernel(prefill_split_kernel<2, 8, 4, true, false>, grid, block, 0, stream, P);
     return finish_launch();
 }
 
@@ -1126,4 +1280,29 @@ extern "C" int fp8kv_prefill_attn_varlen(const void* q, int64_t q_row_stride,
     P.cu_q = cu_seqlens_q;
     P.seq_lens = seq_lens;
     return launch(P, num_seqs, max_query_len, max_query_len, reinterpret_cast<hipStream_t>(stream));
+}
+
+// Where the key-split kernel takes a bf16 call.  Its workgroups cost about 8 us apiece before and after
+// their keys and fill a CU, so it needs contexts of 256 keys, and past one round of single blocks either
+// prompts long enough to pay for it or a GQA whose shape splits the keys two ways or not at all (12
+// prompts of 50..400: 24 / 4 heads 49 us against 35, 28 / 4 40 against 45, 48 / 4 44 against 60; 64
+// tokens alone: 12.1 against 7.0; 300: 15.8 and 17.0; 6 of 37..900 after 200: 70 and 73).  For varlen
+// calls the host knows the longest prompt only and takes it for the context.
+bool fp8kv::prefill_split_takes_bf16(int hkv, int gqa, int num_seqs, int max_query_len, int ctx_hint)
+{
+    if (ctx_hint < kSplitMinContextSingle) return false;
+    const int nb = bf16_split_blocks(gqa);
+    if (split_single_blocks_fit((max_query_len + 16 * nb - 1) / (16 * nb), hkv, num_seqs)) return true;
+    return ctx_hint >= 768 || gqa > 6;
+}
+
+int fp8kv::launch_prefill_split_bf16(const fp8kv::PrefillBf16& A, bool force_paired, hipStream_t stream)
+{
+    Params P = make_params(A.q, A.q_stride, A.k, A.v, A.sk0, A.sk1, A.sk2, A.sv0, A.sv1, A.sv2, A.out,
+                           A.o_stride, A.bt, A.bt_stride, nullptr, nullptr, A.sm_scale, A.hkv * A.gqa, A.hkv, A.pblk);
+    P.cu_q = A.cu_q;
+    P.seq_lens = A.seq_lens;
+    P.q0_host = A.q0;
+    P.qlen_host = A.qlen;
+    return launch_bf16(P, A.num_seqs, A.max_query_len, force_paired, stream);
 }

@@ -3,9 +3,9 @@
 // :143).  For bf16 caches the reference ignores k_scale and v_scale: S = (q . k) * sm_scale and
 // out = softmax(S) . V, with the probabilities rounded to bf16 before P.V (:88,114).
 //
-// gfx950 design (the engine's caches are fp8, so this path serves callers of the reference's
-// run() with bf16 caches; it uses the decode kernel's register-direct chunk loads rather than the
-// fp8 prefill kernels' LDS tile rings):
+// Two kernels.  Contexts long enough to split the keys over a workgroup's waves run the key-split
+// kernel of prefill_attn.hip on 16 KB tiles (prefill_split_takes_bf16 draws the line); the short ones
+// and crowds of short prompts run the one here, whose workgroups are small and cost little to start:
 //   * one workgroup per (16-token block, kv head, group of up to 16 query heads, sequence); each
 //     wave owns two query heads of its block (one for MHA), i.e. two row-sets of 16 queries that
 //     share every K/V load, and streams every key the block sees (q0 + 16 b + 16, capped at the
@@ -21,6 +21,7 @@
 #include "fp8kv_diag.h"
 #include "attn_common.h"
 #include "kv_chunk.h"
+#include "prefill_bf16kv.h"
 
 namespace fp8kv {
 namespace prefill_b16_detail {
@@ -192,12 +193,24 @@ int setup(Params& P, const void* q, int64_t q_row_stride, const void* k_cache, c
 
 // Heads per wave: two wherever GQA > 1, so both row-sets use one set of K/V loads (configs[3]:
 // 222 against 377 us with one head per wave; 1024 over 1024: 98.7 against 122.6 us); one for MHA.
+// 1, 2: this kernel with that many heads per wave; 3, 4: the key-split kernel, 4 with paired blocks.
 thread_local int g_rs_override = 0;
 
 int launch(Params& P, int num_seqs, int max_query_len, hipStream_t stream)
 {
+    // the key-split kernel addresses a row within its cache block with a 32-bit offset
+    const int64_t slot = P.sk1 > P.sv1 ? P.sk1 : P.sv1;
+    const bool fits = (int64_t)(P.pblk - 1) * slot + 2 * kD < ((int64_t)1 << 32);
+    const int ctx_hint = P.cu_q ? max_query_len : P.q0_host + P.qlen_host;
+    if (fits && (g_rs_override > 2 ||
+                 (g_rs_override == 0 && prefill_split_takes_bf16(P.hkv, P.gqa, num_seqs, max_query_len, ctx_hint)))) {
+        const PrefillBf16 A = {P.q, P.k, P.v, P.out, P.cu_q, P.seq_lens, P.bt, P.q_stride, P.o_stride, P.bt_stride,
+                               P.sk0, P.sk1, P.sk2, P.sv0, P.sv1, P.sv2, P.sm_scale, P.hkv, P.gqa, P.pblk,
+                               P.q0_host, P.qlen_host, num_seqs, max_query_len};
+        return launch_prefill_split_bf16(A, g_rs_override == 4, stream);
+    }
     P.n16_grid = (max_query_len + 15) / 16;
-    const int rs = g_rs_override ? g_rs_override : (P.gqa > 1 ? 2 : 1);
+    const int rs = g_rs_override == 1 || P.gqa == 1 ? 1 : 2;
     const int wave_heads = kWavesPerWG * rs;
     const int groups = (P.gqa + wave_heads - 1) / wave_heads;
     const int waves_needed = (P.gqa + rs - 1) / rs;
@@ -270,8 +283,9 @@ extern "C" int fp8kv_prefill_attn_varlen_bf16(const void* q, int64_t q_row_strid
     return launch(P, num_seqs, max_query_len, reinterpret_cast<hipStream_t>(stream));
 }
 
-// Sweeps and tests: query heads per wave (1 or 2); any other value restores the default.
+// Sweeps and tests: query heads per wave (1 or 2), the key-split kernel (3; 4 with paired token
+// blocks); any other value restores the default.
 extern "C" void fp8kv_prefill_bf16_tune(int heads_per_wave)
 {
-    g_rs_override = (heads_per_wave == 1 || heads_per_wave == 2) ? heads_per_wave : 0;
+    g_rs_override = (heads_per_wave >= 1 && heads_per_wave <= 4) ? heads_per_wave : 0;
 }

@@ -391,6 +391,42 @@ def test_bf16_kv_varlen():
     _check_varlen([512] * 4, [0] * 4, seed=94, layout="engine", kv_gen="bf16", PBLK=32)
 
 
+@pytest.mark.parametrize("paired", [False, True])
+@pytest.mark.parametrize("gqa", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 16])
+def test_bf16_kv_key_split_every_gqa(gqa, paired):
+    """The key-split kernel forced at every row-set packing (several blocks per workgroup at GQA 1 and
+    2, repeated row-sets at 3, 5, 7, 9, 12 and 13), below its default contexts as well: one token, a
+    block and one token more, fewer tiles than key residues, a tail block, a context inside a tile."""
+    lib = _lib.load()
+    try:
+        lib.fp8kv_prefill_bf16_tune(4 if paired else 3)
+        for qlen, q0 in ((1, 0), (17, 15), (33, 0), (65, 700), (161, 45)):
+            _check_single(qlen, q0, HQ=4 * gqa, HKV=4, seed=gqa + qlen, kv_gen="bf16", layout="engine")
+        _check_single(250, 7, HQ=3 * gqa, HKV=3, seed=gqa + 290, kv_gen="bf16", PBLK=64)
+        _check_varlen([5, 100, 33, 200, 1], [0, 7, 500, 3, 250], HQ=2 * gqa, HKV=2, seed=gqa + 93, kv_gen="bf16")
+    finally:
+        lib.fp8kv_prefill_bf16_tune(0)
+
+
+def test_bf16_kv_key_split_stale_rows_and_scale_sign():
+    """NaN in every cache row past the context, and a negative softmax scale."""
+    c = workloads.prefill_case([293], [100], seed=98, layout="engine", kv_gen="bf16")
+    c["kv_cache"][int(c["block_table"][0, 24]), :, 393 - 384:] = float("nan")
+    c["k_cache"], c["v_cache"] = workloads.engine_views(c["kv_cache"], 128)
+    c["sm_scale"] = -c["sm_scale"]
+    got = _run_single(c, 100, 293).to(torch.float64)
+    torch.testing.assert_close(got, _oracle_single(c, 100, 293).to(torch.float64), rtol=RTOL, atol=ATOL)
+
+
+def test_bf16_kv_key_split_scores_below_any_e4m3_score():
+    """Every score about -1.6e30 in log2 units, all equal: each row averages the V rows it sees."""
+    c = workloads.prefill_case([300], [100], seed=99, kv_gen="bf16")
+    c["q"].fill_(1e15)
+    c["k_cache"].fill_(-1e14)
+    got = _run_single(c, 100, 300).to(torch.float64)
+    torch.testing.assert_close(got, _oracle_single(c, 100, 300).to(torch.float64), rtol=RTOL, atol=ATOL)
+
+
 def test_bf16_kv_config3_full_size():
     """configs[3] over bf16 caches: 2048 new tokens after 2048 cached, 24/4 heads."""
     _check_single(2048, 2048, seed=95, layout="engine", kv_gen="bf16")
