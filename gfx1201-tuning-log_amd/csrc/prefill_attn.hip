@@ -438,8 +438,7 @@ prefill_kernel(Params P)
 // SIMD.  The ring holds two windows; window i + 1 is copied (each wave issuing one 1 KB copy of
 // every tile) while window i is consumed, and one barrier per window publishes it.  At the end
 // of a block the NR partial (m, l, o) states of each head group merge in LDS in a fixed order:
-// the common max first, then residue 0 stores its rescaled o and l, residues 1 .. NR - 2 add
-// theirs in turn, and residue NR - 1 adds its own in registers, normalises and writes the output.
+// the common max first, then row-set j in the wave of residue j % NR, which normalises and writes it.
 constexpr int kSplitWaves = 8;
 
 constexpr int kStageFloats = 8 * 64 * 4 + 64;        // one row-set: o [n][lane][4], then l [lane]
@@ -583,10 +582,15 @@ prefill_split_kernel(Params P)
     static_assert(NG * NR == W && RS >= 1 && NT <= 64, "split shape");
     constexpr int kWinBytes = NT * TILE;
     constexpr int kRingBytes = RW * kWinBytes;
-    constexpr int kStageBytes = NR > 1 ? NG * RS * kStageFloats * 4 : 0;
+    constexpr int kStageBytes = NG * RS * (NR - 1) * kStageFloats * 4;
     // The merge stage reuses the ring: it is written only after every wave has finished its
     // last tile, and the next block's copies start only after the stage has been read.
-    __shared__ __align__(16) unsigned char ring[kRingBytes > kStageBytes ? kRingBytes : kStageBytes];
+    // the query rows' hand-over: the ring's second window, or behind the ring where that is too small
+    constexpr int kSetBytes = 4 * 1024 + 256;
+    constexpr int kExch = NG * RS * kSetBytes <= kWinBytes ? kWinBytes : kRingBytes;
+    constexpr int kExchEnd = B16 ? 0 : kExch + NG * RS * kSetBytes;
+    constexpr int kLoopBytes = kRingBytes > kExchEnd ? kRingBytes : kExchEnd;
+    __shared__ __align__(16) unsigned char ring[kLoopBytes > kStageBytes ? kLoopBytes : kStageBytes];
     __shared__ float stage_m[NR > 1 ? NG * NR * RS * 16 : 4];
     float* const stage = reinterpret_cast<float*>(ring);
 
@@ -654,14 +658,12 @@ prefill_split_kernel(Params P)
     const uint8_t* const dma_base_v = P.v + (int64_t)kh * P.sv2;   // bf16: the second copy
     const uint32_t voff_lane_v = (uint32_t)dma_r * (uint32_t)P.sv1 + dma_chunk;
 
-    // row-set j of this wave: its head, and the first token of its block in units of the launch's blocks
-    int rs_head[RS], rs_blk[RS];
-#pragma unroll
-    for (int j = 0; j < RS; ++j) {
-        const int rset = min(grp * RS + j, nbt * P.gqa - 1);
-        rs_blk[j] = MB ? rset / P.gqa : 0;
-        rs_head[j] = MB ? rset % P.gqa : rset;
-    }
+    // head, and block within the workgroup, of row-set rset (those past the last repeat it)
+    auto head_of = [&](int rset) {
+        rset = min(rset, nbt * P.gqa - 1);
+        return MB ? rset % P.gqa : rset;
+    };
+    auto block_of = [&](int rset) { return MB ? min(rset, nbt * P.gqa - 1) / P.gqa : 0; };
 
     for (int ph = 0; ph < nphase; ++ph) {
         const int blk = ph == 0 ? blk_b : blk_a;
@@ -674,34 +676,7 @@ prefill_split_kernel(Params P)
         // Q as the B operand of S^T = K.Q^T (lane (n, p): d 16p .. 16p+15 and 64+16p .. +15 of query
         // row n).  e4m3 caches: split exactly into e4m3 hi + lo parts (q_fp8_split), the row's scale
         // folded into this lane's softmax factor qkr.  bf16 caches: the four bf16 fragments.
-        v8i qhi[RS], qlo[RS];
-        float qkr[RS];
-        auto token_of = [&](int j) { return MB ? tok0 + 16 * rs_blk[j] + lr : tok0 + lr; };
-#pragma unroll
-        for (int j = 0; j < RS; ++j) {
-            const u32x4_t zero = {0u, 0u, 0u, 0u};
-            const int tok = token_of(j);
-            const bool tok_ok = tok < qlen;
-            const __bf16* qrow = P.q + (int64_t)(q_begin + (tok_ok ? tok : 0)) * P.q_stride +
-                                 (int64_t)(kh * P.gqa + rs_head[j]) * kD;
-            u32x4_t qf[4];
-            qf[0] = tok_ok ? load_16(qrow + 16 * lp) : zero;
-            qf[1] = tok_ok ? load_16(qrow + 16 * lp + 8) : zero;
-            qf[2] = tok_ok ? load_16(qrow + 64 + 16 * lp) : zero;
-            qf[3] = tok_ok ? load_16(qrow + 64 + 16 * lp + 8) : zero;
-            if constexpr (B16) {
-                qkr[j] = qk;
-#pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    qhi[j][d] = (int)(qf[0][d] ^ qflip);
-                    qhi[j][4 + d] = (int)(qf[1][d] ^ qflip);
-                    qlo[j][d] = (int)(qf[2][d] ^ qflip);
-                    qlo[j][4 + d] = (int)(qf[3][d] ^ qflip);
-                }
-            } else {
-                qkr[j] = qk * q_fp8_split(qf, qflip, qhi[j], qlo[j]);
-            }
-        }
+        auto token_of = [&](int j) { return tok0 + 16 * block_of(grp * RS + j) + lr; };
 
         // Block ids for this wave's copy instruction of each tile of window wi (its 8 rows lie
         // in one 16-key group, hence one cache block; index clamped to the last key): lane u
@@ -738,13 +713,90 @@ prefill_split_kernel(Params P)
                 }
             }
         };
+        // Q as the B operand of S^T = K.Q^T (lane (n, p): d 16p .. 16p+15 and 64+16p .. +15 of query
+        // row n).  e4m3 caches: split exactly into e4m3 hi + lo parts (q_fp8_split), the row's scale
+        // folded into this lane's softmax factor qkr.  The split is about 270 VALU a row-set, and the
+        // NR residues of a head group need the same ones, so each row-set is split by one wave and
+        // handed over through the LDS (the ring's second window is free until the key loop's first barrier)
+        // (with the merge by row-sets, 24 / 4 heads: 2048 tokens
+        // after 2048 102.1 -> 95.3 us, 1000 after 500 31.5 -> 27.7, 8 of 600 95 -> 72).  bf16 caches: the
+        // four bf16 fragments, loaded by each wave.  Window 0's block ids and the query rows are
+        // requested together, ahead of the window's copies (the asm takes the rows, so the compiler waits there and not behind the copies).
+        static_assert(RW == 2, "one window is copied ahead");
+        auto load_query = [&](u32x4_t (&qf)[4], int tok, int head) {
+            const u32x4_t zero = {0u, 0u, 0u, 0u};
+            const bool ok = tok < qlen;
+            const __bf16* qrow = P.q + (int64_t)(q_begin + (ok ? tok : 0)) * P.q_stride + (int64_t)(kh * P.gqa + head) * kD;
+            qf[0] = ok ? load_16(qrow + 16 * lp) : zero;
+            qf[1] = ok ? load_16(qrow + 16 * lp + 8) : zero;
+            qf[2] = ok ? load_16(qrow + 64 + 16 * lp) : zero;
+            qf[3] = ok ? load_16(qrow + 64 + 16 * lp + 8) : zero;
+        };
+        v8i qhi[RS], qlo[RS];
+        float qkr[RS];
+        load_bids(0);
+        if constexpr (B16) {
+            u32x4_t qf[RS][4];
 #pragma unroll
-        for (int wi = 0; wi < RW - 1; ++wi)
-            if (wi < nwin) {
-                load_bids(wi);
-                issue_window(wi, 0, NT);
+            for (int j = 0; j < RS; ++j) load_query(qf[j], token_of(j), head_of(grp * RS + j));
+#pragma unroll
+            for (int j = 0; j < RS; ++j) {
+                asm volatile("" : "+v"(qf[j][0]), "+v"(qf[j][1]), "+v"(qf[j][2]), "+v"(qf[j][3]));
+                qkr[j] = qk;
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    qhi[j][d] = (int)(qf[j][0][d] ^ qflip);
+                    qhi[j][4 + d] = (int)(qf[j][1][d] ^ qflip);
+                    qlo[j][d] = (int)(qf[j][2][d] ^ qflip);
+                    qlo[j][4 + d] = (int)(qf[j][3][d] ^ qflip);
+                }
             }
-        if (RW - 1 < nwin) load_bids(RW - 1);
+            issue_window(0, 0, NT);
+            if (1 < nwin) load_bids(1);
+        } else {
+            constexpr int SETS = NG * RS, PER = (SETS + W - 1) / W;        // row-sets, and splits per wave at most
+            unsigned char* const exch = ring + kExch;
+            int ln = lane;                             // opaque: its addresses stay out of the key loop's registers
+            asm volatile("" : "+v"(ln));
+            u32x4_t qf[PER][4];
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int rset = wave + W * u;
+                load_query(qf[u], tok0 + 16 * block_of(rset) + lr, head_of(rset));
+            }
+#pragma unroll
+            for (int u = 0; u < PER; ++u)
+                asm volatile("" : "+v"(qf[u][0]), "+v"(qf[u][1]), "+v"(qf[u][2]), "+v"(qf[u][3]));
+            issue_window(0, 0, NT);
+            if (1 < nwin) load_bids(1);
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int rset = wave + W * u;
+                if (rset < SETS) {
+                    v8i hi, lo;
+                    const float inv = q_fp8_split(qf[u], qflip, hi, lo);
+                    unsigned char* x = exch + rset * kSetBytes + 16 * ln;
+                    *reinterpret_cast<u32x4_t*>(x) = (u32x4_t){(uint32_t)hi[0], (uint32_t)hi[1], (uint32_t)hi[2], (uint32_t)hi[3]};
+                    *reinterpret_cast<u32x4_t*>(x + 1024) = (u32x4_t){(uint32_t)hi[4], (uint32_t)hi[5], (uint32_t)hi[6], (uint32_t)hi[7]};
+                    *reinterpret_cast<u32x4_t*>(x + 2048) = (u32x4_t){(uint32_t)lo[0], (uint32_t)lo[1], (uint32_t)lo[2], (uint32_t)lo[3]};
+                    *reinterpret_cast<u32x4_t*>(x + 3072) = (u32x4_t){(uint32_t)lo[4], (uint32_t)lo[5], (uint32_t)lo[6], (uint32_t)lo[7]};
+                    *reinterpret_cast<float*>(exch + rset * kSetBytes + 4096 + 4 * ln) = inv;
+                }
+            }
+            lds_barrier();
+#pragma unroll
+            for (int j = 0; j < RS; ++j) {
+                const unsigned char* x = exch + (grp * RS + j) * kSetBytes + 16 * ln;
+                u32x4_t v[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) v[d] = *reinterpret_cast<const u32x4_t*>(x + 1024 * d);
+                qhi[j] = (v8i){(int)v[0][0], (int)v[0][1], (int)v[0][2], (int)v[0][3],
+                               (int)v[1][0], (int)v[1][1], (int)v[1][2], (int)v[1][3]};
+                qlo[j] = (v8i){(int)v[2][0], (int)v[2][1], (int)v[2][2], (int)v[2][3],
+                               (int)v[3][0], (int)v[3][1], (int)v[3][2], (int)v[3][3]};
+                qkr[j] = qk * *reinterpret_cast<const float*>(exch + (grp * RS + j) * kSetBytes + 4096 + 4 * ln);
+            }
+        }
 
         float m_run[RS], l_run[RS];
         f32x4_t o[RS][8];
@@ -891,6 +943,8 @@ prefill_split_kernel(Params P)
             if (i + RW < nwin) load_bids(i + RW);
         }
 
+        int ln = lane;                                 // opaque, as above
+        asm volatile("" : "+v"(ln));
         // ---- merge the NR partial states of each head group, then normalise and store ----------
         if constexpr (NR > 1) {
             // m_run is the same in the four lane groups of a query row: lanes 0..15 publish it.
@@ -909,51 +963,47 @@ prefill_split_kernel(Params P)
 #pragma unroll
                 for (int n = 0; n < 8; ++n) o[j][n] *= f;
             }
-            for (int r = 0; r < NR - 1; ++r) {
-                if (res == r) {
+            // Row-set j is summed and written by residue j % NR, so that the residues work side by side:
+            // every other one stores its state of j, and after one barrier the owner adds them in order.
 #pragma unroll
-                    for (int j = 0; j < RS; ++j) {
-                        float* s = stage + (grp * RS + j) * kStageFloats;
+            for (int j = 0; j < RS; ++j) {
+                if (res == j % NR) continue;
+                const int slot = (res - j % NR + NR) % NR - 1;
+                float* s = stage + (((grp * RS + j) * (NR - 1)) + slot) * kStageFloats;
 #pragma unroll
-                        for (int n = 0; n < 8; ++n) {
-                            f32x4_t* p = reinterpret_cast<f32x4_t*>(s + (n * 64 + lane) * 4);
-                            if (r > 0) o[j][n] += *p;
-                            *p = o[j][n];
-                        }
-                        if (r > 0) l_run[j] += s[8 * 64 * 4 + lane];
-                        s[8 * 64 * 4 + lane] = l_run[j];
-                    }
-                }
-                lds_barrier();
+                for (int n = 0; n < 8; ++n) *reinterpret_cast<f32x4_t*>(s + (n * 64 + ln) * 4) = o[j][n];
+                s[8 * 64 * 4 + ln] = l_run[j];
             }
-            if (res == NR - 1) {
+            lds_barrier();
 #pragma unroll
-                for (int j = 0; j < RS; ++j) {
-                    const float* s = stage + (grp * RS + j) * kStageFloats;
+            for (int j = 0; j < RS; ++j) {
+                if (res != j % NR) continue;
 #pragma unroll
-                    for (int n = 0; n < 8; ++n) o[j][n] += *reinterpret_cast<const f32x4_t*>(s + (n * 64 + lane) * 4);
-                    l_run[j] += s[8 * 64 * 4 + lane];
+                for (int r = 0; r < NR - 1; ++r) {
+                    const float* s = stage + ((grp * RS + j) * (NR - 1) + r) * kStageFloats;
+#pragma unroll
+                    for (int n = 0; n < 8; ++n) o[j][n] += *reinterpret_cast<const f32x4_t*>(s + (n * 64 + ln) * 4);
+                    l_run[j] += s[8 * 64 * 4 + ln];
                 }
             }
         }
-        if (res == NR - 1) {
 #pragma unroll
-            for (int j = 0; j < RS; ++j) {
-                const float l = sum_xor16_32(l_run[j]);
-                const int tok = token_of(j);
-                if (tok >= qlen || grp * RS + j >= nbt * P.gqa) continue;
-                const float f = l > 0.f ? vs / l : 0.f;
-                __bf16* orow = P.out + (int64_t)(q_begin + tok) * P.o_stride +
-                               (int64_t)(kh * P.gqa + rs_head[j]) * kD + 32 * lp;
+        for (int j = 0; j < RS; ++j) {
+            if (res != j % NR) continue;
+            const float l = sum_xor16_32(l_run[j]);
+            const int tok = token_of(j);
+            if (tok >= qlen || grp * RS + j >= nbt * P.gqa) continue;
+            const float f = l > 0.f ? vs / l : 0.f;
+            __bf16* orow = P.out + (int64_t)(q_begin + tok) * P.o_stride +
+                           (int64_t)(kh * P.gqa + head_of(grp * RS + j)) * kD + 32 * lp;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    u32x4_t w;
-                    w[0] = pack_bf16x2(o[j][0][e] * f, o[j][1][e] * f);
-                    w[1] = pack_bf16x2(o[j][2][e] * f, o[j][3][e] * f);
-                    w[2] = pack_bf16x2(o[j][4][e] * f, o[j][5][e] * f);
-                    w[3] = pack_bf16x2(o[j][6][e] * f, o[j][7][e] * f);
-                    *reinterpret_cast<u32x4_t*>(orow + 8 * e) = w;
-                }
+            for (int e = 0; e < 4; ++e) {
+                u32x4_t w;
+                w[0] = pack_bf16x2(o[j][0][e] * f, o[j][1][e] * f);
+                w[1] = pack_bf16x2(o[j][2][e] * f, o[j][3][e] * f);
+                w[2] = pack_bf16x2(o[j][4][e] * f, o[j][5][e] * f);
+                w[3] = pack_bf16x2(o[j][6][e] * f, o[j][7][e] * f);
+                *reinterpret_cast<u32x4_t*>(orow + 8 * e) = w;
             }
         }
         // The next block's copies overwrite the ring, which holds the stage: every wave must be
@@ -988,15 +1038,17 @@ inline int split_shape_for(int gqa)
     return -1;
 }
 
-// Default shape per GQA (measured at configs[3], GQA 6: 8 waves x 2 row-sets with paired token
-// blocks 184 us; 4 x 3 unpaired 251 us; 8 x 2 unpaired 190 us).
+// Default shape per GQA.  The per-wave kernel runs short contexts and batches of short prompts, many
+// more workgroups than CUs, so unpaired blocks, longest first, beat pairs and larger waves (8 waves x 2
+// row-sets, unpaired, against what GQA 6 / 12 took before: 6 prompts of 37..900 after 200 75 -> 55 /
+// 131 -> 93 us, 8 of 600 74 -> 59 / 130 -> 94, 12 of 50..400 34 -> 32 / 59 -> 46, 200 tokens alone 13.4 ->
+// 13.5 / 18.6 -> 13.7).
 inline int choose_shape(int gqa)
 {
     if (g_shape >= 0 && g_shape < kNumShapes) return g_shape;
     if (gqa <= 1) return 5;                       // 4 waves x 1 row-set, 4 token blocks
     if (gqa <= 2) return 4;                       // 4 waves x 2 row-sets, 4 token blocks
-    if (gqa <= 8) return 7;                       // 8 waves x 2 row-sets (paired blocks when nb = 2)
-    return 3;                                     // 4 waves x 4 row-sets
+    return 2;                                     // 8 waves x 2 row-sets
 }
 
 inline int plan_nb(int gqa, const Shape& s)
@@ -1020,13 +1072,16 @@ inline bool split_single_blocks_fit(int n16, int hkv, int num_seqs)
     return (int64_t)((n16 + per - 1) / per * per) * hkv * num_seqs <= kSplitRoundWorkgroups;
 }
 
-// Contexts (in keys) from which the key-split kernel beats the per-wave kernel, measured on MI355X
-// at GQA 6.  With paired blocks: 1024 (512 new tokens after 512 cached 42.8 vs 45.6 us, 512
-// tokens alone 28.0 vs 24.4 us; 4 sequences of 512 32.0 vs 27.3 us).  With one block per
-// workgroup (the grid fits one round): 256 (512 tokens alone 17.4 vs 23.8 us, 1000 alone 24.7 vs
-// 42.5 us, 64 after 900 22.3 vs 42.3 us, 256 alone 13.6 vs 14.4 us, 128 alone 13.1 vs 9.8 us).
-// Below them the split kernel's per-block fixed costs dominate.
+// Contexts (in keys) from which the key-split kernel beats the per-wave kernel, measured on MI355X.
+// With more single blocks than one round holds: 1024 (GQA 6: 3 of 300..1100 and longer; 6 of 37..900
+// after 200 take 59 us split and 55 per wave).  With one block per workgroup in one round: 256 (GQA
+// 6: 300 alone 14 vs 17 us, 1000 after 500 27.7 vs 63).  Below them the split kernel's work per block
+// before and after the keys dominates.
 constexpr int kSplitMinContext = 1024;
+// Shapes that split the keys two ways or not at all (GQA 8, 12, 16) merge less and start from here
+// (6 prompts of 37..900 after 200, GQA 8 / 12 / 6: 46 / 88 / 59 us against 58 / 93 / 55 per wave; 8 of 600:
+// 48 / 98 / 72 against 46 / 94 / 59).
+constexpr int kSplitMinContextFewParts = 768;
 constexpr int kSplitMinContextSingle = 256;
 
 // One launch as planned from the shape alone (no pointers): kernel, block pairing and grid.
@@ -1056,15 +1111,15 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
         split = (g_shape - kNumShapes) % kNumSplitShapes == ss;
         force_paired = g_shape >= kNumShapes + kNumSplitShapes;
     } else if (g_shape < 0 && ss >= 0) {
-        split = ctx_hint >= kSplitMinContext ||
+        split = ctx_hint >= (kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext) ||
                 (ctx_hint >= kSplitMinContextSingle && split_single_blocks_fit(n16, hkv, num_seqs));
     }
     if (split) {
         // Pairs of token blocks (r, n16 - 1 - r) give every workgroup the same causal work; when
         // one block per workgroup still fits in one round of workgroups (one per CU: the ring
         // takes most of the LDS), single blocks finish sooner (the longest workgroup sees about
-        // q0 + qlen keys instead of 2 q0 + qlen; measured at GQA 6: 1024 new tokens after 1024
-        // cached 61.3 -> 38.7 us, 512 after 1024 52.6 -> 30.0 us).
+        // q0 + qlen keys instead of 2 q0 + qlen; measured at GQA 6: 1000 new tokens after 500
+        // cached 41.8 -> 27.7 us).
         L.split = ss;
         L.nb = 2;
         L.paired = (force_paired || !split_single_blocks_fit(n16, hkv, num_seqs)) ? 1 : 0;
