@@ -89,10 +89,10 @@ void fp8kv_prefill_bf16_tune(int heads_per_wave);
 int fp8kv_prefill_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len,
                        int ctx_hint, int* out);
 
-/* Tuning hook for the MXFP4 x MXFP8 GEMM: kernel variant (0..18; any other value selects the
- * default, which picks from the shape; 9 + s is the K-splitting kernel with tile shape s, which K < 512
- * leaves to the default; the per-token entry point runs only 5, 6 and 9..18 and takes its default
- * for the others) and XCD split (0 = chosen by the traffic model, the
+/* Tuning hook for the MXFP4 x MXFP8 GEMM: kernel variant (0..19; any other value selects the
+ * default, which picks from the shape; 9 + s is the K-splitting kernel with tile shape s, 19 variant 5
+ * with two K groups of waves; K < 512 leaves those to the default; the per-token entry point runs
+ * only 5, 6 and 9..19 and takes its default for the others) and XCD split (0 = chosen by the traffic model, the
  * default; 1 = XCDs split the weight blocks only; 2 = XCDs split the token blocks as far as their
  * count allows).  Affects later launches. */
 void fp8kv_gemm_tune(int variant, int order);

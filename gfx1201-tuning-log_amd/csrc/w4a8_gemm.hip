@@ -56,6 +56,30 @@ thread_local int g_gemm_variant = kDefaultVariant;
 constexpr int64_t kGemmCus = 256;
 // 9 + s: the K-splitting kernel (w4a8_slice.hip) with tile shape s of kSliceShapes.
 constexpr int kSliceVariant = 9;
+// 19: variant 5's tiles with two K groups of waves (K % 512 == 0 and scales as for the grouped copies;
+// variant 5 itself otherwise).  Variant 5 takes it on its own for grids of at most one tile per CU.
+constexpr int kKGroupsVariant = kSliceVariant + kNumSliceShapes;
+
+constexpr int kCusPerXcd = 32;
+
+// Split of the XCDs (token blocks gm ways, weight blocks 8 / gm) under which every XCD has a CU for each
+// of its tiles, with the least traffic into the L2s (about (8 / gm) X + gm W bytes); 0 if there is none.
+inline int one_round_split(int nblk, int mblk, int N, int K, int M)
+{
+    int best = 0;
+    int64_t best_cost = 0;
+    for (int gm = 1; gm <= kXcds; gm *= 2) {
+        const int gn = kXcds / gm;
+        const int64_t tiles = (int64_t)((mblk + gm - 1) / gm) * ((nblk + gn - 1) / gn);
+        if (tiles > kCusPerXcd) continue;
+        const int64_t cost = (int64_t)gn * M * K + (int64_t)gm * N * (K / 2);
+        if (best == 0 || cost < best_cost) {
+            best = gm;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
 
 // The first slice shape whose tiles all run at once, one per CU, or -1.  In one round the smallest
 // tile that fits is the fastest: its waves have the fewest bytes to fetch (in a graph, per-token
@@ -68,7 +92,8 @@ inline int slice_shape(int N, int K, int M)
     if (K < kSliceMinK) return -1;
     for (int s = 0; s < kNumSliceShapes; ++s) {
         const int bn = 16 * kSliceShapes[s].tn, bm = 16 * kSliceShapes[s].tm;
-        if ((int64_t)((N + bn - 1) / bn) * ((M + bm - 1) / bm) <= kGemmCus) return s;
+        const int64_t nblk = ((int64_t)N + bn - 1) / bn, mblk = ((int64_t)M + bm - 1) / bm;
+        if (nblk * mblk <= kGemmCus && one_round_split((int)nblk, (int)mblk, N, K, M) > 0) return s;
     }
     return -1;
 }
@@ -320,24 +345,35 @@ struct LdsGeom {
 // P.tok_scale[m]); the activation-scale copies then read weight-scale rows of the tile (clamped
 // into the operand) so that every wave still issues the same copies and the waits stay exact.
 // GS: grouped scale copies (K % 512 == 0), as in gemm_big_kernel.
-template <int WN, int WM, int S, bool DB, bool TOK, bool GS>
+// KG: K groups of waves in a workgroup.  With two, the second WN * WM waves take the second half of the
+// k steps (whole scale groups) through a ring of their own in step with the first, and the first add
+// their accumulators at the end.
+template <int WN, int WM, int S, bool DB, bool TOK, bool GS, int KG = 1>
 __device__ __forceinline__ void gemm_lds_body(const Params& P)
 {
+    static_assert(KG == 1 || (KG == 2 && GS && !DB), "K groups start at a scale group");
     using G = LdsGeom<WN, WM, S>;
     constexpr int STAGE = GS ? G::OPER : G::STAGE;
     constexpr int DPW = GS ? (G::NW_W + G::NW_X) / G::NW : G::DPW;      // copies per wave and step
     constexpr int SG_ROWS = G::sg_rows(TOK), DPW_SG = G::dpw_sg(TOK);     // GS: copies per group
     constexpr int SG_BASE = S * G::OPER;
-    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int GROUP_LDS = SG_BASE + 2 * 16 * SG_ROWS;              // one K group's rings (GS)
+    extern __shared__ __align__(16) unsigned char smem_all[];
     int nb, mb;
     if (!tile_of(P, blockIdx.x, nb, mb)) return;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = KG > 1 ? wave_all / G::NW : 0;
+    const int wave = KG > 1 ? wave_all % G::NW : wave_all;
+    unsigned char* const smem = smem_all + (KG > 1 ? kg * GROUP_LDS : 0);
     const int r = lane & 15, j = lane >> 4;
     const int wn = wave % WN, wm = wave / WN;
     const int N0 = nb * G::BN, M0 = mb * G::BM;
     const int kh = P.K >> 1, ks = P.K >> 5;
-    const int nsteps = P.K / kBK;
+    const int all_steps = P.K / kBK;
+    // the first K group takes the larger half, so its step count is the workgroup's
+    const int half = KG > 1 ? ((all_steps >> 2) + 1) / 2 * 4 : all_steps;
+    const int step0 = kg * half, nsteps = kg ? all_steps - half : half;
 
     // This wave's DMA copies: copy c of wave w is copy d = c * NW + w of the stage, so the kind of
     // every copy (weight codes, activations, scales) is known at compile time (each kind's copy
@@ -387,8 +423,8 @@ __device__ __forceinline__ void gemm_lds_body(const Params& P)
     if constexpr (GS) sg.template setup<G::NW, G::BN, SG_ROWS, SG_BASE>(P, wave, lane, N0, M0, ks);
     auto issue = [&](int step) {
         unsigned char* stage = smem + (step % S) * STAGE;
-        const uint8_t* wb = wtile + (int64_t)step * 64;
-        const uint8_t* xb = xtile + (int64_t)step * 128;
+        const uint8_t* wb = wtile + (int64_t)(step0 + step) * 64;
+        const uint8_t* xb = xtile + (int64_t)(step0 + step) * 128;
 #pragma unroll
         for (int c = 0; c < DPW; ++c) {
             if (c < G::NW_W / G::NW) {
@@ -401,7 +437,7 @@ __device__ __forceinline__ void gemm_lds_body(const Params& P)
                 dma4_to_lds(sbase + loff[c], stage + ldsoff[c]);
             }
         }
-        if constexpr (GS) sg.template issue<SG_ROWS>(step, smem, swtile, sxtile);
+        if constexpr (GS) sg.template issue<SG_ROWS>(step, smem, swtile + (int64_t)step0 * 4, sxtile + (int64_t)step0 * 4);
     };
     // fragment reads: one lane base per kind, tiles at constant offsets from it
     const int abase = (wn * 64 + r) * 64 + 16 * j;
@@ -471,6 +507,24 @@ __device__ __forceinline__ void gemm_lds_body(const Params& P)
             sync_read(f, s);
             compute<TOK>(f, acc, j);
         }
+        if constexpr (KG > 1) {
+            // the second group, at most one scale group shorter, keeps the first one's barriers company
+            for (int s = nsteps; s < half; ++s) lds_barrier_all();
+            lds_barrier_all();                             // every ring is read
+            f32x4_t* const part = reinterpret_cast<f32x4_t*>(smem_all) + wave * (16 * 64) + lane;
+            if (kg) {
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) part[(4 * a + b) * 64] = acc[a][b];
+            }
+            lds_barrier_all();
+            if (kg) return;
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) acc[a][b] += part[(4 * a + b) * 64];
+        }
     }
 
     const int n0 = N0 + wn * 64, m0 = M0 + wm * 64;
@@ -517,6 +571,16 @@ __global__ void __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_
 gemm_lds2_kernel(Params P)
 {
     gemm_lds_body<WN, WM, S, false, TOK, GS>(P);
+}
+
+// Two K groups of four waves (see gemm_lds_body): 128 x 128 tiles that do not give every CU two
+// workgroups.  A lone one has one wave per SIMD, and each step then costs a whole copy latency;
+// two halves of K side by side hide each other's waits as two workgroups do.
+template <bool TOK>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_lds2_kgroups_kernel(Params P)
+{
+    gemm_lds_body<2, 2, 2, false, TOK, true, 2>(P);
 }
 
 // ---- larger wave tiles -------------------------------------------------------------------------
@@ -915,7 +979,6 @@ inline bool has_token_variant(int v) { return v == 5 || v == 6 || v >= kSliceVar
 
 constexpr int64_t kL2Bytes = (int64_t)4 << 20;        // per XCD
 constexpr int kLdsPerCu = 160 * 1024;
-constexpr int kCusPerXcd = 32;
 
 // Split of the 8 XCDs between token blocks (gm ways) and weight blocks (gn = 8 / gm ways).  The
 // XCDs of one token group read its activations, those of one weight group its weights, so a
@@ -955,12 +1018,13 @@ int pick_split(const Params& P, int BM, int lds_bytes, bool act_scales)
 
 int launch_gemm(Params& P, int variant, bool tok, hipStream_t st)
 {
-    if (variant >= kSliceVariant) {
+    if (variant >= kSliceVariant && variant < kKGroupsVariant) {
         const SliceShape sh = kSliceShapes[variant - kSliceVariant];
         P.nblk = (P.N + 16 * sh.tn - 1) / (16 * sh.tn);
         P.mblk = (P.M + 16 * sh.tm - 1) / (16 * sh.tm);
         if ((int64_t)P.nblk * P.mblk > 0x7FFFFFFF - kXcds) return FP8KV_ERR_SHAPE;
-        P.gm = pick_split(P, 16 * sh.tm, kLdsPerCu, !tok);
+        const int one = one_round_split(P.nblk, P.mblk, P.N, P.K, P.M);
+        P.gm = one > 0 ? one : pick_split(P, 16 * sh.tm, kLdsPerCu, !tok);
         P.gn = kXcds / P.gm;
         const int64_t per = (int64_t)((P.mblk + P.gm - 1) / P.gm) * ((P.nblk + P.gn - 1) / P.gn);
         begin_launch();
@@ -985,12 +1049,22 @@ int launch_gemm(Params& P, int variant, bool tok, hipStream_t st)
                   : variant == 2 || variant == 4 ? (gs ? LdsGeom<2, 2, 3>::lds_gs(tok) : LdsGeom<2, 2, 3>::LDS)
                   : variant == 3 ? (gs ? LdsGeom<2, 2, 5>::lds_gs(tok) : LdsGeom<2, 2, 5>::LDS)
                   : (gs ? LdsGeom<2, 2, 2>::lds_gs(tok) : LdsGeom<2, 2, 2>::LDS);
-    const int gm = pick_split(P, BM, lds, !tok);
+    // 128 x 128 tiles, at most one per CU: K groups (in a graph, per-token, us: N = 3584, K = 18944, 1000
+    // rows 98.7 -> 81.7; N = 4096, K = 3584 24.3 -> 21.3; past one round the workgroups pair up by
+    // themselves: 1500 rows 118 / 157)
+    const int one = one_round_split(P.nblk, P.mblk, P.N, P.K, P.M);
+    const bool kgroups = gs && P.K >= 2 * kSliceMinK && (variant == kKGroupsVariant || (variant == 5 && one > 0));
+    const int gm = kgroups && one > 0 ? one : pick_split(P, BM, lds, !tok);
     P.gm = gm;
     P.gn = kXcds / gm;
     const int64_t per_xcd = (int64_t)((P.mblk + gm - 1) / gm) * ((P.nblk + P.gn - 1) / P.gn);
     const int64_t grid = per_xcd * kXcds;
     begin_launch();
+    if (kgroups) {
+        if (tok) launch_kernel(gemm_lds2_kgroups_kernel<true>, dim3((unsigned)grid), dim3(512), 2 * lds, st, P);
+        else launch_kernel(gemm_lds2_kgroups_kernel<false>, dim3((unsigned)grid), dim3(512), 2 * lds, st, P);
+        return finish_launch();
+    }
     if (tok) {
         if (variant == 6 && gs)
             launch_kernel(gemm_big_kernel<2, 2, 8, 4, 2, true, true>, dim3((unsigned)grid), dim3(256), lds, st, P);
@@ -1140,6 +1214,6 @@ extern "C" int h4a8_gemm_token(const void* W, const void* St, const void* Xq, co
 
 extern "C" void fp8kv_gemm_tune(int variant, int order)
 {
-    fp8kv::w4a8_detail::g_gemm_variant = (variant >= 0 && variant < kSliceVariant + kNumSliceShapes) ? variant : -1;
+    fp8kv::w4a8_detail::g_gemm_variant = (variant >= 0 && variant <= kKGroupsVariant) ? variant : -1;
     fp8kv::w4a8_detail::g_gemm_order = (order == 1 || order == 2) ? order : 0;
 }

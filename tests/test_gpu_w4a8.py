@@ -97,6 +97,26 @@ def test_slice_kernel_parity(shape, act, N, K, M):
     assert matvec.bf16_excess_error(out.float().cpu().numpy(), ref) < 1e-4
 
 
+@pytest.mark.parametrize("act", ["mx", "token"])
+@pytest.mark.parametrize("N,K,M", [(128, 1024, 128), (260, 1536, 129), (132, 3584, 65), (640, 18944, 700)])
+def test_k_groups_parity(act, N, K, M):
+    """Two K groups of waves: two scale groups (K = 1024), halves of unequal length (1536: 8 and 4
+    steps; 3584: 16 and 12; 18944: 76 and 72), partial tiles, and the repeat bit for bit."""
+    lib = _lib.load()
+    c, rc, rs = (_token_case if act == "token" else _gemm_case)(N, K, M, seed=N + M)
+    ref = (w4a8.gemm_token if act == "token" else w4a8.gemm)(c["W"].numpy(), c["St"].numpy(), rc, rs)
+    args = [torch.from_numpy(rc).to(DEV), torch.from_numpy(rs).to(DEV), c["W"].to(DEV), c["St"].to(DEV)]
+    gemm = ops.h4a8_gemm_token if act == "token" else ops.h4a8_gemm
+    try:
+        lib.fp8kv_gemm_tune(19, 0)
+        out, again = gemm(*args).clone(), gemm(*args)
+        torch.cuda.synchronize()
+    finally:
+        lib.fp8kv_gemm_tune(-1, 0)
+    assert torch.equal(out, again)
+    assert matvec.bf16_excess_error(out.float().cpu().numpy(), ref) < 1e-4
+
+
 @pytest.mark.parametrize("variant", [-1, 5, 6, 8])
 def test_gemm_scales_only_4_byte_aligned(variant):
     """Scale operands that start 4 bytes past a 16-byte boundary (the entry point requires 4): the
