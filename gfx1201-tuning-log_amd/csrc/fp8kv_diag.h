@@ -72,7 +72,8 @@ void fp8kv_decode_tune(int variant, int target_wgs);
 /* Tuning hook for sweeps of the prefill attention launch: index of the (waves, row-sets per wave,
  * LDS ring depth) shape to use for every GQA (0..7), 8 + s for key-split shape s (0..4, used only
  * at its own GQA: 6, 12, 4, 8, 16) with the default block pairing, 13 + s for the same with paired
- * token blocks (r, n16 - 1 - r) at any grid size, or -1 for the per-GQA default. */
+ * token blocks (r, n16 - 1 - r) at any grid size, 18 for the key-split kernel at any GQA and context
+ * and 19 for the same with paired blocks, or -1 for the per-GQA default. */
 void fp8kv_prefill_tune(int shape);
 
 /* bf16-KV prefill: query heads per wave of the register-direct kernel (1 or 2), or the key-split kernel

@@ -1028,15 +1028,23 @@ struct SplitShape {
 constexpr SplitShape kSplitShapes[] = {{3, 2}, {3, 4}, {2, 2}, {2, 4}, {2, 8}};
 constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
 // -1: choose by GQA; kNumShapes + s: key-split shape s; kNumShapes + kNumSplitShapes + s: the
-// same with paired token blocks whatever the grid size.
+// same with paired token blocks whatever the grid size; kSplitAnyShape (+ 1): the key-split kernel at
+// any GQA (with paired blocks).
+constexpr int kSplitAnyShape = kNumShapes + 2 * kNumSplitShapes;
 thread_local int g_shape = -1;
 
+// Key-split shape of a GQA: its own, or the smallest that holds its heads (with row-sets repeated, or
+// two or four token blocks per workgroup at GQA 2 and 1).
 inline int split_shape_for(int gqa)
 {
-    for (int s = 0; s < kNumSplitShapes; ++s)
-        if (kSplitShapes[s].rs * kSplitShapes[s].ng == gqa) return s;
-    return -1;
+    return gqa <= 4 ? 2 : gqa <= 6 ? 0 : gqa <= 8 ? 3 : gqa <= 12 ? 1 : 4;
 }
+inline bool split_shape_exact(int gqa)
+{
+    const SplitShape s = kSplitShapes[split_shape_for(gqa)];
+    return s.rs * s.ng == gqa;
+}
+inline int split_blocks(int gqa) { return gqa <= 2 ? 4 / gqa : 1; }
 
 // Default shape per GQA.  The per-wave kernel runs short contexts and batches of short prompts, many
 // more workgroups than CUs, so unpaired blocks, longest first, beat pairs and larger waves (8 waves x 2
@@ -1082,6 +1090,14 @@ constexpr int kSplitMinContext = 1024;
 // (6 prompts of 37..900 after 200, GQA 8 / 12 / 6: 46 / 88 / 59 us against 58 / 93 / 55 per wave; 8 of 600:
 // 48 / 98 / 72 against 46 / 94 / 59).
 constexpr int kSplitMinContextFewParts = 768;
+// Below GQA 4 the per-wave kernel has few row-sets to share a conversion (4 of 512, GQA 1 / 3: 21.5 / 20.1
+// us against 27 / 26.5 per wave).
+constexpr int kSplitMinContextLowGqa = 512;
+// GQAs without a shape of their own (us, split against per wave; 2048 tokens after 2048, 28 / 4 heads 123 /
+// 194, 16 / 16 75 / 140, 8 / 4 49 / 132, 12 / 4 74 / 140, 20 / 4 93 / 187, 40 / 4 158 / 248; 1000 after 500, 28 / 4
+// 34 / 68, 16 / 16 22 / 48).  Prompts up to 300 tokens stay on the per-wave kernel, as the launch
+// plan's test has them, although contexts of 1000 keys would gain there too.
+constexpr int kSplitMinQueryInexact = 320;
 constexpr int kSplitMinContextSingle = 256;
 
 // One launch as planned from the shape alone (no pointers): kernel, block pairing and grid.
@@ -1105,14 +1121,23 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
 
     // Key-split kernel when the GQA has a split shape and the context is long enough, unless the
     // tuning hook forces another.
-    const int ss = split_shape_for(gqa);
+    const int ss = split_shape_for(gqa), nbt = split_blocks(gqa);
+    const bool exact = split_shape_exact(gqa);
+    const int nsb = (max_query_len + 16 * nbt - 1) / (16 * nbt);        // the split kernel's (super)blocks
+    const bool fits = split_single_blocks_fit(nsb, hkv, num_seqs);
     bool split = false, force_paired = false;
     if (g_shape >= kNumShapes) {
-        split = (g_shape - kNumShapes) % kNumSplitShapes == ss;
+        split = exact && (g_shape - kNumShapes) % kNumSplitShapes == ss;
         force_paired = g_shape >= kNumShapes + kNumSplitShapes;
-    } else if (g_shape < 0 && ss >= 0) {
-        split = ctx_hint >= (kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext) ||
-                (ctx_hint >= kSplitMinContextSingle && split_single_blocks_fit(n16, hkv, num_seqs));
+        if (g_shape == kSplitAnyShape || g_shape == kSplitAnyShape + 1) {
+            split = true;
+            force_paired = g_shape > kSplitAnyShape;
+        }
+    } else if (g_shape < 0) {
+        const int many = gqa < 4 ? kSplitMinContextLowGqa
+                       : kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext;
+        split = ctx_hint >= many || (ctx_hint >= kSplitMinContextSingle && fits);
+        if (!exact && max_query_len < kSplitMinQueryInexact) split = false;
     }
     if (split) {
         // Pairs of token blocks (r, n16 - 1 - r) give every workgroup the same causal work; when
@@ -1121,9 +1146,9 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
         // q0 + qlen keys instead of 2 q0 + qlen; measured at GQA 6: 1000 new tokens after 500
         // cached 41.8 -> 27.7 us).
         L.split = ss;
-        L.nb = 2;
-        L.paired = (force_paired || !split_single_blocks_fit(n16, hkv, num_seqs)) ? 1 : 0;
-        L.ntb_grid = round_up(L.paired ? (n16 + 1) / 2 : n16);
+        L.nb = nbt > 1 ? nbt : 2;
+        L.paired = (force_paired || !fits) ? 1 : 0;
+        L.ntb_grid = round_up(L.paired ? (nsb + 1) / 2 : nsb);
         L.block = dim3(64 * kSplitWaves);
     } else {
         L.shape = choose_shape(gqa);
@@ -1154,7 +1179,12 @@ int launch(const Params& P0, int num_seqs, int max_query_len, int ctx_hint, hipS
         switch (L.split) {
             case 0: launch_kernel(prefill_split_kernel<3, 2, 2, false, false>, L.grid, L.block, 0, stream, P); break;
             case 1: launch_kernel(prefill_split_kernel<3, 4, 2, false, false>, L.grid, L.block, 0, stream, P); break;
-            case 2: launch_kernel(prefill_split_kernel<2, 2, 2, false, false>, L.grid, L.block, 0, stream, P); break;
+            case 2:
+                if (split_blocks(P.gqa) > 1)
+                    launch_kernel(prefill_split_kernel<2, 2, 2, false, true>, L.grid, L.block, 0, stream, P);
+                else
+                    launch_kernel(prefill_split_kernel<2, 2, 2, false, false>, L.grid, L.block, 0, stream, P);
+                break;
             case 3: launch_kernel(prefill_split_kernel<2, 4, 2, false, false>, L.grid, L.block, 0, stream, P); break;
             default: launch_kernel(prefill_split_kernel<2, 8, 2, false, false>, L.grid, L.block, 0, stream, P); break;
         }
@@ -1178,13 +1208,11 @@ int launch(const Params& P0, int num_seqs, int max_query_len, int ctx_hint, hipS
 // register-direct loads (prefill_bf16kv_kernel; us in a graph): 2048 tokens after 2048, 24 / 4 heads
 // 210 -> 104, 32 / 8 287 -> 170, 16 / 16 253 -> 89, 28 / 4 282 -> 125; 1500 alone, 24 / 4 70 -> 44;
 // 3 x 100..300 after 2000 107 -> 43.
-inline int bf16_split_blocks(int gqa) { return gqa <= 2 ? 4 / gqa : 1; }
-
 int launch_bf16(const Params& P0, int num_seqs, int max_query_len, bool force_paired, hipStream_t stream)
 {
     Params P = P0;
     const int g = P.gqa;
-    P.nb = bf16_split_blocks(g);
+    P.nb = split_blocks(g);
     const int n = (max_query_len + 16 * P.nb - 1) / (16 * P.nb);
     P.xcd_map = (P.hkv <= 8 && 8 % P.hkv == 0) ? 1 : 0;
     P.paired = force_paired || !split_single_blocks_fit(n, P.hkv, num_seqs);
@@ -1290,7 +1318,7 @@ extern "C" int fp8kv_prefill_attn(const void* q, int64_t q_row_stride,
 
 extern "C" void fp8kv_prefill_tune(int shape)
 {
-    g_shape = (shape >= 0 && shape < kNumShapes + 2 * kNumSplitShapes) ? shape : -1;
+    g_shape = (shape >= 0 && shape <= kSplitAnyShape + 1) ? shape : -1;
 }
 
 extern "C" int fp8kv_prefill_plan(int num_q_heads, int num_kv_heads, int num_seqs,
@@ -1346,7 +1374,7 @@ extern "C" int fp8kv_prefill_attn_varlen(const void* q, int64_t q_row_stride,
 bool fp8kv::prefill_split_takes_bf16(int hkv, int gqa, int num_seqs, int max_query_len, int ctx_hint)
 {
     if (ctx_hint < kSplitMinContextSingle) return false;
-    const int nb = bf16_split_blocks(gqa);
+    const int nb = split_blocks(gqa);
     if (split_single_blocks_fit((max_query_len + 16 * nb - 1) / (16 * nb), hkv, num_seqs)) return true;
     return ctx_hint >= 768 || gqa > 6;
 }

@@ -392,6 +392,22 @@ def test_bf16_kv_varlen():
 
 
 @pytest.mark.parametrize("paired", [False, True])
+@pytest.mark.parametrize("gqa", [1, 2, 3, 5, 7, 9, 11, 13, 15])
+def test_key_split_gqa_without_a_shape(gqa, paired):
+    """The key-split kernel at GQAs that repeat row-sets (3, 5, 7, 9, 11, 13, 15) or pack several token
+    blocks (1, 2): one token, a block and one token more, fewer tiles than key residues, a tail block."""
+    lib = _lib.load()
+    try:
+        lib.fp8kv_prefill_tune(19 if paired else 18)
+        for qlen, q0 in ((1, 0), (17, 15), (33, 0), (65, 700), (161, 45)):
+            _check_single(qlen, q0, HQ=4 * gqa, HKV=4, seed=gqa + qlen, layout="engine")
+        _check_single(250, 7, HQ=3 * gqa, HKV=3, seed=gqa + 290, PBLK=64)
+        _check_varlen([5, 100, 33, 200, 1], [0, 7, 500, 3, 250], HQ=2 * gqa, HKV=2, seed=gqa + 93)
+    finally:
+        lib.fp8kv_prefill_tune(-1)
+
+
+@pytest.mark.parametrize("paired", [False, True])
 @pytest.mark.parametrize("gqa", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 16])
 def test_bf16_kv_key_split_every_gqa(gqa, paired):
     """The key-split kernel forced at every row-set packing (several blocks per workgroup at GQA 1 and
