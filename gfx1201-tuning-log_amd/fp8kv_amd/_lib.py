@@ -112,6 +112,8 @@ def lib_path() -> str:
 def load() -> ctypes.CDLL:
     """Load (once) and type the library; raises if it is missing."""
     global _lib
+    if _lib is not None:                     # set once, complete
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

@@ -10,25 +10,30 @@ import torch
 from . import _lib
 
 
+# The wrappers run once per layer and step, so their host time is a decode step's floor.  Checks are
+# written out (a message is formatted when its check fails, not on every call) and the current
+# stream's handle is read without building a Stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.device.index)
     return torch.cuda.current_stream(t.device).cuda_stream
-
-
-def _require(cond: bool, msg: str) -> None:
-    if not cond:
-        raise ValueError(msg)
 
 
 def repack_scales(weight_scale: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """Checkpoint scales uint8 [K/32, N] -> kernel layout [N, K/32] on the device
     (h4mv_repack_scales; the reference's weight_scale.t().contiguous(), h4mv/fp8kv_hipw4.py:32-43)."""
-    _require(weight_scale.is_cuda and weight_scale.dim() == 2 and weight_scale.is_contiguous()
-             and weight_scale.element_size() == 1, "weight_scale must be a contiguous 1-byte [K/32, N] device tensor")
+    if not (weight_scale.is_cuda and weight_scale.dim() == 2 and weight_scale.is_contiguous() and
+            weight_scale.element_size() == 1):
+        raise ValueError("weight_scale must be a contiguous 1-byte [K/32, N] device tensor")
     G, N = weight_scale.shape
     if out is None:
         out = torch.empty((N, G), dtype=weight_scale.dtype, device=weight_scale.device)
-    _require(out.shape == (N, G) and out.is_contiguous() and out.element_size() == 1
-             and out.device == weight_scale.device, "out must be a contiguous [N, K/32] byte tensor")
+    if not (out.shape == (N, G) and out.is_contiguous() and out.element_size() == 1 and out.device
+            == weight_scale.device):
+        raise ValueError("out must be a contiguous [N, K/32] byte tensor")
     lib = _lib.load()
     st = lib.h4mv_repack_scales(weight_scale.data_ptr(), out.data_ptr(), N, 32 * G,
                                 _stream_ptr(weight_scale))
@@ -43,22 +48,26 @@ def h4mv(x: torch.Tensor, weight: torch.Tensor, scales_nk: torch.Tensor,
     Same contract as the reference's ``lib.h4mv_launch`` call in h4mv/fp8kv_hipw4.py:78-83;
     ``out_dtype=torch.float32`` selects the unrounded fp32-output entry point.
     """
-    _require(x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous(),
-             "x must be a contiguous 2-D bf16 device tensor")
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()):
+        raise ValueError("x must be a contiguous 2-D bf16 device tensor")
     M, K = x.shape
-    _require(weight.dtype == torch.uint8 and weight.dim() == 2 and weight.is_contiguous(),
-             "weight must be contiguous uint8 [N, K/2]")
+    if not (weight.dtype == torch.uint8 and weight.dim() == 2 and weight.is_contiguous()):
+        raise ValueError("weight must be contiguous uint8 [N, K/2]")
     N = weight.shape[0]
-    _require(weight.shape[1] * 2 == K, f"weight {tuple(weight.shape)} does not match K={K}")
-    _require(scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32)
-             and scales_nk.is_contiguous(), f"scales must be contiguous uint8 [{N}, {K // 32}]")
-    _require(weight.device == x.device == scales_nk.device, "tensors on different devices")
-    _require(out_dtype in (torch.bfloat16, torch.float32), "out_dtype must be bf16 or fp32")
+    if not (weight.shape[1] * 2 == K):
+        raise ValueError(f"weight {tuple(weight.shape)} does not match K={K}")
+    if not (scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and
+            scales_nk.is_contiguous()):
+        raise ValueError(f"scales must be contiguous uint8 [{N}, {K // 32}]")
+    if not (weight.device == x.device == scales_nk.device):
+        raise ValueError("tensors on different devices")
+    if not (out_dtype in (torch.bfloat16, torch.float32)):
+        raise ValueError("out_dtype must be bf16 or fp32")
     if out is None:
-        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
+        out = x.new_empty((M, N), dtype=out_dtype)
     else:
-        _require(out.dtype == out_dtype and tuple(out.shape) == (M, N) and out.is_contiguous(),
-                 f"out must be contiguous {out_dtype} [M, N]")
+        if not (out.dtype == out_dtype and tuple(out.shape) == (M, N) and out.is_contiguous()):
+            raise ValueError(f"out must be contiguous {out_dtype} [M, N]")
     lib = _lib.load()
     fn = lib.h4mv_launch_status if out_dtype == torch.bfloat16 else lib.h4mv_f32_launch_status
     st = fn(weight.data_ptr(), scales_nk.data_ptr(), x.data_ptr(), out.data_ptr(), N, K, M,
@@ -120,7 +129,8 @@ def decode_scratch(nbytes: int, device, allow_alloc: bool = True) -> torch.Tenso
 def decode_scratch_reset(scratch: torch.Tensor) -> None:
     """Zero a decode scratch buffer on the current stream with the library's fill kernel
     (fp8kv_decode_scratch_reset): for a buffer whose last call did not complete."""
-    _require(scratch.is_cuda and scratch.is_contiguous(), "scratch must be a contiguous device tensor")
+    if not (scratch.is_cuda and scratch.is_contiguous()):
+        raise ValueError("scratch must be a contiguous device tensor")
     st = _lib.load().fp8kv_decode_scratch_reset(scratch.data_ptr(), scratch.numel() * scratch.element_size(),
                                                 _stream_ptr(scratch))
     _lib.check("fp8kv_decode_scratch_reset", st)
@@ -132,16 +142,19 @@ def _ptr(t: torch.Tensor | None):
 
 def _scale_tensor(x, device) -> torch.Tensor:
     if torch.is_tensor(x):
-        _require(x.dtype == torch.float32 and x.numel() >= 1 and x.device == device,
-                 "k/v scales must be fp32 device tensors")
+        if not (x.dtype == torch.float32 and x.numel() >= 1 and x.device == device):
+            raise ValueError("k/v scales must be fp32 device tensors")
         return x
     return torch.tensor([float(x)], dtype=torch.float32, device=device)
 
 
 def _fp8_cache_check(c: torch.Tensor, name: str) -> None:
-    _require(c.is_cuda and c.dim() == 4, f"{name} must be a 4-D device tensor [NB, PBLK, HKV, D]")
-    _require(c.dtype in (torch.float8_e4m3fn, torch.uint8), f"{name} must be float8_e4m3fn (or raw uint8)")
-    _require(c.stride(3) == 1, f"{name} must be contiguous along head_size")
+    if not (c.is_cuda and c.dim() == 4):
+        raise ValueError(f"{name} must be a 4-D device tensor [NB, PBLK, HKV, D]")
+    if not (c.dtype in (torch.float8_e4m3fn, torch.uint8)):
+        raise ValueError(f"{name} must be float8_e4m3fn (or raw uint8)")
+    if not (c.stride(3) == 1):
+        raise ValueError(f"{name} must be contiguous along head_size")
 
 
 def _kv_caches_bf16(k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
@@ -149,9 +162,9 @@ def _kv_caches_bf16(k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
     e4m3 ones (float8_e4m3fn or raw uint8); both caches must agree."""
     if k_cache.dtype == torch.bfloat16 or v_cache.dtype == torch.bfloat16:
         for c, n in ((k_cache, "k_cache"), (v_cache, "v_cache")):
-            _require(c.is_cuda and c.dim() == 4 and c.dtype == torch.bfloat16 and c.stride(3) == 1,
-                     f"{n} must be a 4-D bf16 device tensor [NB, PBLK, HKV, D] contiguous along "
-                     "head_size (both caches bf16, or both e4m3)")
+            if not (c.is_cuda and c.dim() == 4 and c.dtype == torch.bfloat16 and c.stride(3) == 1):
+                raise ValueError(f"{n} must be a 4-D bf16 device tensor [NB, PBLK, HKV, D] contiguous along "
+                                 "head_size (both caches bf16, or both e4m3)")
         return True
     _fp8_cache_check(k_cache, "k_cache")
     _fp8_cache_check(v_cache, "v_cache")
@@ -171,16 +184,19 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     ``num_splits`` defaults to the library's plan for ``max_seq_len`` (read from ``seq_lens`` when
     not given, which synchronises).  ``scratch`` defaults to a per-device cached buffer.
     """
-    _require(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.stride(2) == 1
-             and q.stride(1) == q.shape[2], "q must be bf16 [T, HQ, D] with contiguous heads")
-    _require(out.dtype == torch.bfloat16 and out.dim() == 3 and out.stride(2) == 1
-             and out.stride(1) == out.shape[2] and out.shape[1:] == q.shape[1:],
-             "out must be bf16 [T, HQ, D] with contiguous heads")
+    if not (q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.stride(2) == 1 and
+            q.stride(1) == q.shape[2]):
+        raise ValueError("q must be bf16 [T, HQ, D] with contiguous heads")
+    if not (out.dtype == torch.bfloat16 and out.dim() == 3 and out.stride(2) == 1 and out.stride(1)
+            == out.shape[2] and out.shape[1:] == q.shape[1:]):
+        raise ValueError("out must be bf16 [T, HQ, D] with contiguous heads")
     bf16_kv = _kv_caches_bf16(k_cache, v_cache)
     for t, n in ((query_start_loc, "query_start_loc"), (seq_lens, "seq_lens"),
                  (block_table, "block_table")):
-        _require(t.dtype == torch.int32 and t.is_cuda, f"{n} must be an int32 device tensor")
-    _require(block_table.dim() == 2 and block_table.stride(1) == 1, "block_table must be [NS, max_blocks]")
+        if not (t.dtype == torch.int32 and t.is_cuda):
+            raise ValueError(f"{n} must be an int32 device tensor")
+    if not (block_table.dim() == 2 and block_table.stride(1) == 1):
+        raise ValueError("block_table must be [NS, max_blocks]")
     NS = block_table.shape[0]
     HQ, D = q.shape[1], q.shape[2]
     HKV = k_cache.shape[2]
@@ -196,8 +212,8 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if scratch is None:
         scratch = decode_scratch(need, dev)
     elif need > 0:
-        _require(scratch.is_cuda and scratch.numel() * scratch.element_size() >= need,
-                 f"scratch needs {need} bytes")
+        if not (scratch.is_cuda and scratch.numel() * scratch.element_size() >= need):
+            raise ValueError(f"scratch needs {need} bytes")
     sbytes = 0 if scratch is None else scratch.numel() * scratch.element_size()
     lib = _lib.load()
     name = "fp8kv_decode_attn_bf16" if bf16_kv else "fp8kv_decode_attn"
@@ -216,14 +232,16 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
 # ------------------------------------------------------------------------------ prefill attention
 
 def _prefill_common(q, k_cache, v_cache, out, block_table):
-    _require(q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.stride(2) == 1
-             and q.stride(1) == q.shape[2], "q must be bf16 [T, HQ, D] with contiguous heads")
-    _require(out.dtype == torch.bfloat16 and out.dim() == 3 and out.stride(2) == 1
-             and out.stride(1) == out.shape[2] and out.shape[1:] == q.shape[1:],
-             "out must be bf16 [T, HQ, D] with contiguous heads")
+    if not (q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.stride(2) == 1 and
+            q.stride(1) == q.shape[2]):
+        raise ValueError("q must be bf16 [T, HQ, D] with contiguous heads")
+    if not (out.dtype == torch.bfloat16 and out.dim() == 3 and out.stride(2) == 1 and out.stride(1)
+            == out.shape[2] and out.shape[1:] == q.shape[1:]):
+        raise ValueError("out must be bf16 [T, HQ, D] with contiguous heads")
     bf16_kv = _kv_caches_bf16(k_cache, v_cache)
-    _require(block_table.dtype == torch.int32 and block_table.is_cuda and block_table.dim() == 2
-             and block_table.stride(1) == 1, "block_table must be int32 [NS, max_blocks] on the device")
+    if not (block_table.dtype == torch.int32 and block_table.is_cuda and block_table.dim() == 2 and
+            block_table.stride(1) == 1):
+        raise ValueError("block_table must be int32 [NS, max_blocks] on the device")
     return bf16_kv
 
 
@@ -237,7 +255,8 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     bf16 caches take the reference's K_FP8 = False branch (fp8kv_prefill.py:143): no scales.
     """
     bf16_kv = _prefill_common(q, k_cache, v_cache, out, block_table)
-    _require(0 <= qlen <= q.shape[0] and qlen <= out.shape[0] and q0 >= 0, "bad q0 / qlen")
+    if not (0 <= qlen <= q.shape[0] and qlen <= out.shape[0] and q0 >= 0):
+        raise ValueError("bad q0 / qlen")
     dev = q.device
     ks = None if bf16_kv else _scale_tensor(k_scale, dev)
     vs = None if bf16_kv else _scale_tensor(v_scale, dev)
@@ -265,9 +284,11 @@ def prefill_attention_varlen(q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     """
     bf16_kv = _prefill_common(q, k_cache, v_cache, out, block_table)
     for t, n in ((cu_seqlens_q, "cu_seqlens_q"), (seq_lens, "seq_lens")):
-        _require(t.dtype == torch.int32 and t.is_cuda, f"{n} must be an int32 device tensor")
+        if not (t.dtype == torch.int32 and t.is_cuda):
+            raise ValueError(f"{n} must be an int32 device tensor")
     NS = block_table.shape[0]
-    _require(cu_seqlens_q.numel() == NS + 1 and seq_lens.numel() == NS, "metadata sizes differ")
+    if not (cu_seqlens_q.numel() == NS + 1 and seq_lens.numel() == NS):
+        raise ValueError("metadata sizes differ")
     if max_query_len is None:
         max_query_len = int((cu_seqlens_q[1:] - cu_seqlens_q[:-1]).max().item()) if NS else 0
     dev = q.device
@@ -295,16 +316,18 @@ def cache_write(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     any block / slot / head strides, the layouts the attention wrappers take).  The semantics of
     vLLM's reshape_and_cache_flash with an fp8 cache."""
     for t, n in ((key, "key"), (value, "value")):
-        _require(t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 3 and t.stride(2) == 1
-                 and t.stride(1) == t.shape[2], f"{n} must be bf16 [T, HKV, D] with contiguous heads")
-    _require(key.shape == value.shape, "key and value must have the same shape")
+        if not (t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 3 and t.stride(2) == 1 and
+                t.stride(1) == t.shape[2]):
+            raise ValueError(f"{n} must be bf16 [T, HKV, D] with contiguous heads")
+    if not (key.shape == value.shape):
+        raise ValueError("key and value must have the same shape")
     _fp8_cache_check(k_cache, "k_cache")
     _fp8_cache_check(v_cache, "v_cache")
-    _require(k_cache.shape[1:] == v_cache.shape[1:] and k_cache.shape[2:] == key.shape[1:],
-             "caches must be [NB, PBLK, HKV, D] matching key")
-    _require(slot_mapping.is_cuda and slot_mapping.dtype == torch.int64 and slot_mapping.dim() == 1
-             and slot_mapping.shape[0] == key.shape[0] and slot_mapping.stride(0) == 1,
-             "slot_mapping must be an int64 device tensor [T]")
+    if not (k_cache.shape[1:] == v_cache.shape[1:] and k_cache.shape[2:] == key.shape[1:]):
+        raise ValueError("caches must be [NB, PBLK, HKV, D] matching key")
+    if not (slot_mapping.is_cuda and slot_mapping.dtype == torch.int64 and slot_mapping.dim() == 1
+            and slot_mapping.shape[0] == key.shape[0] and slot_mapping.stride(0) == 1):
+        raise ValueError("slot_mapping must be an int64 device tensor [T]")
     dev = key.device
     ks = _scale_tensor(k_scale, dev)
     vs = _scale_tensor(v_scale, dev)
@@ -323,8 +346,8 @@ def cache_write(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
 # ------------------------------------------------------------------------------ layer epilogues
 
 def _bf16_rows(t: torch.Tensor, name: str) -> None:
-    _require(t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 2 and t.stride(1) == 1,
-             f"{name} must be a 2-D bf16 device tensor with contiguous rows")
+    if not (t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 2 and t.stride(1) == 1):
+        raise ValueError(f"{name} must be a 2-D bf16 device tensor with contiguous rows")
 
 
 def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float,
@@ -338,13 +361,16 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Ten
     _bf16_rows(x, "x")
     _bf16_rows(residual, "residual")
     M, H = x.shape
-    _require(tuple(residual.shape) == (M, H), "residual must match x")
-    _require(weight.is_cuda and weight.dtype == torch.bfloat16 and tuple(weight.shape) == (H,)
-             and weight.is_contiguous(), "weight must be a contiguous bf16 [H] device tensor")
+    if not (tuple(residual.shape) == (M, H)):
+        raise ValueError("residual must match x")
+    if not (weight.is_cuda and weight.dtype == torch.bfloat16 and tuple(weight.shape) == (H,) and
+            weight.is_contiguous()):
+        raise ValueError("weight must be a contiguous bf16 [H] device tensor")
     if out is None:
         out = torch.empty_like(x)
     _bf16_rows(out, "out")
-    _require(tuple(out.shape) == (M, H), "out must match x")
+    if not (tuple(out.shape) == (M, H)):
+        raise ValueError("out must match x")
     st = _lib.load().fp8kv_fused_add_rmsnorm(x.data_ptr(), x.stride(0), residual.data_ptr(),
                                              residual.stride(0), weight.data_ptr(), out.data_ptr(),
                                              out.stride(0), M, H, float(eps), int(mode), _stream_ptr(x))
@@ -357,12 +383,14 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None, mode: int =
     compiled vLLM native form; mode 1: SiLU rounded first, as vLLM's _C.silu_and_mul)."""
     _bf16_rows(gate_up, "gate_up")
     M, d2 = gate_up.shape
-    _require(d2 % 2 == 0, "gate_up width must be even")
+    if not (d2 % 2 == 0):
+        raise ValueError("gate_up width must be even")
     d = d2 // 2
     if out is None:
-        out = torch.empty((M, d), dtype=torch.bfloat16, device=gate_up.device)
+        out = gate_up.new_empty((M, d), dtype=torch.bfloat16)
     _bf16_rows(out, "out")
-    _require(tuple(out.shape) == (M, d), f"out must be [{M}, {d}]")
+    if not (tuple(out.shape) == (M, d)):
+        raise ValueError(f"out must be [{M}, {d}]")
     st = _lib.load().fp8kv_silu_mul(gate_up.data_ptr(), gate_up.stride(0), out.data_ptr(), out.stride(0),
                                     M, d, int(mode), _stream_ptr(gate_up))
     _lib.check("fp8kv_silu_mul", st)
@@ -372,13 +400,13 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None, mode: int =
 def interleave_gate_up(weight: torch.Tensor, scales_nk: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Load-time row interleave of a merged gate/up weight (rows [gate; up]) for h4mv_silu_mul:
     each 16-row tile becomes 8 gate rows then the up rows of the same 8 features."""
-    _require(weight.is_cuda and weight.dtype == torch.uint8 and weight.dim() == 2 and weight.is_contiguous(),
-             "weight must be contiguous uint8 [N, K/2] on the device")
+    if not (weight.is_cuda and weight.dtype == torch.uint8 and weight.dim() == 2 and weight.is_contiguous()):
+        raise ValueError("weight must be contiguous uint8 [N, K/2] on the device")
     N, KH = weight.shape
     K = 2 * KH
-    _require(scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32)
-             and scales_nk.is_contiguous() and scales_nk.device == weight.device,
-             f"scales must be contiguous uint8 [{N}, {K // 32}]")
+    if not (scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and
+            scales_nk.is_contiguous() and scales_nk.device == weight.device):
+        raise ValueError(f"scales must be contiguous uint8 [{N}, {K // 32}]")
     w_out = torch.empty_like(weight)
     s_out = torch.empty_like(scales_nk)
     st = _lib.load().h4mv_interleave_gate_up(weight.data_ptr(), scales_nk.data_ptr(), w_out.data_ptr(),
@@ -391,19 +419,22 @@ def h4mv_silu_mul(x: torch.Tensor, weight_il: torch.Tensor, scales_il: torch.Ten
                   out: torch.Tensor | None = None, mode: int = 0) -> torch.Tensor:
     """[M, N/2] = silu_mul(x . dequant(W)^T) for a gate/up weight from interleave_gate_up, in one
     launch (the same bits as h4mv into [M, N] followed by silu_mul(mode))."""
-    _require(x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous(),
-             "x must be a contiguous 2-D bf16 device tensor")
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()):
+        raise ValueError("x must be a contiguous 2-D bf16 device tensor")
     M, K = x.shape
     N = weight_il.shape[0]
-    _require(weight_il.dtype == torch.uint8 and tuple(weight_il.shape) == (N, K // 2)
-             and weight_il.is_contiguous(), f"weight must be contiguous uint8 [N, {K // 2}]")
-    _require(scales_il.dtype == torch.uint8 and tuple(scales_il.shape) == (N, K // 32)
-             and scales_il.is_contiguous(), f"scales must be contiguous uint8 [{N}, {K // 32}]")
-    _require(weight_il.device == x.device == scales_il.device, "tensors on different devices")
+    if not (weight_il.dtype == torch.uint8 and tuple(weight_il.shape) == (N, K // 2) and
+            weight_il.is_contiguous()):
+        raise ValueError(f"weight must be contiguous uint8 [N, {K // 2}]")
+    if not (scales_il.dtype == torch.uint8 and tuple(scales_il.shape) == (N, K // 32) and
+            scales_il.is_contiguous()):
+        raise ValueError(f"scales must be contiguous uint8 [{N}, {K // 32}]")
+    if not (weight_il.device == x.device == scales_il.device):
+        raise ValueError("tensors on different devices")
     if out is None:
-        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
-    _require(out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N // 2) and out.is_contiguous(),
-             f"out must be contiguous bf16 [{M}, {N // 2}]")
+        out = x.new_empty((M, N // 2), dtype=torch.bfloat16)
+    if not (out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N // 2) and out.is_contiguous()):
+        raise ValueError(f"out must be contiguous bf16 [{M}, {N // 2}]")
     st = _lib.load().h4mv_silu_mul(weight_il.data_ptr(), scales_il.data_ptr(), x.data_ptr(), out.data_ptr(),
                                    N, K, M, int(mode), _stream_ptr(x))
     _lib.check("h4mv_silu_mul", st)
@@ -418,12 +449,13 @@ def quant_mxfp8(x: torch.Tensor, out: tuple[torch.Tensor, torch.Tensor] | None =
     _bf16_rows(x, "x")
     M, K = x.shape
     if out is None:
-        out = (torch.empty((M, K), dtype=torch.uint8, device=x.device),
-               torch.empty((M, K // 32), dtype=torch.uint8, device=x.device))
+        out = (x.new_empty((M, K), dtype=torch.uint8),
+               x.new_empty((M, K // 32), dtype=torch.uint8))
     xq, sx = out
-    _require(xq.dtype == torch.uint8 and tuple(xq.shape) == (M, K) and xq.is_contiguous(), "codes must be uint8 [M, K]")
-    _require(sx.dtype == torch.uint8 and tuple(sx.shape) == (M, K // 32) and sx.is_contiguous(),
-             "scales must be uint8 [M, K/32]")
+    if not (xq.dtype == torch.uint8 and tuple(xq.shape) == (M, K) and xq.is_contiguous()):
+        raise ValueError("codes must be uint8 [M, K]")
+    if not (sx.dtype == torch.uint8 and tuple(sx.shape) == (M, K // 32) and sx.is_contiguous()):
+        raise ValueError("scales must be uint8 [M, K/32]")
     st = _lib.load().h4a8_quant_act(x.data_ptr(), x.stride(0), xq.data_ptr(), sx.data_ptr(), M, K, _stream_ptr(x))
     _lib.check("h4a8_quant_act", st)
     return xq, sx
@@ -434,17 +466,21 @@ def h4a8_gemm(xq: torch.Tensor, sx: torch.Tensor, weight: torch.Tensor, scales_n
     """bf16 [M, N] = dequant(xq, sx) . dequant(weight, scales_nk)^T on the block-scaled MFMA."""
     M, K = xq.shape
     N = weight.shape[0]
-    _require(xq.is_cuda and xq.dtype == torch.uint8 and xq.is_contiguous(), "xq must be contiguous uint8 [M, K]")
-    _require(sx.dtype == torch.uint8 and tuple(sx.shape) == (M, K // 32) and sx.is_contiguous(), "sx must be uint8 [M, K/32]")
-    _require(weight.dtype == torch.uint8 and tuple(weight.shape) == (N, K // 2) and weight.is_contiguous(),
-             "weight must be contiguous uint8 [N, K/2]")
-    _require(scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and scales_nk.is_contiguous(),
-             "scales must be contiguous uint8 [N, K/32]")
-    _require(xq.device == sx.device == weight.device == scales_nk.device, "tensors on different devices")
+    if not (xq.is_cuda and xq.dtype == torch.uint8 and xq.is_contiguous()):
+        raise ValueError("xq must be contiguous uint8 [M, K]")
+    if not (sx.dtype == torch.uint8 and tuple(sx.shape) == (M, K // 32) and sx.is_contiguous()):
+        raise ValueError("sx must be uint8 [M, K/32]")
+    if not (weight.dtype == torch.uint8 and tuple(weight.shape) == (N, K // 2) and weight.is_contiguous()):
+        raise ValueError("weight must be contiguous uint8 [N, K/2]")
+    if not (scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and
+            scales_nk.is_contiguous()):
+        raise ValueError("scales must be contiguous uint8 [N, K/32]")
+    if not (xq.device == sx.device == weight.device == scales_nk.device):
+        raise ValueError("tensors on different devices")
     if out is None:
-        out = torch.empty((M, N), dtype=torch.bfloat16, device=xq.device)
-    _require(out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N) and out.is_contiguous(),
-             "out must be contiguous bf16 [M, N]")
+        out = xq.new_empty((M, N), dtype=torch.bfloat16)
+    if not (out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N) and out.is_contiguous()):
+        raise ValueError("out must be contiguous bf16 [M, N]")
     st = _lib.load().h4a8_gemm(weight.data_ptr(), scales_nk.data_ptr(), xq.data_ptr(), sx.data_ptr(),
                                out.data_ptr(), N, K, M, _stream_ptr(xq))
     _lib.check("h4a8_gemm", st)
@@ -458,11 +494,13 @@ def quant_fp8_per_token(x: torch.Tensor, out: tuple[torch.Tensor, torch.Tensor] 
     _bf16_rows(x, "x")
     M, K = x.shape
     if out is None:
-        out = (torch.empty((M, K), dtype=torch.uint8, device=x.device),
-               torch.empty((M,), dtype=torch.float32, device=x.device))
+        out = (x.new_empty((M, K), dtype=torch.uint8),
+               x.new_empty((M,), dtype=torch.float32))
     xq, sc = out
-    _require(xq.dtype == torch.uint8 and tuple(xq.shape) == (M, K) and xq.is_contiguous(), "codes must be uint8 [M, K]")
-    _require(sc.dtype == torch.float32 and tuple(sc.shape) == (M,) and sc.is_contiguous(), "scales must be fp32 [M]")
+    if not (xq.dtype == torch.uint8 and tuple(xq.shape) == (M, K) and xq.is_contiguous()):
+        raise ValueError("codes must be uint8 [M, K]")
+    if not (sc.dtype == torch.float32 and tuple(sc.shape) == (M,) and sc.is_contiguous()):
+        raise ValueError("scales must be fp32 [M]")
     st = _lib.load().h4a8_quant_act_token(x.data_ptr(), x.stride(0), xq.data_ptr(), sc.data_ptr(), M, K,
                                           _stream_ptr(x))
     _lib.check("h4a8_quant_act_token", st)
@@ -474,18 +512,22 @@ def h4a8_gemm_token(xq: torch.Tensor, token_scales: torch.Tensor, weight: torch.
     """bf16 [M, N] = token_scales[:, None] * (e4m3(xq) . dequant(weight, scales_nk)^T)."""
     M, K = xq.shape
     N = weight.shape[0]
-    _require(xq.is_cuda and xq.dtype == torch.uint8 and xq.is_contiguous(), "xq must be contiguous uint8 [M, K]")
-    _require(token_scales.dtype == torch.float32 and tuple(token_scales.shape) == (M,) and token_scales.is_contiguous(),
-             "token scales must be fp32 [M]")
-    _require(weight.dtype == torch.uint8 and tuple(weight.shape) == (N, K // 2) and weight.is_contiguous(),
-             "weight must be contiguous uint8 [N, K/2]")
-    _require(scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and scales_nk.is_contiguous(),
-             "scales must be contiguous uint8 [N, K/32]")
-    _require(xq.device == token_scales.device == weight.device == scales_nk.device, "tensors on different devices")
+    if not (xq.is_cuda and xq.dtype == torch.uint8 and xq.is_contiguous()):
+        raise ValueError("xq must be contiguous uint8 [M, K]")
+    if not (token_scales.dtype == torch.float32 and tuple(token_scales.shape) == (M,) and
+            token_scales.is_contiguous()):
+        raise ValueError("token scales must be fp32 [M]")
+    if not (weight.dtype == torch.uint8 and tuple(weight.shape) == (N, K // 2) and weight.is_contiguous()):
+        raise ValueError("weight must be contiguous uint8 [N, K/2]")
+    if not (scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and
+            scales_nk.is_contiguous()):
+        raise ValueError("scales must be contiguous uint8 [N, K/32]")
+    if not (xq.device == token_scales.device == weight.device == scales_nk.device):
+        raise ValueError("tensors on different devices")
     if out is None:
-        out = torch.empty((M, N), dtype=torch.bfloat16, device=xq.device)
-    _require(out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N) and out.is_contiguous(),
-             "out must be contiguous bf16 [M, N]")
+        out = xq.new_empty((M, N), dtype=torch.bfloat16)
+    if not (out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N) and out.is_contiguous()):
+        raise ValueError("out must be contiguous bf16 [M, N]")
     st = _lib.load().h4a8_gemm_token(weight.data_ptr(), scales_nk.data_ptr(), xq.data_ptr(), token_scales.data_ptr(),
                                      out.data_ptr(), N, K, M, _stream_ptr(xq))
     _lib.check("h4a8_gemm_token", st)
@@ -499,7 +541,8 @@ def mxfp4_linear(x: torch.Tensor, weight: torch.Tensor, scales_nk: torch.Tensor,
     if act == "token":
         xq, sc = quant_fp8_per_token(x)
         return h4a8_gemm_token(xq, sc, weight, scales_nk)
-    _require(act == "mx", f"unknown activation format {act!r}")
+    if not (act == "mx"):
+        raise ValueError(f"unknown activation format {act!r}")
     xq, sx = quant_mxfp8(x)
     return h4a8_gemm(xq, sx, weight, scales_nk)
 
@@ -541,23 +584,25 @@ def lm_head_topk(x: torch.Tensor, weight: torch.Tensor, scales_nk: torch.Tensor,
     defaults to the per-device cached buffer of ``topk_workspace``, which calls on one device
     share (calls overlapping on different streams must pass their own).  During graph capture
     the cache is not grown: capture a call whose workspace is already large enough, or pass one."""
-    _require(x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous(),
-             "x must be a contiguous 2-D bf16 device tensor")
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()):
+        raise ValueError("x must be a contiguous 2-D bf16 device tensor")
     M, K = x.shape
     N = weight.shape[0]
-    _require(weight.dtype == torch.uint8 and tuple(weight.shape) == (N, K // 2) and weight.is_contiguous(),
-             "weight must be contiguous uint8 [N, K/2]")
-    _require(scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32)
-             and scales_nk.is_contiguous(), f"scales must be contiguous uint8 [{N}, {K // 32}]")
+    if not (weight.dtype == torch.uint8 and tuple(weight.shape) == (N, K // 2) and weight.is_contiguous()):
+        raise ValueError("weight must be contiguous uint8 [N, K/2]")
+    if not (scales_nk.dtype == torch.uint8 and tuple(scales_nk.shape) == (N, K // 32) and
+            scales_nk.is_contiguous()):
+        raise ValueError(f"scales must be contiguous uint8 [{N}, {K // 32}]")
     lib = _lib.load()
     need = int(lib.h4mv_topk_workspace_bytes(N, M, int(k)))
-    _require(need > 0, f"k={k} outside [1, 64]")
+    if not (need > 0):
+        raise ValueError(f"k={k} outside [1, 64]")
     if workspace is None:
         workspace = topk_workspace(need, x.device, allow_alloc=not torch.cuda.is_current_stream_capturing())
-        _require(workspace is not None,
-                 f"lm_head_topk during graph capture needs {need} workspace bytes: pass a workspace")
-    vals = torch.empty((M, k), dtype=torch.float32, device=x.device)
-    idx = torch.empty((M, k), dtype=torch.int32, device=x.device)
+        if not (workspace is not None):
+            raise ValueError(f"lm_head_topk during graph capture needs {need} workspace bytes: pass a workspace")
+    vals = x.new_empty((M, k), dtype=torch.float32)
+    idx = x.new_empty((M, k), dtype=torch.int32)
     st = lib.h4mv_topk(weight.data_ptr(), scales_nk.data_ptr(), x.data_ptr(), N, K, M, int(k),
                        vals.data_ptr(), idx.data_ptr(), workspace.data_ptr(),
                        workspace.numel() * workspace.element_size(), _stream_ptr(x))
@@ -573,12 +618,14 @@ def rerank_exact(embedding: torch.Tensor, x: torch.Tensor, candidates: torch.Ten
     _bf16_rows(x, "x")
     V, H = embedding.shape
     M = x.shape[0]
-    _require(x.shape[1] == H, "x and embedding widths differ")
-    _require(candidates.is_cuda and candidates.dtype == torch.int32 and candidates.dim() == 2
-             and candidates.shape[0] == M and candidates.is_contiguous(), "candidates must be int32 [M, C]")
+    if not (x.shape[1] == H):
+        raise ValueError("x and embedding widths differ")
+    if not (candidates.is_cuda and candidates.dtype == torch.int32 and candidates.dim() == 2 and
+            candidates.shape[0] == M and candidates.is_contiguous()):
+        raise ValueError("candidates must be int32 [M, C]")
     C = candidates.shape[1]
-    vals = torch.empty((M, C), dtype=torch.float32, device=x.device)
-    idx = torch.empty((M, C), dtype=torch.int32, device=x.device)
+    vals = x.new_empty((M, C), dtype=torch.float32)
+    idx = x.new_empty((M, C), dtype=torch.int32)
     st = _lib.load().fp8kv_rerank_exact(embedding.data_ptr(), embedding.stride(0), V, x.data_ptr(), x.stride(0),
                                         candidates.data_ptr(), C, M, H, vals.data_ptr(), idx.data_ptr(),
                                         _stream_ptr(x))
