@@ -1074,10 +1074,10 @@ constexpr int kSplitRoundWorkgroups = 256;
 inline int split_xcd_per(int hkv) { return (hkv <= 8 && 8 % hkv == 0) ? 8 / hkv : 1; }
 
 // True when one 16-token block per workgroup fits in one round of the key-split kernel.
-inline bool split_single_blocks_fit(int n16, int hkv, int num_seqs)
+inline bool split_single_blocks_fit(int n16, int hkv, int num_seqs, int rounds = 1)
 {
     const int per = split_xcd_per(hkv);
-    return (int64_t)((n16 + per - 1) / per * per) * hkv * num_seqs <= kSplitRoundWorkgroups;
+    return (int64_t)((n16 + per - 1) / per * per) * hkv * num_seqs <= rounds * kSplitRoundWorkgroups;
 }
 
 // Contexts (in keys) from which the key-split kernel beats the per-wave kernel, measured on MI355X.
@@ -1099,6 +1099,8 @@ constexpr int kSplitMinContextLowGqa = 512;
 // plan's test has them, although contexts of 1000 keys would gain there too.
 constexpr int kSplitMinQueryInexact = 320;
 constexpr int kSplitMinContextSingle = 256;
+// In two rounds: 512 (4 of 512, 24 / 4 heads: 26.6 us against 28.1 per wave, 48 / 4: 37 against 48).
+constexpr int kSplitMinContextTwoRounds = 512;
 
 // One launch as planned from the shape alone (no pointers): kernel, block pairing and grid.
 struct Plan {
@@ -1136,7 +1138,8 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
     } else if (g_shape < 0) {
         const int many = gqa < 4 ? kSplitMinContextLowGqa
                        : kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext;
-        split = ctx_hint >= many || (ctx_hint >= kSplitMinContextSingle && fits);
+        split = ctx_hint >= many || (ctx_hint >= kSplitMinContextSingle && fits) ||
+                (ctx_hint >= kSplitMinContextTwoRounds && split_single_blocks_fit(nsb, hkv, num_seqs, 2));
         if (!exact && max_query_len < kSplitMinQueryInexact) split = false;
     }
     if (split) {

@@ -105,3 +105,24 @@ def test_empty_and_invalid(lib):
     assert lib.fp8kv_prefill_plan(24, 5, 1, 10, 10, ctypes.addressof(out)) == 2
     assert lib.fp8kv_prefill_plan(24, 4, 0, 10, 10, ctypes.addressof(out)) == 1
     assert lib.fp8kv_prefill_plan(24, 4, 1, 10, 10, None) == 1
+
+
+@pytest.mark.parametrize("hq,hkv,num_seqs,max_q,ctx,split,paired,nb", [
+    (24, 4, 4, 512, 512, 1, 1, 2),      # two rounds of single blocks, from 512 keys
+    (24, 4, 4, 511, 511, 0, 0, 2),
+    (24, 4, 5, 512, 512, 0, 0, 2),      # a third round: per-wave kernel, unpaired
+    (24, 4, 6, 900, 900, 0, 0, 2),
+    (16, 2, 12, 768, 768, 1, 1, 2),     # GQA 8 splits the keys two ways: from 768
+    (16, 2, 12, 767, 767, 0, 0, 2),
+    (28, 4, 1, 320, 1000, 1, 0, 2),     # no shape of its own: from 320-token prompts
+    (28, 4, 1, 319, 1000, 0, 0, 2),
+    (16, 16, 1, 1024, 1024, 1, 0, 4),   # GQA 1: four token blocks per workgroup
+    (8, 4, 1, 1024, 1024, 1, 0, 2),     # GQA 2: two
+    (8, 4, 1, 320, 320, 1, 0, 2),
+    (24, 4, 12, 400, 400, 0, 0, 2)])
+def test_plan_lines(lib, hq, hkv, num_seqs, max_q, ctx, split, paired, nb):
+    """Both sides of the lines between the key-split and the per-wave kernel."""
+    p = plan(lib, hq, hkv, num_seqs, max_q, ctx)
+    assert (p["split"], p["paired"], p["nb"]) == (split, paired, nb)
+    blocks = (max_q + 15) // 16
+    assert p["ntb"] * (2 * (nb if split and hq // hkv < 3 else 1) if p["paired"] else nb) >= blocks
