@@ -492,6 +492,9 @@ thread_local int g_target_wgs = 256;
 // 39.6 in three; 64 of 2048: 24.6 and 30.4).
 constexpr int kMaxPlannedSplits = 32;
 constexpr int kLongContext = 6144;
+// From here on a length says only that the contexts are not known (a graph under capture, replayed for
+// whatever contexts come): the count then follows from the batch shape, without the rule for long ones.
+constexpr int kUnknownContext = 1 << 30;
 // Every planned call fits the library's fixed 8 MiB of scratch at any GQA: 976 records of 16 heads.
 constexpr int kMaxPlannedRecords = 976;
 
@@ -504,7 +507,8 @@ inline int plan_splits(int ns, int hkv, int max_seq_len)
           : max_seq_len / 512 < kMaxPlannedSplits ? (max_seq_len + 511) / 512 : kMaxPlannedSplits;
     const int by_fill = (g_target_wgs + pairs - 1) / pairs;
     if (by_fill > 1) return by_fill < n ? by_fill : n;
-    return max_seq_len >= kLongContext && pairs <= kMaxPlannedRecords ? kMaxPlannedRecords / pairs : 1;
+    const bool known_long = max_seq_len >= kLongContext && max_seq_len < kUnknownContext;
+    return known_long && pairs <= kMaxPlannedRecords ? kMaxPlannedRecords / pairs : 1;
 }
 
 // Zero-fill of a decode scratch region (ticket counters and records), a kernel rather than a

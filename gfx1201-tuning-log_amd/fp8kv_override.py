@@ -32,8 +32,8 @@ if _PKG not in sys.path:
     sys.path.insert(0, _PKG)
 
 TAG = "[fp8kv-override]"
-# Context length the split planner is given while a graph is being captured: long enough that the
-# plan depends only on the batch shape (sequences x kv heads).
+# Context length the split planner is given while a graph is being captured: the planner's mark for
+# contexts that are not known, whose plan depends only on the batch shape (sequences x kv heads).
 CAPTURE_PLAN_SEQ_LEN = 1 << 30
 COUNTERS = {"impl_forward": 0, "fallback": 0}
 _STATE = {"installed": False, "orig": None, "diag_done": False, "engaged": False}

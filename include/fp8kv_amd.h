@@ -146,7 +146,9 @@ int fp8kv_decode_attn_noalloc(const void* q, int64_t q_row_stride,
 
 /* Split count the library would choose for a batch whose longest context is max_seq_len
  * (replaces the fixed NSPLIT = 8 of vllm-fp8kv/fp8kv_override.py:43).  Any value in [1, 256]
- * gives the same result up to rounding; this one fills the GPU. */
+ * gives the same result up to rounding; this one fills the GPU.  max_seq_len >= 2^30 means that the
+ * contexts are not known, as while a graph is captured: the count then depends on the batch shape
+ * alone, and a batch with a workgroup per CU from its (sequence, kv head) pairs is not split. */
 int fp8kv_decode_num_splits(int num_seqs, int num_kv_heads, int max_seq_len);
 
 /* Scratch bytes fp8kv_decode_attn needs for this geometry and split count (0 = none; 0 is also

@@ -226,6 +226,22 @@ def test_decode_capture_plans_from_batch_shape(monkeypatch):
     assert ops.decode_num_splits(3, 4, 1) == 1                 # what the dummy context would give
 
 
+@pytest.mark.parametrize("ns", [64, 100, 122])
+def test_decode_capture_of_a_large_batch_is_not_split(monkeypatch, ns):
+    """A batch whose (sequence, kv head) pairs fill the GPU is captured in one split, which needs no
+    scratch: the graph replays short contexts too, and the rule for known long ones is not for it."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    cls, calls = _fake_vllm(monkeypatch)
+    rec = Recorder()
+    from fp8kv_amd import ops
+    monkeypatch.setattr(ops, "decode_attention", rec("decode"))
+    monkeypatch.setattr(ops, "_scratch_cache", {})
+    _fresh(monkeypatch, "fp8kv_override")
+    md, layer, kv, q, out = _batch(ns=ns, ctx=(9000,) * ns)
+    cls.forward(_impl(cls), layer, q, None, None, kv, md, out)
+    assert calls == [] and [kw["num_splits"] for _, _, kw in rec.calls] == [1]
+
+
 def test_decode_scratch_never_frees_a_replaced_buffer(monkeypatch):
     """A larger request replaces the cached scratch but keeps the old buffer alive (graphs captured
     with it replay into it)."""
