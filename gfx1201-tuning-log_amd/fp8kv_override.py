@@ -105,7 +105,10 @@ def make_forward(orig, fp8_per_tensor, ops, is_capturing):
         plan_len = CAPTURE_PLAN_SEQ_LEN if capturing else int(attn_metadata.max_seq_len)
         nsplit = ops.decode_num_splits(NS, HKV, plan_len)
         need = ops.decode_scratch_bytes(NS, HQ, HKV, nsplit, hs)
-        scratch = ops.decode_scratch(need, query.device, allow_alloc=not capturing)
+        # An eager call allocates the scratch also where its own contexts are too short to need it: the
+        # graphs captured after the warm-up need it for their longer ones and cannot allocate it.
+        scratch = ops.decode_scratch(need if capturing else max(need, 1), query.device,
+                                     allow_alloc=not capturing)
         if need > 0 and scratch is None:
             COUNTERS["fallback"] += 1
             _log(f"scratch of {need} bytes not allocated before graph capture; stock path")

@@ -242,6 +242,23 @@ def test_decode_capture_of_a_large_batch_is_not_split(monkeypatch, ns):
     assert calls == [] and [kw["num_splits"] for _, _, kw in rec.calls] == [1]
 
 
+def test_decode_warm_up_of_short_contexts_allocates_the_capture_scratch(monkeypatch):
+    """Eager calls too short to be split still leave the scratch that a capture afterwards needs."""
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    cls, calls = _fake_vllm(monkeypatch)
+    rec = Recorder()
+    from fp8kv_amd import ops
+    monkeypatch.setattr(ops, "decode_attention", rec("decode"))
+    monkeypatch.setattr(ops, "_scratch_cache", {})
+    _fresh(monkeypatch, "fp8kv_override")
+    for capturing[0] in (False, True):
+        md, layer, kv, q, out = _batch(ctx=(40, 200, 7))
+        cls.forward(_impl(cls), layer, q, None, None, kv, md, out)
+    assert calls == [] and [kw["num_splits"] > 1 for _, _, kw in rec.calls] == [False, True]
+    assert rec.calls[1][2]["scratch"].numel() >= ops.DECODE_SCRATCH_MIN_BYTES
+
+
 def test_decode_scratch_never_frees_a_replaced_buffer(monkeypatch):
     """A larger request replaces the cached scratch but keeps the old buffer alive (graphs captured
     with it replay into it)."""
