@@ -136,6 +136,26 @@ def decode_scratch_reset(scratch: torch.Tensor) -> None:
     _lib.check("fp8kv_decode_scratch_reset", st)
 
 
+# The tickets at the start of a decode scratch, which a call expects zero.
+_DECODE_TICKET_BYTES = 256 << 10
+
+
+def _call_scratch(nbytes: int, device) -> torch.Tensor | None:
+    """Scratch of one decode call that was given none: the device's cached buffer.  Under graph capture
+    a buffer that would have to be allocated first belongs to that capture and is not cached: its
+    memory is the graph's, and its zeroes are written only when the graph is replayed."""
+    if nbytes <= 0:
+        return None
+    buf = decode_scratch(nbytes, device, allow_alloc=False)
+    if buf is not None:
+        return buf
+    if not torch.cuda.is_current_stream_capturing():
+        return decode_scratch(nbytes, device)
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    decode_scratch_reset(buf[:_DECODE_TICKET_BYTES])
+    return buf
+
+
 def _ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
@@ -210,7 +230,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         num_splits = decode_num_splits(NS, HKV, int(max_seq_len))
     need = decode_scratch_bytes(NS, HQ, HKV, num_splits, D)
     if scratch is None:
-        scratch = decode_scratch(need, dev)
+        scratch = _call_scratch(need, dev)
     elif need > 0:
         if not (scratch.is_cuda and scratch.numel() * scratch.element_size() >= need):
             raise ValueError(f"scratch needs {need} bytes")

@@ -185,6 +185,37 @@ def test_graph_capture_replay():
         assert torch.equal(got, eager), f"replay {it}"
 
 
+def test_graph_capture_without_warm_up(monkeypatch):
+    """A capture that finds no scratch takes one of its own: eager calls before and between the replays
+    get a zeroed buffer, and every replay equals them."""
+    c = workloads.decode_case([600, 1500], seed=15)
+    d = workloads.to_device(c, DEV)
+    ks = torch.tensor([c["k_scale"]], device=DEV)
+    vs = torch.tensor([c["v_scale"]], device=DEV)
+    out, eager = torch.zeros_like(d["q"]), torch.zeros_like(d["q"])
+    args = (d["q"], d["k_cache"], d["v_cache"])
+    rest = (d["qsl"], d["seq_lens"], d["block_table"], ks, vs, c["sm_scale"])
+    ops.decode_attention(*args, eager, *rest, num_splits=8)                # loads the kernels
+    monkeypatch.setattr(ops, "_scratch_cache", {})
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(graph, stream=s):
+            ops.decode_attention(*args, out, *rest, num_splits=8)
+            ops.decode_attention(*args, out, *rest, num_splits=8)
+    torch.cuda.current_stream().wait_stream(s)
+    assert ops._scratch_cache == {}
+    for it in range(3):
+        ops.decode_attention(*args, eager, *rest, num_splits=8)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), f"replay {it}"
+        d["q"].neg_()
+    torch.testing.assert_close(_rows(c, eager), _oracle(c), rtol=RTOL, atol=ATOL)
+
+
 def test_rejects_unsupported_geometry():
     c = workloads.decode_case([64], D=64, seed=14)
     d = workloads.to_device(c, DEV)

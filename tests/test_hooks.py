@@ -274,6 +274,24 @@ def test_decode_scratch_never_frees_a_replaced_buffer(monkeypatch):
     assert ops.decode_scratch(10, "cpu", allow_alloc=False) is b
 
 
+def test_decode_scratch_of_a_capture_is_not_cached(monkeypatch):
+    """A scratch allocated while a graph is captured holds no zeroes until a replay, so later calls must
+    not find it in the cache; outside capture the buffer is cached as before."""
+    from fp8kv_amd import ops
+    resets, capturing = [], [True]
+    monkeypatch.setattr(ops, "_scratch_cache", {})
+    monkeypatch.setattr(ops, "decode_scratch_reset", resets.append)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    a = ops._call_scratch(300 << 10, "cpu")
+    assert a.numel() == 300 << 10 and ops._scratch_cache == {}
+    assert [r.numel() for r in resets] == [256 << 10] and resets[0].data_ptr() == a.data_ptr()
+    capturing[0] = False
+    b = ops._call_scratch(300 << 10, "cpu")
+    assert b.numel() == ops.DECODE_SCRATCH_MIN_BYTES and list(ops._scratch_cache.values()) == [b]
+    capturing[0] = True
+    assert ops._call_scratch(300 << 10, "cpu") is b and len(resets) == 1
+
+
 def test_decode_errors_propagate(monkeypatch, no_capture):
     """fp8kv_override.py:102-106 does not catch kernel errors; neither does this hook."""
     cls, calls = _fake_vllm(monkeypatch)
