@@ -470,14 +470,9 @@ constexpr Variant kVariants[] = {{8, 4, 1, false}, {8, 2, 1, false}, {4, 4, 1, f
                                  {8, 2, 2, true},  {8, 2, 2, false}, {8, 2, 1, true}};
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
-// Launch tunables (host state; fp8kv_decode_tune changes them for sweeps).  The default is one
-// chunk of two 16-token groups in flight per wave: at 118 VGPRs two 8-wave workgroups share a CU,
-// and the second one's stream covers the first one's start and merge.  Against two chunks in
-// flight (variant 5, 149 VGPRs, one workgroup per CU; us in a graph, fp8): one sequence of 777 tokens
-// 5.96 / 6.15, of 16000 13.3 / 14.2, 8 of 1024..4096 10.15 / 10.25, 8 of 4096 equal (10.6), 16 of
-// 300..3000 11.1 / 12.8, 64 of 512..4096 36.8 / 37.9.
-constexpr int kDefaultVariant = 1;
-thread_local int g_variant = kDefaultVariant;
+// Launch tunables (host state; fp8kv_decode_tune changes them for sweeps); -1 chooses the variant.
+thread_local int g_variant = -1;
+constexpr int kCus = 256;
 thread_local int g_target_wgs = 256;
 
 // Splits per (sequence, kv head).  Up to g_target_wgs workgroups, as many as fill the GPU (one per
@@ -509,6 +504,27 @@ inline int plan_splits(int ns, int hkv, int max_seq_len)
     if (by_fill > 1) return by_fill < n ? by_fill : n;
     const bool known_long = max_seq_len >= kLongContext && max_seq_len < kUnknownContext;
     return known_long && pairs <= kMaxPlannedRecords ? kMaxPlannedRecords / pairs : 1;
+}
+
+// Variant 1 holds one chunk of two 16-token groups in flight per wave: at 118 VGPRs two 8-wave workgroups
+// share a CU, and the second one's stream covers the first one's start and merge.  Variant 5 holds two
+// (149 VGPRs, one workgroup per CU).  Up to one workgroup per CU variant 1 is the faster (us in a graph,
+// fp8, 1 / 5: one sequence of 777 tokens 5.96 / 6.15, of 16000 13.3 / 14.2, 8 of 1024..4096 10.15 / 10.25,
+// 16 of 300..3000 11.1 / 12.8).  Past that it depends on the tokens of a split, which the caller's longest
+// context gives: short ones gain from the shared CU (160 of 200 tokens, 4 kv heads: 0.7 of the time), but
+// long ones of unequal length lose more than equal ones gain, because all workgroups start at once and the
+// CUs that drew two of the longest finish last, where variant 5 hands a CU its next workgroup as it falls
+// free (12 sequences of 2048..16384, 8 kv heads, in three: 74.5 / 52.4; of 16384 each 98.3 / 99.1).  The lines
+// are where ragged batches (1 to 8) break even: 1024 tokens a split up to two workgroups per CU (0.6-1.06
+// below, to 1.43 above), 2048 past that (0.6-1.02, to 1.12).  Contexts that are not known take 5.
+constexpr int kShareMaxSpan = 1024, kShareMaxSpanManyWgs = 2048;
+
+inline int pick_variant(int64_t wgs, int nsplit, int max_seq_len)
+{
+    if (g_variant >= 0) return g_variant;
+    if (wgs <= kCus) return 1;
+    if (max_seq_len <= 0 || max_seq_len >= kUnknownContext) return 5;
+    return max_seq_len <= (int64_t)nsplit * (wgs <= 2 * kCus ? kShareMaxSpan : kShareMaxSpanManyWgs) ? 1 : 5;
 }
 
 // Zero-fill of a decode scratch region (ticket counters and records), a kernel rather than a
@@ -611,11 +627,12 @@ int decode_launch_bf16kv(const Params& P, int num_seqs, hipStream_t st)
     return finish_launch();
 }
 
-int decode_launch(const Params& P, int num_seqs, hipStream_t st)
+// max_seq_len: the longest context, or 0 where the caller did not say.
+int decode_launch(const Params& P, int num_seqs, int max_seq_len, hipStream_t st)
 {
     const dim3 grid((unsigned)P.nsplit, (unsigned)P.hkv, (unsigned)num_seqs);
     begin_launch();
-    switch (g_variant) {
+    switch (pick_variant((int64_t)P.nsplit * P.hkv * num_seqs, P.nsplit, max_seq_len)) {
         case 0: launch_kernel(decode_kernel<8, 4, 1, false>, grid, dim3(8 * 64), 0, st, P.seq_lens, P.qsl, P); break;
         case 1: launch_kernel(decode_kernel<8, 2, 1, false>, grid, dim3(8 * 64), 0, st, P.seq_lens, P.qsl, P); break;
         case 2: launch_kernel(decode_kernel<4, 4, 1, false>, grid, dim3(4 * 64), 0, st, P.seq_lens, P.qsl, P); break;
@@ -696,6 +713,31 @@ extern "C" int fp8kv_decode_scratch_reset(void* scratch_buf, size_t scratch_byte
     return launch_scratch_zero(scratch_buf, scratch_bytes_given, reinterpret_cast<hipStream_t>(stream));
 }
 
+extern "C" int fp8kv_decode_attn_ctx(const void* q, int64_t q_row_stride,
+                                     const void* k_cache, const void* v_cache,
+                                     int64_t sk0, int64_t sk1, int64_t sk2,
+                                     int64_t sv0, int64_t sv1, int64_t sv2,
+                                     void* out, int64_t out_row_stride,
+                                     const int32_t* query_start_loc, const int32_t* seq_lens,
+                                     const int32_t* block_table, int64_t bt_stride,
+                                     const float* k_scale, const float* v_scale, float sm_scale,
+                                     int num_seqs, int num_q_heads, int num_kv_heads, int head_size,
+                                     int block_size, int num_splits, void* scratch_buf,
+                                     size_t scratch_bytes_given, int max_seq_len, void* stream)
+{
+    Params P;
+    size_t need = 0;
+    const int rc = decode_setup(P, q, q_row_stride, k_cache, v_cache, sk0, sk1, sk2, sv0, sv1, sv2, out,
+                                out_row_stride, query_start_loc, seq_lens, block_table, bt_stride, k_scale,
+                                v_scale, sm_scale, num_seqs, num_q_heads, num_kv_heads, head_size, block_size,
+                                num_splits, need);
+    if (rc != FP8KV_OK) return rc;
+    if (need > 0 && (!scratch_buf || scratch_bytes_given < need || !aligned(scratch_buf, 256)))
+        return FP8KV_ERR_SCRATCH;
+    use_scratch(P, scratch_buf, need);
+    return decode_launch(P, num_seqs, max_seq_len, reinterpret_cast<hipStream_t>(stream));
+}
+
 extern "C" int fp8kv_decode_attn(const void* q, int64_t q_row_stride,
                                  const void* k_cache, const void* v_cache,
                                  int64_t sk0, int64_t sk1, int64_t sk2,
@@ -708,17 +750,10 @@ extern "C" int fp8kv_decode_attn(const void* q, int64_t q_row_stride,
                                  int block_size, int num_splits, void* scratch_buf,
                                  size_t scratch_bytes_given, void* stream)
 {
-    Params P;
-    size_t need = 0;
-    const int rc = decode_setup(P, q, q_row_stride, k_cache, v_cache, sk0, sk1, sk2, sv0, sv1, sv2, out,
-                                out_row_stride, query_start_loc, seq_lens, block_table, bt_stride, k_scale,
-                                v_scale, sm_scale, num_seqs, num_q_heads, num_kv_heads, head_size, block_size,
-                                num_splits, need);
-    if (rc != FP8KV_OK) return rc;
-    if (need > 0 && (!scratch_buf || scratch_bytes_given < need || !aligned(scratch_buf, 256)))
-        return FP8KV_ERR_SCRATCH;
-    use_scratch(P, scratch_buf, need);
-    return decode_launch(P, num_seqs, reinterpret_cast<hipStream_t>(stream));
+    return fp8kv_decode_attn_ctx(q, q_row_stride, k_cache, v_cache, sk0, sk1, sk2, sv0, sv1, sv2, out, out_row_stride,
+                                 query_start_loc, seq_lens, block_table, bt_stride, k_scale, v_scale, sm_scale, num_seqs,
+                                 num_q_heads, num_kv_heads, head_size, block_size, num_splits, scratch_buf,
+                                 scratch_bytes_given, 0, stream);
 }
 
 extern "C" int fp8kv_decode_attn_noalloc(const void* q, int64_t q_row_stride,
@@ -747,7 +782,7 @@ extern "C" int fp8kv_decode_attn_noalloc(const void* q, int64_t q_row_stride,
         if (rc != FP8KV_OK) return rc;
     }
     use_scratch(P, ptr, need);
-    return decode_launch(P, num_seqs, st);
+    return decode_launch(P, num_seqs, 0, st);
 }
 
 extern "C" int fp8kv_decode_attn_bf16(const void* q, int64_t q_row_stride,
@@ -777,6 +812,11 @@ extern "C" int fp8kv_decode_attn_bf16(const void* q, int64_t q_row_stride,
 
 extern "C" void fp8kv_decode_tune(int variant, int target_wgs)
 {
-    g_variant = (variant >= 0 && variant < kNumVariants) ? variant : kDefaultVariant;
+    g_variant = (variant >= 0 && variant < kNumVariants) ? variant : -1;
     g_target_wgs = target_wgs > 0 ? target_wgs : 256;
+}
+
+extern "C" int fp8kv_decode_variant(int num_seqs, int num_kv_heads, int num_splits, int max_seq_len)
+{
+    return pick_variant((int64_t)num_seqs * num_kv_heads * num_splits, num_splits, max_seq_len);
 }

@@ -64,10 +64,15 @@ void fp8kv_h4mv_mx_chunk_tune(int steps_log2);
 int fp8kv_h4mv_plan(int N, int K, int M, int* out);
 
 /* Tuning hook for sweeps of the decode attention launch: kernel variant index (0..6; any other
- * value, e.g. -1, selects the default, variant 1: 8 waves, one chunk of 2 groups of 16 keys in
- * flight per wave, each group's K and V bytes requested together) and the workgroup count its split planner
- * aims for (0 = default 256).  Affects later launches. */
+ * value, e.g. -1, selects the default, variant 1 or 5 by the grid and the longest context: 8 waves, one
+ * or two chunks of 2 groups of 16 keys in flight per wave, each group's K and V bytes requested
+ * together) and the workgroup count its split planner aims for (0 = default 256).  Affects later
+ * launches. */
 void fp8kv_decode_tune(int variant, int target_wgs);
+
+/* Variant the e4m3 decode entry points launch for this grid under the current tuning hook (host only):
+ * max_seq_len as for fp8kv_decode_attn_ctx. */
+int fp8kv_decode_variant(int num_seqs, int num_kv_heads, int num_splits, int max_seq_len);
 
 /* Tuning hook for sweeps of the prefill attention launch: index of the (waves, row-sets per wave,
  * LDS ring depth) shape to use for every GQA (0..7), 8 + s for key-split shape s (0..4, used only

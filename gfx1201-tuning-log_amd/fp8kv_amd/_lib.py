@@ -37,6 +37,9 @@ SIGNATURES: dict[str, tuple] = {
     "fp8kv_decode_attn": (_c_i, [_c_vp, _c_i64, _c_vp, _c_vp] + [_c_i64] * 6 + [_c_vp, _c_i64]
                           + [_c_vp] * 3 + [_c_i64] + [_c_vp] * 2 + [_c_f] + [_c_i] * 6
                           + [_c_vp, _c_sz, _c_vp]),
+    "fp8kv_decode_attn_ctx": (_c_i, [_c_vp, _c_i64, _c_vp, _c_vp] + [_c_i64] * 6 + [_c_vp, _c_i64]
+                              + [_c_vp] * 3 + [_c_i64] + [_c_vp] * 2 + [_c_f] + [_c_i] * 6
+                              + [_c_vp, _c_sz, _c_i, _c_vp]),
     # paged fp8 causal prefill attention (csrc/prefill_attn.hip)
     "fp8kv_prefill_attn": (_c_i, [_c_vp, _c_i64, _c_vp, _c_vp] + [_c_i64] * 6 + [_c_vp, _c_i64]
                            + [_c_vp, _c_i64] + [_c_vp] * 2 + [_c_f] + [_c_i] * 6 + [_c_vp]),
@@ -80,6 +83,7 @@ SIGNATURES: dict[str, tuple] = {
     "fp8kv_h4mv_mx_chunk_tune": (None, [_c_i]),
     "fp8kv_h4mv_plan": (_c_i, [_c_i, _c_i, _c_i, _c_vp]),
     "fp8kv_decode_tune": (None, [_c_i] * 2),
+    "fp8kv_decode_variant": (_c_i, [_c_i] * 4),
     "fp8kv_prefill_tune": (None, [_c_i]),
     "fp8kv_prefill_bf16_tune": (None, [_c_i]),
     "fp8kv_prefill_plan": (_c_i, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_vp]),

@@ -202,7 +202,9 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     views with arbitrary block/slot/head strides, int32 metadata, device fp32 scales).  bf16
     caches take the reference's K_FP8 = False branch (fp8kv_v3.py:135): the scales are ignored.
     ``num_splits`` defaults to the library's plan for ``max_seq_len`` (read from ``seq_lens`` when
-    not given, which synchronises).  ``scratch`` defaults to a per-device cached buffer.
+    not given, which synchronises).  With ``num_splits`` given, ``max_seq_len`` still helps the
+    library choose its launch where the batch has more workgroups than the GPU has CUs.  ``scratch``
+    defaults to a per-device cached buffer.
     """
     if not (q.is_cuda and q.dtype == torch.bfloat16 and q.dim() == 3 and q.stride(2) == 1 and
             q.stride(1) == q.shape[2]):
@@ -236,7 +238,8 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
             raise ValueError(f"scratch needs {need} bytes")
     sbytes = 0 if scratch is None else scratch.numel() * scratch.element_size()
     lib = _lib.load()
-    name = "fp8kv_decode_attn_bf16" if bf16_kv else "fp8kv_decode_attn"
+    name = "fp8kv_decode_attn_bf16" if bf16_kv else "fp8kv_decode_attn_ctx"
+    known = () if bf16_kv else (int(max_seq_len or 0),)
     st = getattr(lib, name)(
         q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
         k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
@@ -244,7 +247,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         out.data_ptr(), out.stride(0), query_start_loc.data_ptr(), seq_lens.data_ptr(),
         block_table.data_ptr(), block_table.stride(0), _ptr(ks), _ptr(vs),
         float(sm_scale), NS, HQ, HKV, D, PBLK, int(num_splits),
-        None if scratch is None else scratch.data_ptr(), sbytes, _stream_ptr(q))
+        None if scratch is None else scratch.data_ptr(), sbytes, *known, _stream_ptr(q))
     _lib.check(name, st)
     return out
 

@@ -121,7 +121,8 @@ def make_forward(orig, fp8_per_tensor, ops, is_capturing):
         ops.decode_attention(query[:n], key_cache, value_cache, output[:n],
                              attn_metadata.query_start_loc, attn_metadata.seq_lens,
                              attn_metadata.block_table, layer._k_scale, layer._v_scale, self.scale,
-                             num_splits=nsplit, scratch=scratch)
+                             num_splits=nsplit, max_seq_len=None if capturing else plan_len,
+                             scratch=scratch)
         return output
 
     _forward.__fp8kv_wraps__ = orig

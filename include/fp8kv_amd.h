@@ -121,6 +121,23 @@ int fp8kv_decode_attn(const void* q, int64_t q_row_stride,
                       int block_size, int num_splits, void* scratch, size_t scratch_bytes,
                       void* stream);
 
+/* fp8kv_decode_attn for a caller that knows the batch's longest context: the same arguments and
+ * results (bit for bit), and max_seq_len lets the library choose how workgroups share the CUs where
+ * the grid exceeds them (num_seqs * num_kv_heads * num_splits > 256; up to 0.6 of the time for short
+ * contexts).  max_seq_len <= 0 or >= 2^30: not known, the choice of fp8kv_decode_attn.  It need not be
+ * exact and is no bound on seq_lens.  No counterpart in the reference. */
+int fp8kv_decode_attn_ctx(const void* q, int64_t q_row_stride,
+                          const void* k_cache, const void* v_cache,
+                          int64_t sk0, int64_t sk1, int64_t sk2,
+                          int64_t sv0, int64_t sv1, int64_t sv2,
+                          void* out, int64_t out_row_stride,
+                          const int32_t* query_start_loc, const int32_t* seq_lens,
+                          const int32_t* block_table, int64_t bt_stride,
+                          const float* k_scale, const float* v_scale, float sm_scale,
+                          int num_seqs, int num_q_heads, int num_kv_heads, int head_size,
+                          int block_size, int num_splits, void* scratch, size_t scratch_bytes,
+                          int max_seq_len, void* stream);
+
 /* fp8kv_decode_attn without a scratch argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid allocation).  No
  * counterpart in the reference.  The tickets and split records live in a file-scope device array

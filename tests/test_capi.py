@@ -132,6 +132,23 @@ def test_decode_split_plan(lib, ns, hkv, ctx, want):
             assert 1 <= splits <= 32 and lib.fp8kv_decode_scratch_bytes(n, 16 * kv, kv, 128, splits) <= 8 << 20
 
 
+@pytest.mark.parametrize("ns,hkv,splits,ctx,want", [
+    (64, 4, 1, 0, 1), (64, 4, 1, 100000, 1), (8, 8, 4, 100000, 1),           # a workgroup per CU
+    (65, 4, 1, 1024, 1), (65, 4, 1, 1025, 5), (65, 4, 1, 0, 5), (65, 4, 1, 1 << 30, 5),
+    (12, 8, 3, 3072, 1), (12, 8, 3, 3073, 5), (128, 4, 1, 1025, 5),
+    (129, 4, 1, 2048, 1), (129, 4, 1, 2049, 5), (96, 4, 2, 4096, 1), (96, 4, 2, 4097, 5)])
+def test_decode_variant_lines(lib, ns, hkv, splits, ctx, want):
+    """Grids past one workgroup per CU share the CUs only where the caller's longest context says that a
+    split is short."""
+    assert lib.fp8kv_decode_variant(ns, hkv, splits, ctx) == want
+
+
+def test_decode_ctx_rejects_as_the_plain_call(lib):
+    for kw, code in ((dict(q=0), 1), (dict(hd=64), 2), (dict(k=A + 8), 3), (dict(nsplit=8), 5)):
+        a = _decode_args(**kw)
+        assert lib.fp8kv_decode_attn_ctx(*a[:-1], 4096, a[-1]) == code
+
+
 # fp8kv_cache_write: every call below is rejected before any HIP call (fake pointers).
 CW_OK = [A, 512, A, 512, A, A, 8192, 512, 128, 8192, 512, 128, A, A, A, 4, 4, 128, 16, None]
 

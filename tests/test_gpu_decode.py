@@ -216,6 +216,20 @@ def test_graph_capture_without_warm_up(monkeypatch):
     torch.testing.assert_close(_rows(c, eager), _oracle(c), rtol=RTOL, atol=ATOL)
 
 
+def test_known_and_unknown_contexts_give_the_same_bits():
+    """280 workgroups: the launch chosen with the longest context and the one without it."""
+    c = workloads.decode_case([1 + 7 * i for i in range(70)], seed=16)
+    d = workloads.to_device(c, DEV)
+    ks, vs = (torch.tensor([c[k]], device=DEV) for k in ("k_scale", "v_scale"))
+    outs = [torch.zeros_like(d["q"]) for _ in range(2)]
+    for out, longest in zip(outs, (484, None)):
+        ops.decode_attention(d["q"], d["k_cache"], d["v_cache"], out, d["qsl"], d["seq_lens"], d["block_table"], ks, vs,
+                             c["sm_scale"], num_splits=1, max_seq_len=longest)
+    torch.cuda.synchronize()
+    assert torch.equal(*outs)
+    torch.testing.assert_close(_rows(c, outs[0]), _oracle(c), rtol=RTOL, atol=ATOL)
+
+
 def test_rejects_unsupported_geometry():
     c = workloads.decode_case([64], D=64, seed=14)
     d = workloads.to_device(c, DEV)
