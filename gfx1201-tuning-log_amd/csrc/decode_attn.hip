@@ -475,11 +475,17 @@ thread_local int g_variant = -1;
 constexpr int kCus = 256;
 thread_local int g_target_wgs = 256;
 
-// Splits per (sequence, kv head).  Up to g_target_wgs workgroups, as many as fill the GPU (one per
-// CU: at b8@4k 8 splits take 10.6 us, 12 and 16 13.7 and 12.6), but no shorter than pays for the
-// merge: one split up to 256 tokens (200 tokens: 4.7 us in one, 5.4 in two), about 128 tokens each
-// up to 16 splits (777 tokens: 6.0 us in 8, 6.4 in 16), and above 16, where the merge holds 32
-// records, 512 tokens each (4000 tokens: 7.9 us in 16, 9.0 in 32; 16000: 13.3 and 12.1).
+// Splits per (sequence, kv head), never shorter than pays for the merge: one split up to 256 tokens (200
+// tokens: 4.7 us in one, 5.4 in two), about 128 tokens each up to 16 splits (777 tokens: 6.0 us in 8, 6.4 in
+// 16), and above 16, where the merge holds 32 records, 512 tokens each (4000 tokens: 7.9 us in 16, 9.0 in
+// 32; 16000: 13.3 and 12.1).
+// No more of them than fill the GPU with one workgroup per CU (b8@4k: 10.6 us in 8, 13.7 and 12.6 in 12 and
+// 16).  Where the pairs do not divide the CUs, a count rounded up runs a second, nearly empty round and one
+// rounded down leaves CUs idle, so that the longest sequence of an unequal batch takes longer.  Rounded
+// down is far better on equal contexts (12 sequences of 4096, 4 kv heads: 13.0 us in five, 16.6 in six; 96 pairs
+// of 4096: 0.76 of the time in two) and on unequal ones (1 to 8) as long as a split is short; the lines are
+// where the latter break even: none from six splits on (0.6-1.05), 2048 tokens a split for four and
+// five, 1024 below (60 x 4 pairs of 130..1024: 0.83; 33 x 4 of 187..1500: 13.9 us in one, 9.8 in two).
 // With a workgroup per CU or more from the pairs alone, the host knows only the longest context.
 // Long ones are split as often as kMaxPlannedRecords allows, because a ragged batch otherwise ends
 // with a few CUs walking its longest sequences (32 sequences of 512..8192, 8 kv heads, in three: 69.6
@@ -493,17 +499,29 @@ constexpr int kUnknownContext = 1 << 30;
 // Every planned call fits the library's fixed 8 MiB of scratch at any GQA: 976 records of 16 heads.
 constexpr int kMaxPlannedRecords = 976;
 
+// Splits that the workgroups of `pairs` pairs fill the GPU with (see above), pairs <= g_target_wgs.
+inline int fill_splits(int64_t pairs, int max_seq_len)
+{
+    const int64_t down = g_target_wgs / pairs;
+    const int64_t max_span = down >= 4 ? 2048 : 1024;
+    const bool up = g_target_wgs % pairs != 0 && down < 6 && max_seq_len > down * max_span;
+    return (int)(up ? down + 1 : down);
+}
+
 inline int plan_splits(int ns, int hkv, int max_seq_len)
 {
     if (max_seq_len <= 256) return 1;
-    const int pairs = ns * hkv;
-    int n = max_seq_len <= 16 * 128 ? (max_seq_len + 127) / 128
-          : max_seq_len <= 16 * 512 ? 16
-          : max_seq_len / 512 < kMaxPlannedSplits ? (max_seq_len + 511) / 512 : kMaxPlannedSplits;
-    const int by_fill = (g_target_wgs + pairs - 1) / pairs;
-    if (by_fill > 1) return by_fill < n ? by_fill : n;
-    const bool known_long = max_seq_len >= kLongContext && max_seq_len < kUnknownContext;
-    return known_long && pairs <= kMaxPlannedRecords ? kMaxPlannedRecords / pairs : 1;
+    const int64_t pairs = (int64_t)ns * hkv;
+    int n = 1;
+    if (pairs <= g_target_wgs) {
+        n = max_seq_len <= 16 * 128 ? (max_seq_len + 127) / 128
+          : max_seq_len <= 16 * 512 ? 16 : max_seq_len / 512 + (max_seq_len % 512 ? 1 : 0);
+        const int fill = fill_splits(pairs, max_seq_len);
+        if (n > fill) n = fill;
+    }
+    if (pairs >= kCus && max_seq_len >= kLongContext && max_seq_len < kUnknownContext) n = kMaxPlannedSplits;
+    const int64_t most = kMaxPlannedRecords / pairs < kMaxPlannedSplits ? kMaxPlannedRecords / pairs : kMaxPlannedSplits;
+    return n <= most ? n : most > 1 ? (int)most : 1;
 }
 
 // Variant 1 holds one chunk of two 16-token groups in flight per wave: at 118 VGPRs two 8-wave workgroups

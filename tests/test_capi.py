@@ -132,6 +132,30 @@ def test_decode_split_plan(lib, ns, hkv, ctx, want):
             assert 1 <= splits <= 32 and lib.fp8kv_decode_scratch_bytes(n, 16 * kv, kv, 128, splits) <= 8 << 20
 
 
+@pytest.mark.parametrize("ns,hkv,ctx,want", [
+    (6, 4, 1 << 30, 10), (10, 4, 1 << 30, 6),                        # from six on rounded down at any length
+    (12, 4, 5 * 2048, 5), (12, 4, 5 * 2048 + 1, 6), (14, 4, 4 * 2048, 4), (14, 4, 4 * 2048 + 1, 5),
+    (20, 4, 3 * 1024, 3), (20, 4, 3 * 1024 + 1, 4), (33, 4, 1024, 1), (33, 4, 1025, 2), (33, 4, 1 << 30, 2),
+    (16, 4, 100000, 4), (32, 4, 100000, 2)])                         # pairs that divide the CUs
+def test_decode_split_plan_rounds_by_span(lib, ns, hkv, ctx, want):
+    assert lib.fp8kv_decode_num_splits(ns, hkv, ctx) == want
+
+
+@pytest.mark.parametrize("target", [1, 32, 256, 4096, 1 << 30])
+def test_decode_split_plan_bounds_hold_at_any_target(lib, target):
+    """A tuned workgroup target moves the plan, not its bounds: 32 splits, the records of the call that
+    takes no scratch, and one split where the target is met by the pairs alone."""
+    try:
+        lib.fp8kv_decode_tune(-1, target)
+        for ns in (1, 3, 8, 33, 64, 128, 512, 65535):
+            for ctx in (300, 4096, 8193, 100000, 1 << 30, (1 << 31) - 1):
+                n = lib.fp8kv_decode_num_splits(ns, 4, ctx)
+                assert 1 <= n <= 32 and lib.fp8kv_decode_scratch_bytes(ns, 64, 4, 128, n) <= 8 << 20
+                assert n == 1 or ns * 4 <= target or ns * 4 >= 256, (ns, ctx, n)
+    finally:
+        lib.fp8kv_decode_tune(-1, 0)
+
+
 @pytest.mark.parametrize("ns,hkv,splits,ctx,want", [
     (64, 4, 1, 0, 1), (64, 4, 1, 100000, 1), (8, 8, 4, 100000, 1),           # a workgroup per CU
     (65, 4, 1, 1024, 1), (65, 4, 1, 1025, 5), (65, 4, 1, 0, 5), (65, 4, 1, 1 << 30, 5),
