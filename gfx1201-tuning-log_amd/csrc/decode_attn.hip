@@ -477,8 +477,9 @@ thread_local int g_target_wgs = 256;
 
 // Splits per (sequence, kv head), never shorter than pays for the merge: one split up to 256 tokens (200
 // tokens: 4.7 us in one, 5.4 in two), about 128 tokens each up to 16 splits (777 tokens: 6.0 us in 8, 6.4 in
-// 16), and above 16, where the merge holds 32 records, 512 tokens each (4000 tokens: 7.9 us in 16, 9.0 in
-// 32; 16000: 13.3 and 12.1).
+// 16).  Above 16 the merge holds 32 records whatever the count, so it is 16 up to 8192 tokens and 32 from
+// there (4 pairs, 16 / 24 / 32 splits: 6144 tokens 8.2 / 9.2 / 8.8 us, 9000 9.7 / 10.1 / 9.5, 12000 11.0 / 11.1 /
+// 10.2, 16384 13.0 / 12.7 / 11.1).
 // No more of them than fill the GPU with one workgroup per CU (b8@4k: 10.6 us in 8, 13.7 and 12.6 in 12 and
 // 16).  Where the pairs do not divide the CUs, a count rounded up runs a second, nearly empty round and one
 // rounded down leaves CUs idle, so that the longest sequence of an unequal batch takes longer.  Rounded
@@ -515,7 +516,7 @@ inline int plan_splits(int ns, int hkv, int max_seq_len)
     int n = 1;
     if (pairs <= g_target_wgs) {
         n = max_seq_len <= 16 * 128 ? (max_seq_len + 127) / 128
-          : max_seq_len <= 16 * 512 ? 16 : max_seq_len / 512 + (max_seq_len % 512 ? 1 : 0);
+          : max_seq_len <= 16 * 512 ? 16 : kMaxPlannedSplits;
         const int fill = fill_splits(pairs, max_seq_len);
         if (n > fill) n = fill;
     }

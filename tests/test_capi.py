@@ -120,7 +120,7 @@ def test_decode_split_planner(lib):
 
 
 @pytest.mark.parametrize("ns,hkv,ctx,want", [
-    (1, 4, 256, 1), (1, 4, 257, 3), (1, 4, 2048, 16), (1, 4, 2049, 16), (1, 4, 8193, 17), (1, 4, 1 << 30, 32),
+    (1, 4, 256, 1), (1, 4, 257, 3), (1, 4, 2048, 16), (1, 4, 2049, 16), (1, 4, 8193, 32), (1, 4, 1 << 30, 32),
     (8, 4, 300, 3), (63, 4, 4096, 2), (64, 4, 6143, 1), (64, 4, 6144, 3), (122, 8, 1 << 30, 1), (125, 8, 1 << 30, 1)])
 def test_decode_split_plan(lib, ns, hkv, ctx, want):
     """Both sides of each line of the split rule, and every plan's records within the 8 MiB of the
