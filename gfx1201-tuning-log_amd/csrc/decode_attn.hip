@@ -487,11 +487,13 @@ thread_local int g_target_wgs = 256;
 // of 4096: 0.76 of the time in two) and on unequal ones (1 to 8) as long as a split is short; the lines are
 // where the latter break even: none from six splits on (0.6-1.05), 2048 tokens a split for four and
 // five, 1024 below (60 x 4 pairs of 130..1024: 0.83; 33 x 4 of 187..1500: 13.9 us in one, 9.8 in two).
-// With a workgroup per CU or more from the pairs alone, the host knows only the longest context.
-// Long ones are split as often as kMaxPlannedRecords allows, because a ragged batch otherwise ends
-// with a few CUs walking its longest sequences (32 sequences of 512..8192, 8 kv heads, in three: 69.6
-// -> 62.0 us, bf16 126 -> 105); shorter ones are not (64 of 512..4096, 4 kv heads: 36.8 us in one,
-// 39.6 in three; 64 of 2048: 24.6 and 30.4).
+// With more than a workgroup per CU from the pairs alone, long contexts (the host knows only the longest) are
+// split as often as kMaxPlannedRecords allows: the last round of workgroups is otherwise partly empty, and a
+// batch of unequal lengths ends with a few CUs walking its longest sequences.  Time against one split,
+// longest 8192, shortest 1/16, 1/8, 1/4, 1/2 of it and equal: 40 x 8 pairs 0.82 0.84 0.83 0.82 0.80, 56 x 8
+// 0.81 0.82 0.85 0.90 1.04, 112 x 4 0.91 0.92 0.93 0.92 1.09 (e4m3; bf16 alike).  Exactly one workgroup per
+// CU has no empty round to fill: e4m3 0.98-1.04 on unequal contexts and 1.07 on equal ones, so one split; shorter
+// contexts neither (64 of 512..4096, 4 kv heads: 36.8 us in one, 39.6 in three).
 constexpr int kMaxPlannedSplits = 32;
 constexpr int kLongContext = 6144;
 // From here on a length says only that the contexts are not known (a graph under capture, replayed for
@@ -520,7 +522,7 @@ inline int plan_splits(int ns, int hkv, int max_seq_len)
         const int fill = fill_splits(pairs, max_seq_len);
         if (n > fill) n = fill;
     }
-    if (pairs >= kCus && max_seq_len >= kLongContext && max_seq_len < kUnknownContext) n = kMaxPlannedSplits;
+    if (pairs > kCus && max_seq_len >= kLongContext && max_seq_len < kUnknownContext) n = kMaxPlannedSplits;
     const int64_t most = kMaxPlannedRecords / pairs < kMaxPlannedSplits ? kMaxPlannedRecords / pairs : kMaxPlannedSplits;
     return n <= most ? n : most > 1 ? (int)most : 1;
 }
@@ -535,15 +537,19 @@ inline int plan_splits(int ns, int hkv, int max_seq_len)
 // CUs that drew two of the longest finish last, where variant 5 hands a CU its next workgroup as it falls
 // free (12 sequences of 2048..16384, 8 kv heads, in three: 74.5 / 52.4; of 16384 each 98.3 / 99.1).  The lines
 // are where ragged batches (1 to 8) break even: 1024 tokens a split up to two workgroups per CU (0.6-1.06
-// below, to 1.43 above), 2048 past that (0.6-1.02, to 1.12).  Contexts that are not known take 5.
-constexpr int kShareMaxSpan = 1024, kShareMaxSpanManyWgs = 2048;
+// below, to 1.43 above), 2048 past that (0.6-1.02, to 1.12), and 4096 where it is split counts that fill
+// the GPU more than twice, which spreads each sequence over the CUs already (0.68-1.09, 0.96-1.07 on
+// contexts of 6144 and more).  Contexts that are not known take 5, or 1 in the last case.
+constexpr int kShareMaxSpan = 1024, kShareMaxSpanManyWgs = 2048, kShareMaxSpanManySplits = 4096;
 
 inline int pick_variant(int64_t wgs, int nsplit, int max_seq_len)
 {
     if (g_variant >= 0) return g_variant;
     if (wgs <= kCus) return 1;
-    if (max_seq_len <= 0 || max_seq_len >= kUnknownContext) return 5;
-    return max_seq_len <= (int64_t)nsplit * (wgs <= 2 * kCus ? kShareMaxSpan : kShareMaxSpanManyWgs) ? 1 : 5;
+    const bool many = wgs > 2 * kCus;
+    if (max_seq_len <= 0 || max_seq_len >= kUnknownContext) return many && nsplit > 1 ? 1 : 5;
+    const int span = many ? (nsplit > 1 ? kShareMaxSpanManySplits : kShareMaxSpanManyWgs) : kShareMaxSpan;
+    return max_seq_len <= (int64_t)nsplit * span ? 1 : 5;
 }
 
 // Zero-fill of a decode scratch region (ticket counters and records), a kernel rather than a

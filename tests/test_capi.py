@@ -121,7 +121,7 @@ def test_decode_split_planner(lib):
 
 @pytest.mark.parametrize("ns,hkv,ctx,want", [
     (1, 4, 256, 1), (1, 4, 257, 3), (1, 4, 2048, 16), (1, 4, 2049, 16), (1, 4, 8193, 32), (1, 4, 1 << 30, 32),
-    (8, 4, 300, 3), (63, 4, 4096, 2), (64, 4, 6143, 1), (64, 4, 6144, 3), (122, 8, 1 << 30, 1), (125, 8, 1 << 30, 1)])
+    (8, 4, 300, 3), (63, 4, 4096, 2), (64, 4, 6143, 1), (64, 4, 6144, 1), (80, 4, 6143, 1), (80, 4, 6144, 3), (122, 8, 1 << 30, 1), (125, 8, 1 << 30, 1)])
 def test_decode_split_plan(lib, ns, hkv, ctx, want):
     """Both sides of each line of the split rule, and every plan's records within the 8 MiB of the
     call that takes no scratch, at the widest GQA."""
@@ -160,7 +160,8 @@ def test_decode_split_plan_bounds_hold_at_any_target(lib, target):
     (64, 4, 1, 0, 1), (64, 4, 1, 100000, 1), (8, 8, 4, 100000, 1),           # a workgroup per CU
     (65, 4, 1, 1024, 1), (65, 4, 1, 1025, 5), (65, 4, 1, 0, 5), (65, 4, 1, 1 << 30, 5),
     (12, 8, 3, 3072, 1), (12, 8, 3, 3073, 5), (128, 4, 1, 1025, 5),
-    (129, 4, 1, 2048, 1), (129, 4, 1, 2049, 5), (96, 4, 2, 4096, 1), (96, 4, 2, 4097, 5)])
+    (129, 4, 1, 2048, 1), (129, 4, 1, 2049, 5), (96, 4, 2, 8192, 1), (96, 4, 2, 8193, 5),
+    (96, 4, 2, 0, 1), (64, 4, 2, 0, 5), (64, 4, 2, 2049, 5)])
 def test_decode_variant_lines(lib, ns, hkv, splits, ctx, want):
     """Grids past one workgroup per CU share the CUs only where the caller's longest context says that a
     split is short."""
