@@ -493,7 +493,8 @@ thread_local int g_target_wgs = 256;
 // longest 8192, shortest 1/16, 1/8, 1/4, 1/2 of it and equal: 40 x 8 pairs 0.82 0.84 0.83 0.82 0.80, 56 x 8
 // 0.81 0.82 0.85 0.90 1.04, 112 x 4 0.91 0.92 0.93 0.92 1.09 (e4m3; bf16 alike).  Exactly one workgroup per
 // CU has no empty round to fill: e4m3 0.98-1.04 on unequal contexts and 1.07 on equal ones, so one split; shorter
-// contexts neither (64 of 512..4096, 4 kv heads: 36.8 us in one, 39.6 in three).
+// contexts neither (64 of 512..4096, 4 kv heads: 36.8 us in one, 39.6 in three).  Over bf16 caches 8 kv heads, which
+// put the same sequences on every XCD, still gain: 0.89 0.91 0.93 0.97 1.05 (4 heads: 0.95 0.98 1.03 1.08 1.07).
 constexpr int kMaxPlannedSplits = 32;
 constexpr int kLongContext = 6144;
 // From here on a length says only that the contexts are not known (a graph under capture, replayed for
@@ -503,26 +504,44 @@ constexpr int kUnknownContext = 1 << 30;
 constexpr int kMaxPlannedRecords = 976;
 
 // Splits that the workgroups of `pairs` pairs fill the GPU with (see above), pairs <= g_target_wgs.
-inline int fill_splits(int64_t pairs, int max_seq_len)
+inline int fill_splits(int64_t pairs, int max_seq_len, bool bf16)
 {
     const int64_t down = g_target_wgs / pairs;
-    const int64_t max_span = down >= 4 ? 2048 : 1024;
-    const bool up = g_target_wgs % pairs != 0 && down < 6 && max_seq_len > down * max_span;
+    const int64_t max_span = bf16 ? 512 : down >= 4 ? 2048 : 1024;
+    const bool up = g_target_wgs % pairs != 0 && (down < 6 || bf16) && max_seq_len > down * max_span;
     return (int)(up ? down + 1 : down);
 }
 
-inline int plan_splits(int ns, int hkv, int max_seq_len)
+// Splits that a context is worth on an empty GPU.
+inline int worth_splits(int len)
 {
-    if (max_seq_len <= 256) return 1;
+    return len <= 256 ? 1 : len <= 16 * 128 ? (len + 127) / 128 : len <= 16 * 512 ? 16 : kMaxPlannedSplits;
+}
+
+// bf16 caches hold twice the bytes per token, and their kernel keeps one workgroup per CU, so shorter spans
+// pay (24 / 4 heads, one sequence, us: 129 tokens 5.1 in one split and 5.3 in four, 256 6.2 and 5.2; 400 6.2 in
+// four, 5.8 in eight; 777 and 1024 6.5 and 6.7 in eight, 6.5 in 16; 5000 10.5 in 16 and in 32, 6144 11.2 and 11.1,
+// 8192 12.8 and 12.3, 12000 17.3 and 13.8; three sequences, whose 12 pairs leave room for 21, 6144: 11.9 in 16, 13.7
+// in 21; six, of 1024: 7.4 in eight, 8.0 in ten).  Counts that do not divide the CUs are rounded down up to 512 tokens a split (unequal contexts, 1 to 8: 0.67-1.0
+// of the time there, to 1.15 above; 10 of 512..4096, 4 kv heads: 16.8 in six, 14.3 in seven).
+inline int worth_splits_bf16(int len)
+{
+    return len <= 176 ? 1 : len <= 352 ? 4 : len <= 768 ? 8 : len <= 5632 ? 16 : kMaxPlannedSplits;
+}
+
+inline int plan_splits(int ns, int hkv, int max_seq_len, bool bf16)
+{
+    if (max_seq_len <= 1) return 1;
     const int64_t pairs = (int64_t)ns * hkv;
     int n = 1;
     if (pairs <= g_target_wgs) {
-        n = max_seq_len <= 16 * 128 ? (max_seq_len + 127) / 128
-          : max_seq_len <= 16 * 512 ? 16 : kMaxPlannedSplits;
-        const int fill = fill_splits(pairs, max_seq_len);
-        if (n > fill) n = fill;
+        n = bf16 ? worth_splits_bf16(max_seq_len) : worth_splits(max_seq_len);
+        const int fill = fill_splits(pairs, max_seq_len, bf16);
+        // the merge reads 8, 16 or 32 records: a count just past 8 or 16 pays for the next size on long spans only
+        if (n > fill) n = fill > 16 && max_seq_len <= 10240 ? 16 : bf16 && fill > 8 && fill < 16 && max_seq_len <= 2048 ? 8 : fill;
     }
-    if (pairs > kCus && max_seq_len >= kLongContext && max_seq_len < kUnknownContext) n = kMaxPlannedSplits;
+    if (max_seq_len >= kLongContext && max_seq_len < kUnknownContext && (pairs > kCus || (bf16 && pairs == kCus && hkv % 8 == 0)))
+        n = kMaxPlannedSplits;
     const int64_t most = kMaxPlannedRecords / pairs < kMaxPlannedSplits ? kMaxPlannedRecords / pairs : kMaxPlannedSplits;
     return n <= most ? n : most > 1 ? (int)most : 1;
 }
@@ -721,7 +740,13 @@ using namespace fp8kv::decode_detail;
 extern "C" int fp8kv_decode_num_splits(int num_seqs, int num_kv_heads, int max_seq_len)
 {
     if (num_seqs < 1 || num_kv_heads < 1) return 1;
-    return plan_splits(num_seqs, num_kv_heads, max_seq_len);
+    return plan_splits(num_seqs, num_kv_heads, max_seq_len, false);
+}
+
+extern "C" int fp8kv_decode_num_splits_bf16(int num_seqs, int num_kv_heads, int max_seq_len)
+{
+    if (num_seqs < 1 || num_kv_heads < 1) return 1;
+    return plan_splits(num_seqs, num_kv_heads, max_seq_len, true);
 }
 
 extern "C" size_t fp8kv_decode_scratch_bytes(int num_seqs, int num_q_heads, int num_kv_heads,

@@ -30,6 +30,7 @@ SIGNATURES: dict[str, tuple] = {
     "h4mv_repack_scales": (_c_i, [_c_vp, _c_vp, _c_i, _c_i, _c_vp]),
     # paged fp8 decode attention (csrc/decode_attn.hip)
     "fp8kv_decode_num_splits": (_c_i, [_c_i] * 3),
+    "fp8kv_decode_num_splits_bf16": (_c_i, [_c_i] * 3),
     "fp8kv_decode_scratch_bytes": (_c_sz, [_c_i] * 5),
     "fp8kv_decode_scratch_reset": (_c_i, [_c_vp, _c_sz, _c_vp]),
     "fp8kv_decode_attn_noalloc": (_c_i, [_c_vp, _c_i64, _c_vp, _c_vp] + [_c_i64] * 6 + [_c_vp, _c_i64]

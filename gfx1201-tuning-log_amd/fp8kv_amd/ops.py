@@ -89,8 +89,10 @@ _scratch_retired: list = []
 DECODE_SCRATCH_MIN_BYTES = 8 << 20
 
 
-def decode_num_splits(num_seqs: int, num_kv_heads: int, max_seq_len: int) -> int:
-    return int(_lib.load().fp8kv_decode_num_splits(num_seqs, num_kv_heads, max_seq_len))
+def decode_num_splits(num_seqs: int, num_kv_heads: int, max_seq_len: int, bf16_kv: bool = False) -> int:
+    lib = _lib.load()
+    plan = lib.fp8kv_decode_num_splits_bf16 if bf16_kv else lib.fp8kv_decode_num_splits
+    return int(plan(num_seqs, num_kv_heads, max_seq_len))
 
 
 def decode_scratch_bytes(num_seqs: int, num_q_heads: int, num_kv_heads: int, num_splits: int,
@@ -229,7 +231,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if num_splits is None:
         if max_seq_len is None:
             max_seq_len = int(seq_lens.max().item()) if NS > 0 else 0
-        num_splits = decode_num_splits(NS, HKV, int(max_seq_len))
+        num_splits = decode_num_splits(NS, HKV, int(max_seq_len), bf16_kv)
     need = decode_scratch_bytes(NS, HQ, HKV, num_splits, D)
     if scratch is None:
         scratch = _call_scratch(need, dev)

@@ -168,6 +168,9 @@ int fp8kv_decode_attn_noalloc(const void* q, int64_t q_row_stride,
  * alone, and a batch with a workgroup per CU from its (sequence, kv head) pairs is not split. */
 int fp8kv_decode_num_splits(int num_seqs, int num_kv_heads, int max_seq_len);
 
+/* The same for bf16 caches (fp8kv_decode_attn_bf16), whose tokens hold twice the bytes. */
+int fp8kv_decode_num_splits_bf16(int num_seqs, int num_kv_heads, int max_seq_len);
+
 /* Scratch bytes fp8kv_decode_attn needs for this geometry and split count (0 = none; 0 is also
  * returned for a geometry the kernel rejects).  Replaces the scratch sizing of
  * vllm-fp8kv/fp8kv_v3.py:121-124 and vllm-fp8kv/fp8kv_override.py:87-96. */

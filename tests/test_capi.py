@@ -133,12 +133,24 @@ def test_decode_split_plan(lib, ns, hkv, ctx, want):
 
 
 @pytest.mark.parametrize("ns,hkv,ctx,want", [
-    (6, 4, 1 << 30, 10), (10, 4, 1 << 30, 6),                        # from six on rounded down at any length
+    (3, 4, 10240, 16), (3, 4, 10241, 21), (6, 4, 1 << 30, 10), (10, 4, 1 << 30, 6),      # from six on rounded down at any length
     (12, 4, 5 * 2048, 5), (12, 4, 5 * 2048 + 1, 6), (14, 4, 4 * 2048, 4), (14, 4, 4 * 2048 + 1, 5),
     (20, 4, 3 * 1024, 3), (20, 4, 3 * 1024 + 1, 4), (33, 4, 1024, 1), (33, 4, 1025, 2), (33, 4, 1 << 30, 2),
     (16, 4, 100000, 4), (32, 4, 100000, 2)])                         # pairs that divide the CUs
 def test_decode_split_plan_rounds_by_span(lib, ns, hkv, ctx, want):
     assert lib.fp8kv_decode_num_splits(ns, hkv, ctx) == want
+
+
+@pytest.mark.parametrize("ns,hkv,ctx,want", [
+    (1, 4, 1, 1), (1, 4, 176, 1), (1, 4, 177, 4), (1, 4, 352, 4), (1, 4, 353, 8), (1, 4, 768, 8), (1, 4, 769, 16),
+    (1, 4, 5632, 16), (1, 4, 5633, 32), (3, 4, 10240, 16), (3, 4, 10241, 21), (6, 4, 2048, 8), (6, 4, 2049, 10), (6, 4, 5120, 10), (6, 4, 5633, 11), (24, 4, 1024, 2),
+    (24, 4, 1025, 3), (33, 4, 512, 1), (33, 4, 513, 2),
+    (32, 8, 6143, 1), (32, 8, 6144, 3), (64, 4, 6144, 1), (40, 8, 6144, 3), (32, 8, 1 << 30, 1), (200, 8, 9000, 1)])
+def test_decode_split_plan_bf16(lib, ns, hkv, ctx, want):
+    assert lib.fp8kv_decode_num_splits_bf16(ns, hkv, ctx) == want
+    for n in range(1, 400):
+        splits = lib.fp8kv_decode_num_splits_bf16(n, hkv, ctx)
+        assert 1 <= splits <= 32 and lib.fp8kv_decode_scratch_bytes(n, 16 * hkv, hkv, 128, splits) <= 8 << 20
 
 
 @pytest.mark.parametrize("target", [1, 32, 256, 4096, 1 << 30])
