@@ -99,22 +99,29 @@ __device__ __forceinline__ void v_fragments_b16(const u32x4_t (&vr)[8], u32x4_t 
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 
-// D += A . B^T over 128 k on the block-scaled MFMA with e4m3 A and B (both block scales 1.0):
-// lane (r, p) supplies row r's k 16p .. 16p+15 in bytes 0..15 and 64+16p .. +15 in bytes 16..31
-// of each operand; the products are exact and accumulate in fp32.
+// Exponent of the lo part of a split query row (q_fp8_split).
+constexpr int kQLoExp = -5;
+
+// D += A . B^T over 128 k (times 2^kQLoExp with LO) on the block-scaled MFMA with e4m3 A and B: lane (r, p)
+// supplies row r's k 16p .. 16p+15 in bytes 0..15 and 64+16p .. +15 in bytes 16..31 of each operand; the
+// products are exact and accumulate in fp32.  Both scales are bytes of one register.
+template <bool LO>
 __device__ __forceinline__ f32x4_t mfma_fp8_16x16x128(const v8i& a, const v8i& b, f32x4_t c)
 {
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 0, 127);
+    constexpr int scales = 127 | (127 + kQLoExp) << 8;
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, scales, LO ? 1 : 0, scales);
 }
 
 // One query row's 32 bf16 values held by this lane (the 128-value row is spread over the four
-// lanes n, n + 16, n + 32, n + 48) -> e4m3 hi and lo parts with q * 2^e = hi + lo, where 2^e is
-// the row's scale: the largest |q| of the row times 2^e lies in [128, 256).  Returns 2^-e.
-// hi is q * 2^e rounded to 4 significant bits; the remainder lo is a multiple of the bf16 value's
-// last place below 2^-4 of it, exact in e4m3 whenever |q| >= 2^-9 of the row's largest |q| (the
-// subnormal range covers smaller values to 2^-10 of their place).  The products of the two MFMAs
-// with exact e4m3 K then sum to the bf16 path's S up to fp32 accumulation order.  sign_mask
-// (0x80808080 or 0) negates the row in e4m3 (exact).
+// lanes n, n + 16, n + 32, n + 48) -> e4m3 hi and lo parts with q * 2^e = hi + lo * 2^kQLoExp, where 2^e
+// is the row's scale: the largest |q| of the row times 2^e lies in [128, 256).  Returns 2^-e.
+// hi is q * 2^e rounded to 4 significant bits; the remainder, at most 8, is a multiple of the bf16 value's
+// last place below 2^-4 of it, and is held 2^5 times as large so that it uses the range of its own: it is
+// exact wherever |q| >= 2^-14 of the row's largest, and smaller values are off by at most 2^-22 of the
+// largest (in units of hi the line was 2^-9 and the error 2^-17, which a dimension some hundred times the
+// others carried into their scores).  The products of the two MFMAs with exact e4m3 K then sum to the bf16
+// path's S up to fp32 accumulation order and that bound.  sign_mask (0x80808080 or 0) negates the row in
+// e4m3 (exact).
 __device__ __forceinline__ float q_fp8_split(const u32x4_t (&qf)[4], uint32_t sign_mask, v8i& hi, v8i& lo)
 {
     float amax = 0.f;
@@ -144,8 +151,9 @@ __device__ __forceinline__ float q_fp8_split(const u32x4_t (&qf)[4], uint32_t si
             hw = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], (int)hw, true);
             const auto h01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hw, false);
             const auto h23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hw, true);
-            uint32_t lw = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[0] - h01[0], x[1] - h01[1], 0, false);
-            lw = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2] - h23[0], x[3] - h23[1], (int)lw, true);
+            constexpr float up = (float)(1 << -kQLoExp);
+            uint32_t lw = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32((x[0] - h01[0]) * up, (x[1] - h01[1]) * up, 0, false);
+            lw = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32((x[2] - h23[0]) * up, (x[3] - h23[1]) * up, (int)lw, true);
             // chunk c holds d 16p + 8 (c & 1) + 4 h .. of the low half (c < 2) or the high half
             const int slot = 4 * (c >> 1) + 2 * (c & 1) + h;
             hw ^= sign_mask;

@@ -673,9 +673,6 @@ prefill_split_kernel(Params P)
         const int ntiles = (k_hi + kBN - 1) / kBN;
         const int nwin = (ntiles + NT - 1) / NT;
 
-        // Q as the B operand of S^T = K.Q^T (lane (n, p): d 16p .. 16p+15 and 64+16p .. +15 of query
-        // row n).  e4m3 caches: split exactly into e4m3 hi + lo parts (q_fp8_split), the row's scale
-        // folded into this lane's softmax factor qkr.  bf16 caches: the four bf16 fragments.
         auto token_of = [&](int j) { return tok0 + 16 * block_of(grp * RS + j) + lr; };
 
         // Block ids for this wave's copy instruction of each tile of window wi (its 8 rows lie
@@ -714,7 +711,7 @@ prefill_split_kernel(Params P)
             }
         };
         // Q as the B operand of S^T = K.Q^T (lane (n, p): d 16p .. 16p+15 and 64+16p .. +15 of query
-        // row n).  e4m3 caches: split exactly into e4m3 hi + lo parts (q_fp8_split), the row's scale
+        // row n).  e4m3 caches: split into e4m3 hi + lo parts (q_fp8_split has the bound), the row's scale
         // folded into this lane's softmax factor qkr.  The split is about 270 VALU a row-set, and the
         // NR residues of a head group need the same ones, so each row-set is split by one wave and
         // handed over through the LDS (the ring's second window is free until the key loop's first barrier)
@@ -880,8 +877,8 @@ prefill_split_kernel(Params P)
 #pragma unroll
                         for (int kg = 0; kg < 2; ++kg) {
                             const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-                            f32x4_t acc = mfma_fp8_16x16x128(kf[kg], qhi[j], zero);
-                            sc[j][kg] = mfma_fp8_16x16x128(kf[kg], qlo[j], acc);
+                            f32x4_t acc = mfma_fp8_16x16x128<false>(kf[kg], qhi[j], zero);
+                            sc[j][kg] = mfma_fp8_16x16x128<true>(kf[kg], qlo[j], acc);
                         }
                     // Interleave: one MFMA, then up to four VALU (the V widening, 48 instructions).
 #pragma unroll

@@ -459,3 +459,18 @@ def test_bf16_kv_through_the_reference_run():
     torch.cuda.synchronize()
     ref = _oracle_single(c, 100, 200).to(torch.float64)
     torch.testing.assert_close(out.cpu().to(torch.float64), ref, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("outlier", [300.0, 2048.0])
+@pytest.mark.parametrize("hq", [24, 28, 16, 4])
+def test_query_row_with_an_outlier_dimension(hq, outlier):
+    """One dimension far above the others, against keys that are zero there, so that the small elements
+    alone make the scores.  The key-split kernel holds them within 2^-22 of the row's largest: at 2048
+    times the others a score of standard deviation 8 is off by 2048 * 2^-22 / sqrt(3) * 8 = 2.3e-3 rms, below
+    the bf16 rounding of the probabilities (a remainder in units of the row's scale: 2^5 times that)."""
+    c = workloads.prefill_case([350], [300], HQ=hq, HKV=4, seed=hq)
+    c["q"][..., 5] = outlier * torch.sign(c["q"][..., 5].float()).to(torch.bfloat16)
+    c["k_cache"].view(torch.uint8)[..., 5] = 0
+    c["sm_scale"] = 8 / 128 ** 0.5
+    got = _run_single(c, 300, 350).to(torch.float64)
+    torch.testing.assert_close(got, _oracle_single(c, 300, 350).to(torch.float64), rtol=RTOL, atol=ATOL)
