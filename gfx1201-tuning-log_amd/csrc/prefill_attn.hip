@@ -446,8 +446,14 @@ constexpr int kStageFloats = 8 * 64 * 4 + 64;        // one row-set: o [n][lane]
 // Running-max floor of the key-split kernel: finite, so that no -inf ever enters the softmax
 // arithmetic (exp2(kMaxFloor - m) is 0 for any real row max m, and a row that has seen no key
 // keeps l = 0 and o = 0).
-constexpr float kMaxFloor = -1e30f;
-constexpr float kMaxFloor16 = -3e38f;      // bf16 caches are not bounded by a scale: below any finite score
+constexpr float kMaxFloor = -3e38f;
+// Smallest softmax factor of a row, so that -inf * factor stays -inf where a scale is 0: times the largest
+// score it is applied to (e4m3: 256 * 448 * 128 in units of the row's scale; bf16: any) it is 0 to exp2.
+constexpr float kMinFactor = 1e-37f, kMinFactor16 = 1.4e-45f;
+// Largest e4m3 factor: the scores it is applied to stay below 2^30 and row_probs may fuse.  A row past it, which
+// takes scores of full-range keys to 10^9, is held there: that leaves the weights alone wherever the largest
+// score stands out by 24 / kMaxFactor = 0.33 of those units or is shared.
+constexpr float kMaxFactor = 1073741824.f / (256.f * 448.f * 128.f);
 
 // max without the NaN-quieting canonicalisation the compiler adds to fmaxf of values that come
 // from MFMA results or lane swaps (the scores are never NaN: finite fp8 and bf16 inputs).
@@ -518,8 +524,8 @@ __device__ __forceinline__ void rescale_rows(const f32x4_t (&sc)[RS][2], float (
 
 // Probabilities of row-set j's tile in bf16 (the P^T operand), their fp32 sum added to l.  FUSED takes
 // score * qk - m in one fma: m is the rounded product of the row's largest score, so beyond |m| ~ 1e9
-// the difference is the rounding error, not 0.  e4m3 scores stay far below; bf16 ones are unbounded
-// and round the product like m.
+// the difference is the rounding error, not 0.  kMaxFactor keeps e4m3 scores below that; bf16 ones are
+// unbounded and round the product like m (which costs an e4m3 call 2.7%, and a branch between the two spills).
 template <bool FUSED>
 __device__ __forceinline__ u32x4_t row_probs(const f32x4_t (&sc)[2], float qk, float m_run, float& l)
 {
@@ -574,7 +580,6 @@ __global__ void __launch_bounds__(kSplitWaves * 64)
 prefill_split_kernel(Params P)
 {
     constexpr int W = kSplitWaves;
-    constexpr float floor_m = B16 ? kMaxFloor16 : kMaxFloor;
     constexpr int TILE = B16 ? kTileBytes16 : kTileBytes;
     constexpr int RW = 2;                                  // ring windows
     constexpr int NR = W / NG;
@@ -631,9 +636,10 @@ prefill_split_kernel(Params P)
     const int nphase = blk_b > blk_a ? 2 : 1;
     const int32_t* btrow = P.bt + (int64_t)seq * P.bt_stride;
     const float qk_signed = B16 ? P.sm_scale * kLog2e : P.sm_scale * P.k_scale[0] * kLog2e;
-    const float qk = fmaxf(fabsf(qk_signed), 1e-30f);         // > 0: -inf * qk stays -inf
+    auto uniform = [](float f) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(f))); };
+    const float qk = uniform(fabsf(qk_signed));                // a NaN reaches the output through vs
     const uint32_t qflip = qk_signed < 0.f ? (B16 ? 0x80008000u : 0x80808080u) : 0u;   // negate Q (exact)
-    const float vs = B16 ? 1.f : P.v_scale[0];
+    const float vs = uniform((B16 ? 1.f : P.v_scale[0]) + (qk_signed == qk_signed ? 0.f : qk_signed));
 
     // This wave's copies of every tile, lane (row, chunk).  e4m3: one, of K rows (waves 0-3) or V rows
     // (waves 4-7) 8 (wave & 3) .. +7, as chosen by dma_lane_rc; bf16: two, of K and V rows 4 wave .. +3.
@@ -739,7 +745,7 @@ prefill_split_kernel(Params P)
 #pragma unroll
             for (int j = 0; j < RS; ++j) {
                 asm volatile("" : "+v"(qf[j][0]), "+v"(qf[j][1]), "+v"(qf[j][2]), "+v"(qf[j][3]));
-                qkr[j] = qk;
+                qkr[j] = fmaxf(qk, kMinFactor16);
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
                     qhi[j][d] = (int)(qf[j][0][d] ^ qflip);
@@ -777,7 +783,7 @@ prefill_split_kernel(Params P)
                     *reinterpret_cast<u32x4_t*>(x + 1024) = (u32x4_t){(uint32_t)hi[4], (uint32_t)hi[5], (uint32_t)hi[6], (uint32_t)hi[7]};
                     *reinterpret_cast<u32x4_t*>(x + 2048) = (u32x4_t){(uint32_t)lo[0], (uint32_t)lo[1], (uint32_t)lo[2], (uint32_t)lo[3]};
                     *reinterpret_cast<u32x4_t*>(x + 3072) = (u32x4_t){(uint32_t)lo[4], (uint32_t)lo[5], (uint32_t)lo[6], (uint32_t)lo[7]};
-                    *reinterpret_cast<float*>(exch + rset * kSetBytes + 4096 + 4 * ln) = inv;
+                    *reinterpret_cast<float*>(exch + rset * kSetBytes + 4096 + 4 * ln) = fminf(fmaxf(qk * inv, kMinFactor), kMaxFactor);
                 }
             }
             lds_barrier();
@@ -791,7 +797,7 @@ prefill_split_kernel(Params P)
                                (int)v[1][0], (int)v[1][1], (int)v[1][2], (int)v[1][3]};
                 qlo[j] = (v8i){(int)v[2][0], (int)v[2][1], (int)v[2][2], (int)v[2][3],
                                (int)v[3][0], (int)v[3][1], (int)v[3][2], (int)v[3][3]};
-                qkr[j] = qk * *reinterpret_cast<const float*>(exch + (grp * RS + j) * kSetBytes + 4096 + 4 * ln);
+                qkr[j] = *reinterpret_cast<const float*>(exch + (grp * RS + j) * kSetBytes + 4096 + 4 * ln);
             }
         }
 
@@ -799,7 +805,7 @@ prefill_split_kernel(Params P)
         f32x4_t o[RS][8];
 #pragma unroll
         for (int j = 0; j < RS; ++j) {
-            m_run[j] = floor_m;
+            m_run[j] = kMaxFloor;
             l_run[j] = 0.f;
 #pragma unroll
             for (int n = 0; n < 8; ++n) o[j][n] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -952,7 +958,7 @@ prefill_split_kernel(Params P)
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < RS; ++j) {
-                float mg = floor_m;
+                float mg = kMaxFloor;
 #pragma unroll
                 for (int r = 0; r < NR; ++r) mg = fmaxf(mg, stage_m[((grp * NR + r) * RS + j) * 16 + lr]);
                 const float f = __builtin_amdgcn_exp2f(m_run[j] - mg);

@@ -474,3 +474,29 @@ def test_query_row_with_an_outlier_dimension(hq, outlier):
     c["sm_scale"] = 8 / 128 ** 0.5
     got = _run_single(c, 300, 350).to(torch.float64)
     torch.testing.assert_close(got, _oracle_single(c, 300, 350).to(torch.float64), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("kv_gen", ["amax", "bf16"])
+@pytest.mark.parametrize("hq", [24, 28])
+def test_key_split_scale_edges(hq, kv_gen):
+    """A softmax scale of 0 gives every key the same weight however large q is, and a NaN scale gives NaN."""
+    c = workloads.prefill_case([340], [30], HQ=hq, HKV=4, seed=hq + 1, kv_gen=kv_gen)
+    c["q"].mul_(1e30)
+    c["sm_scale"] = 0.0
+    got = _run_single(c, 30, 340).to(torch.float64)
+    ref = workloads.prefill_case([340], [30], HQ=hq, HKV=4, seed=hq + 1, kv_gen=kv_gen)
+    ref["sm_scale"] = 0.0
+    torch.testing.assert_close(got, _oracle_single(ref, 30, 340).to(torch.float64), rtol=RTOL, atol=ATOL)
+    c["sm_scale"] = float("nan")
+    assert torch.isnan(_run_single(c, 30, 340)).all()
+
+
+@pytest.mark.parametrize("hq", [24, 28, 64])
+@pytest.mark.parametrize("q", [1e9, -1e9, 3e30])
+def test_key_split_scores_past_the_fused_range(hq, q):
+    """Scores from 1e11 to 1e33 in log2 units, equal for the keys of a row: each row averages the V rows it sees."""
+    c = workloads.prefill_case([340], [30], HQ=hq, HKV=4, seed=hq + 2)
+    c["q"].fill_(q)
+    c["k_cache"].view(torch.uint8).fill_(0x7A)                  # 320
+    got = _run_single(c, 30, 340, 1.0).to(torch.float64)
+    torch.testing.assert_close(got, _oracle_single(c, 30, 340, 1.0).to(torch.float64), rtol=RTOL, atol=ATOL)
