@@ -678,6 +678,10 @@ prefill_split_kernel(Params P)
         const int k_hi = q0 + min(tok0 + 16 * nbt, qlen);         // keys [0, k_hi)
         const int ntiles = (k_hi + kBN - 1) / kBN;
         const int nwin = (ntiles + NT - 1) / NT;
+        // Several blocks: a wave leaves out the tiles above the diagonal of its own.  They cost time, and an
+        // infinity or NaN in the V row of a later token reaches the rows of every tile that holds it (0 * V).
+        // At GQA 1 a wave's two blocks share their last tile (leaving out one row-set only spills).
+        const int my_tiles = MB ? min(ntiles, (qpos0 + 16 * block_of(grp * RS + RS - 1) + 15) / kBN + 1) : ntiles;
 
         auto token_of = [&](int j) { return tok0 + 16 * block_of(grp * RS + j) + lr; };
 
@@ -826,7 +830,7 @@ prefill_split_kernel(Params P)
                 if (more) issue_window(i + RW - 1, v * NT / TPW, (v + 1) * NT / TPW);
                 const int tw = res * TPW + v;                    // tile within the window
                 const int t = i * NT + tw;
-                if (t >= ntiles) continue;
+                if (t >= my_tiles) continue;
                 const int k0 = t * kBN;
                 const unsigned char* buf = ring + (i % RW) * kWinBytes + tw * TILE;
                 f32x4_t sc[RS][2];

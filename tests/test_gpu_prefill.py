@@ -500,3 +500,32 @@ def test_key_split_scores_past_the_fused_range(hq, q):
     c["k_cache"].view(torch.uint8).fill_(0x7A)                  # 320
     got = _run_single(c, 30, 340, 1.0).to(torch.float64)
     torch.testing.assert_close(got, _oracle_single(c, 30, 340, 1.0).to(torch.float64), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("kv_gen", ["amax", "bf16"])
+@pytest.mark.parametrize("paired", [False, True])
+@pytest.mark.parametrize("hq", [4, 8, 12])
+def test_key_split_leaves_later_tokens_out(hq, paired, kv_gen):
+    """GQA 1, 2 and 3.  A NaN V row reaches a query only through a tile that holds keys which the rows of its
+    wave see: 16 of them, two blocks at GQA 1.  Rows whose blocks end before the NaN's 32-key tile stay finite
+    and equal the oracle, whatever else their workgroup owns.  The first offset leaves blocks and tiles
+    aligned, the second moves them half a tile."""
+    lib = _lib.load()
+    tune = (lib.fp8kv_prefill_tune, (18, 19), -1) if kv_gen == "amax" else (lib.fp8kv_prefill_bf16_tune, (3, 4), 0)
+    try:
+        tune[0](tune[1][paired])
+        for q0 in (64, 80):
+            c = workloads.prefill_case([150], [q0], HQ=hq, HKV=4, seed=hq + q0, kv_gen=kv_gen)
+            want = _oracle_single(c, q0, 150).to(torch.float64)
+            for tok in (16, 47, 63, 100, 149):
+                key = q0 + tok
+                bad = dict(c, v_cache=c["v_cache"].clone())
+                v = bad["v_cache"][int(c["block_table"][0, key // 16]), key % 16]
+                v.view(torch.uint8).fill_(0x7F) if kv_gen == "amax" else v.fill_(float("nan"))
+                got = _run_single(bad, q0, 150).to(torch.float64)
+                rows = 32 if hq == 4 else 16
+                clean = [t for t in range(150) if q0 + t // rows * rows + rows - 1 < key // 32 * 32]
+                torch.testing.assert_close(got[clean], want[clean], rtol=RTOL, atol=ATOL)
+                assert torch.isnan(got[tok:]).all()
+    finally:
+        tune[0](tune[2])
