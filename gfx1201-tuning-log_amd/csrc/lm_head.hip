@@ -192,10 +192,13 @@ merge_topk_kernel(const uint64_t* __restrict__ cand, int ncand, int k, float* __
 
 // Dot product of a candidate's embedding row with the activation row over one wave (bf16 products
 // summed in fp32, 8-element piece p on lane p % 64, pieces in order, then a butterfly over the
-// lanes).  The loads of kRowBatch pieces per lane go out together - one row of 3584 is 7 - because a
-// row is a random 7 KB of a table far above the caches, and a load per iteration would pay its full
-// round trip every time.  Pieces past the row re-read its last one and count as zero.
-constexpr int kRowBatch = 8;
+// lanes).  The loads of kRowBatch pieces per lane go out together, because a row is a random 7 KB of a
+// table far above the caches, and a load per iteration would pay its full round trip every time.  Four
+// pieces, half a row of 3584, hide as much as eight and leave room for more waves (16 candidates, us per call
+// in a graph: 1024 rows 21.8 against 25.6, 4096 rows 73.5 / 93.0, one row 4.5 both).  Past the row's end no load is
+// issued (a lane past the last piece of a partly filled 64 re-reads that piece and counts zero): issued all the
+// same, they cost rows of 1024, two pieces a lane, up to three times the time.
+constexpr int kRowBatch = 4;
 
 __device__ __forceinline__ float row_score(const __bf16* x, const __bf16* e, int pieces, int lane)
 {
@@ -204,12 +207,14 @@ __device__ __forceinline__ float row_score(const __bf16* x, const __bf16* e, int
         u32x4_t a[kRowBatch], b[kRowBatch];
 #pragma unroll
         for (int i = 0; i < kRowBatch; ++i) {
+            if (p0 + 64 * i >= pieces) break;                                // uniform
             const int p = min(p0 + 64 * i + lane, pieces - 1);
-            b[i] = load_nt_16(e + 8 * p);
+            b[i] = load_16(e + 8 * p);
             a[i] = load_16(x + 8 * p);
         }
 #pragma unroll
         for (int i = 0; i < kRowBatch; ++i) {
+            if (p0 + 64 * i >= pieces) break;
             if (p0 + 64 * i + lane >= pieces) a[i] = b[i] = (u32x4_t){0u, 0u, 0u, 0u};
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
@@ -239,28 +244,34 @@ __device__ __forceinline__ void write_ranked(const uint64_t* keys, int C, int m,
     out_idx[(size_t)m * C + rank] = mine ? key_index(mine) : -1;
 }
 
-// Exact rerank of C candidate rows of E against X[m].  The reads are M * C rows at random addresses,
-// so latency bounds it, and one workgroup per row of X leaves nearly all CUs idle.  Up to
-// kRerankOneMaxC candidates: one launch, grid (M), a wave per candidate.  More: rerank_score_kernel
-// gives every candidate of every row its own wave over the whole GPU (the scores wait in out_val),
-// and rerank_order_kernel sorts each row in place.  Measured in a graph, H = 3584, 128167 rows, us
-// per call at M = 1 / 4 / 16: 64 candidates 6.2 / 6.7 / 7.2 in two launches, 16.7 / 17.1 / 17.7 with
-// 16 waves in one, 45 / 63 / 67 with four waves and a load per iteration; 8 candidates at M = 4: 4.2
-// in one launch, 5.2 in two.
+// Exact rerank of C candidate rows of E against X[m].  The reads are M * C rows at random addresses.  With few rows
+// of X latency bounds it, and one workgroup per row of X leaves nearly all CUs idle: up to
+// kRerankOneMaxC candidates take one launch, grid (M), a wave per candidate; more take two:
+// rerank_score_kernel gives every candidate of every row its own wave over the whole GPU (the scores wait in
+// out_val), and rerank_order_kernel sorts each row in place.  From kRerankManyRows rows on the workgroups fill the
+// GPU by themselves and starting a wave per candidate is what costs: one launch, eight waves a row (H = 1024, 64
+// candidates: 512 rows 14.9 against 17.7 in two, 24.1 with four waves and a load per iteration, 4096 rows 79 /
+// 90 / 79; H = 3584: 41.7 / 43.4 / 77.7 and 282 / 290 / 321).  Measured in a
+// graph, H = 3584, 128167 rows, us per call at M = 1 / 4 / 16: 64 candidates 6.2 / 6.7 / 7.2 in two launches,
+// 16.7 / 17.1 / 17.7 with 16 waves in one, 45 / 63 / 67 with four waves and a load per iteration; 8 candidates
+// at M = 4: 4.2 in one launch, 5.2 in two.
 constexpr int kRerankOneMaxC = 16;
+constexpr int kRerankManyRows = 512;
+constexpr int kRerankManyWaves = 8;
 
 __global__ void __launch_bounds__(64 * kRerankOneMaxC)
 rerank_kernel(const __bf16* __restrict__ E, int64_t e_stride, int V, const __bf16* __restrict__ X,
               int64_t x_stride, const int32_t* __restrict__ cand, int C, int H,
               float* __restrict__ out_val, int32_t* __restrict__ out_idx)
 {
-    __shared__ uint64_t keys[kRerankOneMaxC];
+    __shared__ uint64_t keys[kMaxRerank];
     const int m = blockIdx.x, lane = threadIdx.x & 63;
-    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);        // the grid has a wave per candidate
-    const int32_t idx = cand[(size_t)m * C + c];
-    const bool ok = idx >= 0 && idx < V;
-    const float s = row_score(X + (int64_t)m * x_stride, E + (int64_t)(ok ? idx : 0) * e_stride, H / 8, lane);
-    if (lane == 0) keys[c] = ok ? rank_key(s, (uint32_t)idx) : 0;
+    for (int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); c < C; c += blockDim.x >> 6) {
+        const int32_t idx = cand[(size_t)m * C + c];
+        const bool ok = idx >= 0 && idx < V;
+        const float s = row_score(X + (int64_t)m * x_stride, E + (int64_t)(ok ? idx : 0) * e_stride, H / 8, lane);
+        if (lane == 0) keys[c] = ok ? rank_key(s, (uint32_t)idx) : 0;
+    }
     __syncthreads();
     write_ranked(keys, C, m, out_val, out_idx);
 }
@@ -356,8 +367,9 @@ extern "C" int fp8kv_rerank_exact(const void* E, int64_t e_row_stride, int V, co
     const __bf16* x = static_cast<const __bf16*>(X);
     const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     begin_launch();
-    if (C <= kRerankOneMaxC) {
-        launch_kernel(rerank_kernel, dim3((unsigned)M), dim3(64 * C), 0, st, e, e_row_stride, V, x, x_row_stride,
+    const int waves = M < kRerankManyRows ? C : C < kRerankManyWaves ? C : kRerankManyWaves;
+    if (waves <= kRerankOneMaxC) {
+        launch_kernel(rerank_kernel, dim3((unsigned)M), dim3(64 * waves), 0, st, e, e_row_stride, V, x, x_row_stride,
                       cand_idx, C, H, out_val, out_idx);
         return finish_launch();
     }

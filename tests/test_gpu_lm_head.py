@@ -123,10 +123,12 @@ def test_rerank_exact_against_oracle():
 
 
 @pytest.mark.parametrize("M,C,H", [(1, 1, 8), (3, 15, 512), (2, 16, 4096), (2, 17, 4096), (1, 33, 4104),
-                                   (5, 64, 520), (65540, 18, 8)])
+                                   (5, 64, 520), (65540, 18, 8), (511, 64, 2056), (512, 64, 2048), (600, 9, 1544),
+                                   (700, 3, 512)])
 def test_rerank_launch_forms(M, C, H):
-    """One launch (C <= 16) and two, a row of one piece, exactly one batch of loads per lane (4096), one
-    piece past it, partial batches, and more rows than a grid's second dimension holds.  The scores
+    """One launch (C <= 16) and two, a row of one piece, whole batches of loads per lane (2048, 4096), one
+    piece past them, partial batches, and from 512 rows on eight waves a row, with more, fewer and as many
+    candidates.  The scores
     are integers that fp32 holds exactly, so values and order are the oracle's."""
     V = 300
     g = torch.Generator().manual_seed(M + C + H)
