@@ -1080,11 +1080,20 @@ constexpr int kSplitRoundWorkgroups = 256;
 // Token-block ranks per (sequence, kv head) padded for the XCD-aware grid (8 % HKV == 0).
 inline int split_xcd_per(int hkv) { return (hkv <= 8 && 8 % hkv == 0) ? 8 / hkv : 1; }
 
-// True when one 16-token block per workgroup fits in one round of the key-split kernel.
-inline bool split_single_blocks_fit(int n16, int hkv, int num_seqs, int rounds = 1)
+// Workgroups of a grid of n ranks per sequence and kv head, and whether the key-split kernel runs them in
+// one round: with one 16-token block each, n blocks, or with pairs of them, (n + 1) / 2.
+inline int64_t split_workgroups(int n, int hkv, int num_seqs)
 {
     const int per = split_xcd_per(hkv);
-    return (int64_t)((n16 + per - 1) / per * per) * hkv * num_seqs <= rounds * kSplitRoundWorkgroups;
+    return (int64_t)((n + per - 1) / per * per) * hkv * num_seqs;
+}
+inline bool split_single_blocks_fit(int n16, int hkv, int num_seqs)
+{
+    return split_workgroups(n16, hkv, num_seqs) <= kSplitRoundWorkgroups;
+}
+inline bool split_pairs_fit(int n16, int hkv, int num_seqs)
+{
+    return split_workgroups((n16 + 1) / 2, hkv, num_seqs) <= kSplitRoundWorkgroups;
 }
 
 // Contexts (in keys) from which the key-split kernel beats the per-wave kernel, measured on MI355X.
@@ -1097,17 +1106,20 @@ constexpr int kSplitMinContext = 1024;
 // (6 prompts of 37..900 after 200, GQA 8 / 12 / 6: 46 / 88 / 59 us against 58 / 93 / 55 per wave; 8 of 600:
 // 48 / 98 / 72 against 46 / 94 / 59).
 constexpr int kSplitMinContextFewParts = 768;
-// Below GQA 4 the per-wave kernel has few row-sets to share a conversion (4 of 512, GQA 1 / 3: 21.5 / 20.1
-// us against 27 / 26.5 per wave).
-constexpr int kSplitMinContextLowGqa = 512;
+// Below GQA 4 the per-wave kernel has few row-sets to share a conversion, but its workgroups are small: past one
+// round of pairs it is the split kernel that runs a second, partly empty one.  GQA 1: from 1024 keys (5 of 512,
+// 16 / 16 heads, in two rounds 33.5 us per wave and 35.9 split, 8 of 320..520 31 and 37); GQA 2: 640 (8 of 600, 8 / 4,
+// 36.5 and 37.8); GQA 3: single prompts only (8 of 600, 12 / 4, 36.7 and 56.0; 3 of 1500 0.79 of the time per wave, 6 of
+// 1400 0.88; one of 3000 1.47).
+constexpr int kSplitMinContextGqa1 = 1024, kSplitMinContextGqa2 = 640;
 // GQAs without a shape of their own (us, split against per wave; 2048 tokens after 2048, 28 / 4 heads 123 /
 // 194, 16 / 16 75 / 140, 8 / 4 49 / 132, 12 / 4 74 / 140, 20 / 4 93 / 187, 40 / 4 158 / 248; 1000 after 500, 28 / 4
 // 34 / 68, 16 / 16 22 / 48).  Prompts up to 300 tokens stay on the per-wave kernel, as the launch
 // plan's test has them, although contexts of 1000 keys would gain there too.
 constexpr int kSplitMinQueryInexact = 320;
 constexpr int kSplitMinContextSingle = 256;
-// In two rounds: 512 (4 of 512, 24 / 4 heads: 26.6 us against 28.1 per wave, 48 / 4: 37 against 48).
-constexpr int kSplitMinContextTwoRounds = 512;
+// In one round of pairs: 512 (4 of 512, 24 / 4 heads: 26.6 us against 28.1 per wave, 48 / 4: 37 against 48).
+constexpr int kSplitMinContextPairs = 512;
 
 // One launch as planned from the shape alone (no pointers): kernel, block pairing and grid.
 struct Plan {
@@ -1143,10 +1155,11 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
             force_paired = g_shape > kSplitAnyShape;
         }
     } else if (g_shape < 0) {
-        const int many = gqa < 4 ? kSplitMinContextLowGqa
+        const int many = gqa == 1 ? kSplitMinContextGqa1 : gqa == 2 ? kSplitMinContextGqa2
+                       : gqa == 3 && num_seqs > 1 ? INT32_MAX
                        : kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext;
         split = ctx_hint >= many || (ctx_hint >= kSplitMinContextSingle && fits) ||
-                (ctx_hint >= kSplitMinContextTwoRounds && split_single_blocks_fit(nsb, hkv, num_seqs, 2));
+                (ctx_hint >= kSplitMinContextPairs && split_pairs_fit(nsb, hkv, num_seqs));
         if (!exact && max_query_len < kSplitMinQueryInexact) split = false;
     }
     if (split) {

@@ -107,6 +107,18 @@ def test_empty_and_invalid(lib):
     assert lib.fp8kv_prefill_plan(24, 4, 1, 10, 10, None) == 1
 
 
+@pytest.mark.parametrize("hq,hkv,num_seqs,max_q,ctx,split", [
+    (16, 16, 2, 1000, 1000, 1), (16, 16, 5, 1000, 1000, 0), (16, 16, 5, 1024, 1024, 1),     # GQA 1
+    (4, 4, 12, 512, 512, 1), (4, 4, 12, 600, 600, 0),                   # 5 pairs of superblocks, rounded to 6: 288
+    (8, 4, 8, 600, 600, 0), (8, 4, 8, 640, 640, 1), (8, 4, 5, 600, 600, 1),                 # GQA 2
+    (12, 4, 4, 512, 512, 1), (12, 4, 4, 600, 600, 0), (12, 4, 3, 1500, 1500, 0),            # GQA 3
+    (12, 4, 1, 3000, 3000, 1), (12, 4, 8, 320, 320, 0)])
+def test_low_gqa_lines(lib, hq, hkv, num_seqs, max_q, ctx, split):
+    """Below GQA 4 the key-split kernel takes one round of single blocks or of pairs, and beyond it only the
+    contexts that pay for a second, partly empty one."""
+    assert plan(lib, hq, hkv, num_seqs, max_q, ctx)["split"] == split
+
+
 @pytest.mark.parametrize("hq,hkv,num_seqs,max_q,ctx,split,paired,nb", [
     (24, 4, 4, 512, 512, 1, 1, 2),      # two rounds of single blocks, from 512 keys
     (24, 4, 4, 511, 511, 0, 0, 2),
