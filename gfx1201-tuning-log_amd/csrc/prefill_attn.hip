@@ -1053,17 +1053,24 @@ inline bool split_shape_exact(int gqa)
 }
 inline int split_blocks(int gqa) { return gqa <= 2 ? 4 / gqa : 1; }
 
-// Default shape per GQA.  The per-wave kernel runs short contexts and batches of short prompts, many
-// more workgroups than CUs, so unpaired blocks, longest first, beat pairs and larger waves (8 waves x 2
-// row-sets, unpaired, against what GQA 6 / 12 took before: 6 prompts of 37..900 after 200 75 -> 55 /
-// 131 -> 93 us, 8 of 600 74 -> 59 / 130 -> 94, 12 of 50..400 34 -> 32 / 59 -> 46, 200 tokens alone 13.4 ->
-// 13.5 / 18.6 -> 13.7).
-inline int choose_shape(int gqa)
+// Workgroups of the key-split kernel resident at once on a gfx950 part (256 CUs, one each).
+constexpr int kSplitRoundWorkgroups = 256;
+
+// Default shape per GQA of the per-wave kernel (short contexts and batches of short prompts).  From GQA 3 to 8 two
+// forms of 8 waves x 2 row-sets: paired blocks (7), whose workgroups all see the same keys, or consecutive ones
+// (2), longest first.  One round of workgroups ends with its longest, and pairs are shorter there (GQA 7: 200
+// tokens 13.4 against 14.5 us, 256 15.4 / 17.4; GQA 6 1.01 on average).  Past one round consecutive blocks fill
+// the last one and walk fewer tiles: GQA 6 0.90 of the time (6 prompts of 37..900 after 200 75 -> 55, 8 of 600
+// 74 -> 59), GQA 7 and 8 0.8 to 1.2 according to how full the last round is, which the host cannot
+// tell for unequal prompts (8 of 512 1.16, 3 of 100..700 1.19, 4 of 600 0.78; all measured 1.00), so they keep
+// pairs.  From GQA 9 on one block (GQA 12 against 4 waves x 4 row-sets: 131 -> 93, 8 of 600 130 -> 94).
+inline int choose_shape(int gqa, int n16, int hkv, int num_seqs)
 {
     if (g_shape >= 0 && g_shape < kNumShapes) return g_shape;
     if (gqa <= 1) return 5;                       // 4 waves x 1 row-set, 4 token blocks
     if (gqa <= 2) return 4;                       // 4 waves x 2 row-sets, 4 token blocks
-    return 2;                                     // 8 waves x 2 row-sets
+    if (gqa <= 8 && (gqa > 6 || (int64_t)((n16 + 1) / 2) * hkv * num_seqs < kSplitRoundWorkgroups)) return 7;
+    return 2;
 }
 
 inline int plan_nb(int gqa, const Shape& s)
@@ -1074,8 +1081,6 @@ inline int plan_nb(int gqa, const Shape& s)
     return nb;
 }
 
-// Workgroups of the key-split kernel resident at once on a gfx950 part (256 CUs, one each).
-constexpr int kSplitRoundWorkgroups = 256;
 
 // Token-block ranks per (sequence, kv head) padded for the XCD-aware grid (8 % HKV == 0).
 inline int split_xcd_per(int hkv) { return (hkv <= 8 && 8 % hkv == 0) ? 8 / hkv : 1; }
@@ -1174,7 +1179,7 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
         L.ntb_grid = round_up(L.paired ? (nsb + 1) / 2 : nsb);
         L.block = dim3(64 * kSplitWaves);
     } else {
-        L.shape = choose_shape(gqa);
+        L.shape = choose_shape(gqa, n16, hkv, num_seqs);
         const Shape sh = kShapes[L.shape];
         if (sh.waves * sh.rs < gqa) return FP8KV_ERR_SHAPE;
         L.nb = plan_nb(gqa, sh);

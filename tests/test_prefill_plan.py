@@ -125,13 +125,17 @@ def test_low_gqa_lines(lib, hq, hkv, num_seqs, max_q, ctx, split):
     (24, 4, 5, 512, 512, 0, 0, 2),      # a third round: per-wave kernel, unpaired
     (24, 4, 6, 900, 900, 0, 0, 2),
     (16, 2, 12, 768, 768, 1, 1, 2),     # GQA 8 splits the keys two ways: from 768
-    (16, 2, 12, 767, 767, 0, 0, 2),
+    (16, 2, 12, 767, 767, 0, 1, 2),
     (28, 4, 1, 320, 1000, 1, 0, 2),     # no shape of its own: from 320-token prompts
-    (28, 4, 1, 319, 1000, 0, 0, 2),
+    (28, 4, 1, 319, 1000, 0, 1, 2),
     (16, 16, 1, 1024, 1024, 1, 0, 4),   # GQA 1: four token blocks per workgroup
     (8, 4, 1, 1024, 1024, 1, 0, 2),     # GQA 2: two
     (8, 4, 1, 320, 320, 1, 0, 2),
-    (24, 4, 12, 400, 400, 0, 0, 2)])
+    (24, 4, 12, 400, 400, 0, 0, 2),
+    (24, 4, 1, 200, 200, 0, 1, 2),      # per-wave kernel, one round: paired
+    (24, 4, 9, 200, 200, 0, 1, 2), (24, 4, 10, 200, 200, 0, 0, 2),      # 252 workgroups, 280
+    (28, 4, 16, 256, 256, 0, 1, 2),     # GQA 7 and 8: paired at any count
+    (36, 4, 1, 100, 100, 0, 0, 1)])
 def test_plan_lines(lib, hq, hkv, num_seqs, max_q, ctx, split, paired, nb):
     """Both sides of the lines between the key-split and the per-wave kernel."""
     p = plan(lib, hq, hkv, num_seqs, max_q, ctx)
