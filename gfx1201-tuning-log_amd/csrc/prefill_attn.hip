@@ -1019,8 +1019,9 @@ prefill_split_kernel(Params P)
     }
 }
 
-// Launch shapes: (waves, row-sets per wave, ring depth).  nb token blocks of 16 per workgroup is
-// the largest count whose nb * GQA row-sets fit waves * RS.
+// Launch shapes: (waves, row-sets per wave, ring depth, paired blocks).  nb token blocks of 16 per workgroup is
+// the largest count whose nb * GQA row-sets fit waves * RS.  The plan takes 2, 4, 5 and 7 (choose_shape); 0, 1, 3 and 6
+// are there for sweeps through the tuning hook, which the figures of the others are measured against.
 struct Shape {
     int waves, rs, ring, paired;
 };
@@ -1117,11 +1118,13 @@ constexpr int kSplitMinContextFewParts = 768;
 // 36.5 and 37.8); GQA 3: single prompts only (8 of 600, 12 / 4, 36.7 and 56.0; 3 of 1500 0.79 of the time per wave, 6 of
 // 1400 0.88; one of 3000 1.47).
 constexpr int kSplitMinContextGqa1 = 1024, kSplitMinContextGqa2 = 640;
-// GQAs without a shape of their own (us, split against per wave; 2048 tokens after 2048, 28 / 4 heads 123 /
-// 194, 16 / 16 75 / 140, 8 / 4 49 / 132, 12 / 4 74 / 140, 20 / 4 93 / 187, 40 / 4 158 / 248; 1000 after 500, 28 / 4
-// 34 / 68, 16 / 16 22 / 48).  Prompts up to 300 tokens stay on the per-wave kernel, as the launch
-// plan's test has them, although contexts of 1000 keys would gain there too.
-constexpr int kSplitMinQueryInexact = 320;
+// GQAs without a shape of their own repeat row-sets or pack blocks (us, split against per wave; 2048 tokens after
+// 2048, 28 / 4 heads 123 / 194, 16 / 16 75 / 140, 8 / 4 49 / 132, 12 / 4 74 / 140, 20 / 4 93 / 187, 40 / 4 158 / 248; 1000
+// after 500, 28 / 4 34 / 68, 16 / 16 22 / 48).  Prompts of fewer than 320 tokens take it from 512 keys, where the host
+// knows the context (a prompt of 64 to 300 after 500 cached: GQA 1 0.50-0.63 of the time, 2 0.38-0.47, 3
+// 0.39-0.48, 7 0.51-0.55, 10 0.76-0.85; after 2048 0.29-0.67); alone they stand at 0.6-1.55 and after 100 at
+// 0.5-1.18, the lower the longer, and stay.
+constexpr int kSplitMinQueryInexact = 320, kSplitMinContextInexact = 512;
 constexpr int kSplitMinContextSingle = 256;
 // In one round of pairs: 512 (4 of 512, 24 / 4 heads: 26.6 us against 28.1 per wave, 48 / 4: 37 against 48).
 constexpr int kSplitMinContextPairs = 512;
@@ -1145,8 +1148,7 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
     const int per = split_xcd_per(hkv);                // token-block ranks per kv head per XCD round
     auto round_up = [&](int n) { return (n + per - 1) / per * per; };
 
-    // Key-split kernel when the GQA has a split shape and the context is long enough, unless the
-    // tuning hook forces another.
+    // Key-split kernel when the context is long enough for the GQA's shape, unless the tuning hook forces another.
     const int ss = split_shape_for(gqa), nbt = split_blocks(gqa);
     const bool exact = split_shape_exact(gqa);
     const int nsb = (max_query_len + 16 * nbt - 1) / (16 * nbt);        // the split kernel's (super)blocks
@@ -1165,7 +1167,7 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
                        : kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext;
         split = ctx_hint >= many || (ctx_hint >= kSplitMinContextSingle && fits) ||
                 (ctx_hint >= kSplitMinContextPairs && split_pairs_fit(nsb, hkv, num_seqs));
-        if (!exact && max_query_len < kSplitMinQueryInexact) split = false;
+        if (!exact && max_query_len < kSplitMinQueryInexact && ctx_hint < kSplitMinContextInexact) split = false;
     }
     if (split) {
         // Pairs of token blocks (r, n16 - 1 - r) give every workgroup the same causal work; when

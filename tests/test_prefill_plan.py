@@ -90,10 +90,10 @@ def test_forced_split_shape_other_gqa_uses_per_wave_kernel(tuned):
 
 
 @pytest.mark.parametrize("hq,hkv,qlen,ctx", [(24, 4, 200, 200), (24, 4, 128, 128),
-                                             (4, 4, 300, 5000), (28, 4, 197, 258)])
+                                             (4, 4, 300, 511), (28, 4, 197, 258)])
 def test_per_wave_plans(lib, hq, hkv, qlen, ctx):
-    """Short contexts and GQAs without a split shape (1, 7) take the per-wave kernel; every block
-    is covered."""
+    """Short contexts take the per-wave kernel, at GQAs without a key-split shape of their own (1, 7) those of
+    short prompts up to 511 keys; every block is covered."""
     p = plan(lib, hq, hkv, 1, qlen, ctx)
     assert p["split"] == 0
     check_cover(p, hkv, 1, (qlen + 15) // 16)
@@ -127,7 +127,9 @@ def test_low_gqa_lines(lib, hq, hkv, num_seqs, max_q, ctx, split):
     (16, 2, 12, 768, 768, 1, 1, 2),     # GQA 8 splits the keys two ways: from 768
     (16, 2, 12, 767, 767, 0, 1, 2),
     (28, 4, 1, 320, 1000, 1, 0, 2),     # no shape of its own: from 320-token prompts
-    (28, 4, 1, 319, 1000, 0, 1, 2),
+    (28, 4, 1, 319, 511, 0, 1, 2),
+    (28, 4, 1, 64, 512, 1, 0, 2),       # or from 512 keys
+    (4, 4, 1, 300, 5000, 1, 0, 4),
     (16, 16, 1, 1024, 1024, 1, 0, 4),   # GQA 1: four token blocks per workgroup
     (8, 4, 1, 1024, 1024, 1, 0, 2),     # GQA 2: two
     (8, 4, 1, 320, 320, 1, 0, 2),
