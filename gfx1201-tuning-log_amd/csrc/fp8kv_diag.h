@@ -95,6 +95,9 @@ void fp8kv_prefill_bf16_tune(int heads_per_wave);
 int fp8kv_prefill_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len,
                        int ctx_hint, int* out);
 
+/* The same for bf16 caches, as far as it has a choice: 1 where the key-split kernel takes the call. */
+int fp8kv_prefill_bf16_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len, int ctx_hint);
+
 /* Tuning hook for the MXFP4 x MXFP8 GEMM: kernel variant (0..19; any other value selects the
  * default, which picks from the shape; 9 + s is the K-splitting kernel with tile shape s, 19 variant 5
  * with two K groups of waves; K < 512 leaves those to the default; the per-token entry point runs

@@ -1101,6 +1101,12 @@ inline bool split_pairs_fit(int n16, int hkv, int num_seqs)
 {
     return split_workgroups((n16 + 1) / 2, hkv, num_seqs) <= kSplitRoundWorkgroups;
 }
+// Pairs that run a second round for an eighth of one or less.
+inline bool split_pairs_overflow(int n16, int hkv, int num_seqs)
+{
+    const int64_t w = split_workgroups((n16 + 1) / 2, hkv, num_seqs);
+    return w > kSplitRoundWorkgroups && w <= kSplitRoundWorkgroups + kSplitRoundWorkgroups / 8;
+}
 
 // Contexts (in keys) from which the key-split kernel beats the per-wave kernel, measured on MI355X.
 // With more single blocks than one round holds: 1024 (GQA 6: 3 of 300..1100 and longer; 6 of 37..900
@@ -1400,13 +1406,22 @@ extern "C" int fp8kv_prefill_attn_varlen(const void* q, int64_t q_row_stride,
 // prompts long enough to pay for it or a GQA whose shape splits the keys two ways or not at all (12
 // prompts of 50..400: 24 / 4 heads 49 us against 35, 28 / 4 40 against 45, 48 / 4 44 against 60; 64
 // tokens alone: 12.1 against 7.0; 300: 15.8 and 17.0; 6 of 37..900 after 200: 70 and 73).  For varlen
-// calls the host knows the longest prompt only and takes it for the context.
+// calls the host knows the longest prompt only and takes it for the context; cached tokens that it does not see
+// make the split worth more (40..300 at 28 / 4: 12 alone 34.1 us split against 29.2, 8 after 1500 76 against 167).  A single
+// prompt, whose context it knows, is left to the other kernel below 1700 keys where its pairs overflow one round by
+// an eighth or less and would run a second for them (1100 alone, 48 / 8: 63.9 against 57.5).
 bool fp8kv::prefill_split_takes_bf16(int hkv, int gqa, int num_seqs, int max_query_len, int ctx_hint)
 {
     if (ctx_hint < kSplitMinContextSingle) return false;
-    const int nb = split_blocks(gqa);
-    if (split_single_blocks_fit((max_query_len + 16 * nb - 1) / (16 * nb), hkv, num_seqs)) return true;
+    const int nb = split_blocks(gqa), n = (max_query_len + 16 * nb - 1) / (16 * nb);
+    if (split_single_blocks_fit(n, hkv, num_seqs)) return true;
+    if (num_seqs == 1 && ctx_hint < 1700 && split_pairs_overflow(n, hkv, 1)) return false;
     return ctx_hint >= 768 || gqa > 6;
+}
+
+extern "C" int fp8kv_prefill_bf16_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len, int ctx_hint)
+{
+    return prefill_split_takes_bf16(num_kv_heads, num_q_heads / num_kv_heads, num_seqs, max_query_len, ctx_hint) ? 1 : 0;
 }
 
 int fp8kv::launch_prefill_split_bf16(const fp8kv::PrefillBf16& A, bool force_paired, hipStream_t stream)

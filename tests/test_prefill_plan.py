@@ -144,3 +144,15 @@ def test_plan_lines(lib, hq, hkv, num_seqs, max_q, ctx, split, paired, nb):
     assert (p["split"], p["paired"], p["nb"]) == (split, paired, nb)
     blocks = (max_q + 15) // 16
     assert p["ntb"] * (2 * (nb if split and hq // hkv < 3 else 1) if p["paired"] else nb) >= blocks
+
+
+@pytest.mark.parametrize("hq,hkv,num_seqs,max_q,ctx,split", [
+    (24, 4, 1, 256, 256, 1), (24, 4, 1, 255, 255, 0), (24, 4, 6, 767, 767, 0), (24, 4, 6, 768, 768, 1),
+    (48, 4, 12, 320, 320, 1), (28, 4, 12, 300, 300, 1), (24, 4, 3, 768, 768, 1),
+    (48, 8, 1, 1024, 1024, 1),                                          # 256 pairs
+    (48, 8, 1, 1040, 1040, 0), (48, 8, 1, 1100, 1699, 0), (48, 8, 1, 1100, 1700, 1), (48, 8, 1, 1152, 1152, 0),
+    (48, 8, 1, 1168, 1168, 1)])                                         # 288, 296
+def test_bf16_plan_lines(lib, hq, hkv, num_seqs, max_q, ctx, split):
+    """The lines of the key-split kernel over bf16 caches, and the single prompts whose pairs overflow one
+    round by an eighth or less."""
+    assert lib.fp8kv_prefill_bf16_plan(hq, hkv, num_seqs, max_q, ctx) == split
