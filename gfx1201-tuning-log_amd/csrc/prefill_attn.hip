@@ -1119,11 +1119,14 @@ constexpr int kSplitMinContext = 1024;
 // 48 / 98 / 72 against 46 / 94 / 59).
 constexpr int kSplitMinContextFewParts = 768;
 // Below GQA 4 the per-wave kernel has few row-sets to share a conversion, but its workgroups are small: past one
-// round of pairs it is the split kernel that runs a second, partly empty one.  GQA 1: from 1024 keys (5 of 512,
-// 16 / 16 heads, in two rounds 33.5 us per wave and 35.9 split, 8 of 320..520 31 and 37); GQA 2: 640 (8 of 600, 8 / 4,
-// 36.5 and 37.8); GQA 3: single prompts only (8 of 600, 12 / 4, 36.7 and 56.0; 3 of 1500 0.79 of the time per wave, 6 of
-// 1400 0.88; one of 3000 1.47).
-constexpr int kSplitMinContextGqa1 = 1024, kSplitMinContextGqa2 = 640;
+// round of pairs it is the split kernel that runs another, partly empty one.  GQA 1 and 3, several prompts (fresh /
+// after 1500 cached tokens, which the host does not see and which make the split worth more; time split against
+// per wave): up to two rounds from 640 and 768 keys (16 / 16 heads, 4 of 100..700 0.71 / 0.49, 5 of 768 0.92 /
+// 0.62; 12 / 4, 3 of 120..900 0.58 / 0.54, 5 of 768 1.13 / 1.05), except where a round overflows by an eighth or less
+// (3 of 768: 1.27 / 0.89 and 1.44 / 0.93); past two, GQA 1 from 1024 (6 of 200..1400 0.95 / 0.75) and GQA 3 not at
+// all (8 of 600 1.53, 6 of 1400 1.14, 3 of 1500 1.27).  GQA 2 from 512 (8 of 600 1.04 / 0.58).
+constexpr int kSplitMinContextGqa1 = 640, kSplitMinContextGqa1Long = 1024, kSplitMinContextGqa2 = 512;
+constexpr int kSplitMinContextGqa3 = 768;
 // GQAs without a shape of their own repeat row-sets or pack blocks (us, split against per wave; 2048 tokens after
 // 2048, 28 / 4 heads 123 / 194, 16 / 16 75 / 140, 8 / 4 49 / 132, 12 / 4 74 / 140, 20 / 4 93 / 187, 40 / 4 158 / 248; 1000
 // after 500, 28 / 4 34 / 68, 16 / 16 22 / 48).  Prompts of fewer than 320 tokens take it from 512 keys, where the host
@@ -1168,9 +1171,12 @@ int plan_launch(int gqa, int hkv, int num_seqs, int max_query_len, int ctx_hint,
             force_paired = g_shape > kSplitAnyShape;
         }
     } else if (g_shape < 0) {
-        const int many = gqa == 1 ? kSplitMinContextGqa1 : gqa == 2 ? kSplitMinContextGqa2
-                       : gqa == 3 && num_seqs > 1 ? INT32_MAX
-                       : kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext;
+        const bool two_rounds = split_workgroups((nsb + 1) / 2, hkv, num_seqs) <= 2 * kSplitRoundWorkgroups;
+        int many = gqa == 1 ? (two_rounds ? kSplitMinContextGqa1 : kSplitMinContextGqa1Long)
+                 : gqa == 2 ? kSplitMinContextGqa2
+                 : gqa == 3 && num_seqs > 1 ? (two_rounds ? kSplitMinContextGqa3 : INT32_MAX)
+                 : kSplitShapes[ss].ng >= 4 ? kSplitMinContextFewParts : kSplitMinContext;
+        if ((gqa == 1 || gqa == 3) && many < kSplitMinContext && split_pairs_overflow(nsb, hkv, num_seqs)) many = kSplitMinContext;
         split = ctx_hint >= many || (ctx_hint >= kSplitMinContextSingle && fits) ||
                 (ctx_hint >= kSplitMinContextPairs && split_pairs_fit(nsb, hkv, num_seqs));
         if (!exact && max_query_len < kSplitMinQueryInexact && ctx_hint < kSplitMinContextInexact) split = false;

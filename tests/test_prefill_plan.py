@@ -108,11 +108,12 @@ def test_empty_and_invalid(lib):
 
 
 @pytest.mark.parametrize("hq,hkv,num_seqs,max_q,ctx,split", [
-    (16, 16, 2, 1000, 1000, 1), (16, 16, 5, 1000, 1000, 0), (16, 16, 5, 1024, 1024, 1),     # GQA 1
+    (16, 16, 4, 639, 639, 0), (16, 16, 4, 640, 640, 1), (16, 16, 3, 768, 768, 0),       # GQA 1; 288 pairs
+    (16, 16, 8, 700, 700, 0), (16, 16, 8, 1023, 1023, 0), (16, 16, 8, 1024, 1024, 1),   # past two rounds
     (4, 4, 12, 512, 512, 1), (4, 4, 12, 600, 600, 0),                   # 5 pairs of superblocks, rounded to 6: 288
-    (8, 4, 8, 600, 600, 0), (8, 4, 8, 640, 640, 1), (8, 4, 5, 600, 600, 1),                 # GQA 2
-    (12, 4, 4, 512, 512, 1), (12, 4, 4, 600, 600, 0), (12, 4, 3, 1500, 1500, 0),            # GQA 3
-    (12, 4, 1, 3000, 3000, 1), (12, 4, 8, 320, 320, 0)])
+    (8, 4, 8, 511, 511, 0), (8, 4, 8, 600, 600, 1),                                     # GQA 2
+    (12, 4, 4, 512, 512, 1), (12, 4, 4, 600, 600, 0), (12, 4, 4, 767, 767, 0), (12, 4, 4, 768, 768, 1),  # GQA 3
+    (12, 4, 3, 768, 768, 0), (12, 4, 3, 1500, 1500, 0), (12, 4, 1, 3000, 3000, 1), (12, 4, 8, 320, 320, 0)])
 def test_low_gqa_lines(lib, hq, hkv, num_seqs, max_q, ctx, split):
     """Below GQA 4 the key-split kernel takes one round of single blocks or of pairs, and beyond it only the
     contexts that pay for a second, partly empty one."""
