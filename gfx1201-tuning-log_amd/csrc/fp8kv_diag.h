@@ -106,6 +106,10 @@ int fp8kv_prefill_bf16_plan(int num_q_heads, int num_kv_heads, int num_seqs, int
  * count allows).  Affects later launches. */
 void fp8kv_gemm_tune(int variant, int order);
 
+/* Kernel variant (as for fp8kv_gemm_tune) that h4a8_gemm, or h4a8_gemm_token with `token`, runs for this
+ * shape under the current tuning hook.  Host only. */
+int fp8kv_gemm_plan(int N, int K, int M, int token);
+
 /* Measurement hook: the next kernel launched by this host thread through any entry point records
  * start_event / stop_event (hipEvent_t, either may be NULL) at its own start and end, via
  * hipExtLaunchKernel.  hipEventElapsedTime between them is then the kernel's execution time.

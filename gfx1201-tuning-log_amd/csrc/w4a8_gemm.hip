@@ -85,12 +85,18 @@ inline int one_round_split(int nblk, int mblk, int N, int K, int M)
 // tile that fits is the fastest: its waves have the fewest bytes to fetch (in a graph, per-token
 // activations, us against the 128 x 128 or 256 x 128 kernel; N = 4096, K = 3584: 17 rows 5.2 / 20.1,
 // 64 6.7 / 20.4, 128 8.1 / 21.2, 256 10.7 / 21.4, 512 15.6 / 21.8; N = 3584, K = 18944: 17 rows 16.3 /
-// 104.5, 128 28.2 / 111.8, 512 55.9 / 113.4).  Past one round the larger tiles' smaller traffic wins (N = 37888,
-// K = 3584: 64 rows 38.0 / 32.2; N = 4096: 1000 rows 28.7 / 23.9).
+// 104.5, 128 28.2 / 111.8, 512 55.9 / 113.4; N = 28672, K = 4096, a 128 x 64 tile up to 64 rows: 17 rows 18.6 /
+// 23.3, 64 20.6 / 24.5).  Past one round the larger tiles' smaller traffic wins (N = 37888, K = 3584: 64 rows 38.0 /
+// 32.2; N = 4096: 1000 rows 28.7 / 23.9).  The two largest tiles need steps enough for their four waves: at K = 512,
+// 640 and 768 they take 1.00-1.13 of the time of the 128 x 128 kernel, at 1024 0.90-0.98 (N = 2048, MXFP8, 700 rows
+// 8.2 / 7.4 us at K = 640).
+constexpr int kSliceLargeTile = 8;                     // first of kSliceShapes with a 128 side
+constexpr int kSliceLargeMinK = 1024;
 inline int slice_shape(int N, int K, int M)
 {
     if (K < kSliceMinK) return -1;
     for (int s = 0; s < kNumSliceShapes; ++s) {
+        if (s >= kSliceLargeTile && K < kSliceLargeMinK) break;
         const int bn = 16 * kSliceShapes[s].tn, bm = 16 * kSliceShapes[s].tm;
         const int64_t nblk = ((int64_t)N + bn - 1) / bn, mblk = ((int64_t)M + bm - 1) / bm;
         if (nblk * mblk <= kGemmCus && one_round_split((int)nblk, (int)mblk, N, K, M) > 0) return s;
@@ -1210,6 +1216,12 @@ extern "C" int h4a8_gemm_token(const void* W, const void* St, const void* Xq, co
     int variant = pick_variant(N, K, M);
     if (!has_token_variant(variant)) variant = default_variant(N, K, M);
     return launch_gemm(P, variant, true, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int fp8kv_gemm_plan(int N, int K, int M, int token)
+{
+    const int variant = pick_variant(N, K, M);
+    return token && !has_token_variant(variant) ? default_variant(N, K, M) : variant;
 }
 
 extern "C" void fp8kv_gemm_tune(int variant, int order)

@@ -90,6 +90,7 @@ SIGNATURES: dict[str, tuple] = {
     "fp8kv_prefill_plan": (_c_i, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_vp]),
     "fp8kv_prefill_bf16_plan": (_c_i, [_c_i] * 5),
     "fp8kv_gemm_tune": (None, [_c_i, _c_i]),
+    "fp8kv_gemm_plan": (_c_i, [_c_i] * 4),
     "fp8kv_time_next_launch": (None, [_c_vp, _c_vp]),
 }
 
