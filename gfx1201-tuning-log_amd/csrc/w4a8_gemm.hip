@@ -56,8 +56,8 @@ thread_local int g_gemm_variant = kDefaultVariant;
 constexpr int64_t kGemmCus = 256;
 // 9 + s: the K-splitting kernel (w4a8_slice.hip) with tile shape s of kSliceShapes.
 constexpr int kSliceVariant = 9;
-// 19: variant 5's tiles with two K groups of waves (K % 512 == 0 and scales as for the grouped copies;
-// variant 5 itself otherwise).  Variant 5 takes it on its own where one_round_split gives every tile a CU.
+// 19: variant 5's tiles with two K groups of waves (K % 512 == 0, K >= 1024 and scales as for the grouped copies;
+// variant 5 itself otherwise).  The default takes it where one_round_split gives every tile a CU.
 constexpr int kKGroupsVariant = kSliceVariant + kNumSliceShapes;
 
 constexpr int kCusPerXcd = 32;
@@ -109,7 +109,13 @@ inline int default_variant(int N, int K, int M)
     const int s = slice_shape(N, K, M);
     if (s >= 0) return kSliceVariant + s;
     const int64_t tiles6 = (int64_t)((N + 255) / 256) * ((M + 127) / 128);
-    return tiles6 > kGemmCus ? 6 : 5;
+    if (tiles6 > kGemmCus) return 6;
+    // 128 x 128 tiles, at most one per CU: K groups (in a graph, per-token, us: N = 3584, K = 18944, 1000
+    // rows 98.7 -> 81.7; N = 4096, K = 3584 24.3 -> 21.3; past one round the workgroups pair up by
+    // themselves: 1500 rows 118 / 157)
+    const bool kgroups = K % 512 == 0 && K >= 2 * kSliceMinK &&
+                         one_round_split((N + kBN - 1) / kBN, (M + kBM - 1) / kBM, N, K, M) > 0;
+    return kgroups ? kKGroupsVariant : 5;
 }
 
 // A forced slice shape needs kSliceMinK like a planned one.
@@ -1029,7 +1035,7 @@ int launch_gemm(Params& P, int variant, bool tok, hipStream_t st)
         P.nblk = (P.N + 16 * sh.tn - 1) / (16 * sh.tn);
         P.mblk = (P.M + 16 * sh.tm - 1) / (16 * sh.tm);
         if ((int64_t)P.nblk * P.mblk > 0x7FFFFFFF - kXcds) return FP8KV_ERR_SHAPE;
-        const int one = one_round_split(P.nblk, P.mblk, P.N, P.K, P.M);
+        const int one = g_gemm_order == 0 ? one_round_split(P.nblk, P.mblk, P.N, P.K, P.M) : 0;
         P.gm = one > 0 ? one : pick_split(P, 16 * sh.tm, kLdsPerCu, !tok);
         P.gn = kXcds / P.gm;
         const int64_t per = (int64_t)((P.mblk + P.gm - 1) / P.gm) * ((P.nblk + P.gn - 1) / P.gn);
@@ -1055,12 +1061,9 @@ int launch_gemm(Params& P, int variant, bool tok, hipStream_t st)
                   : variant == 2 || variant == 4 ? (gs ? LdsGeom<2, 2, 3>::lds_gs(tok) : LdsGeom<2, 2, 3>::LDS)
                   : variant == 3 ? (gs ? LdsGeom<2, 2, 5>::lds_gs(tok) : LdsGeom<2, 2, 5>::LDS)
                   : (gs ? LdsGeom<2, 2, 2>::lds_gs(tok) : LdsGeom<2, 2, 2>::LDS);
-    // 128 x 128 tiles, at most one per CU: K groups (in a graph, per-token, us: N = 3584, K = 18944, 1000
-    // rows 98.7 -> 81.7; N = 4096, K = 3584 24.3 -> 21.3; past one round the workgroups pair up by
-    // themselves: 1500 rows 118 / 157)
-    const int one = one_round_split(P.nblk, P.mblk, P.N, P.K, P.M);
-    const bool kgroups = gs && P.K >= 2 * kSliceMinK && (variant == kKGroupsVariant || (variant == 5 && one > 0));
-    const int gm = kgroups && one > 0 ? one : pick_split(P, BM, lds, !tok);
+    const bool kgroups = gs && P.K >= 2 * kSliceMinK && variant == kKGroupsVariant;
+    const int one = kgroups && g_gemm_order == 0 ? one_round_split(P.nblk, P.mblk, P.N, P.K, P.M) : 0;
+    const int gm = one > 0 ? one : pick_split(P, BM, lds, !tok);
     P.gm = gm;
     P.gn = kXcds / gm;
     const int64_t per_xcd = (int64_t)((P.mblk + gm - 1) / gm) * ((P.nblk + P.gn - 1) / P.gn);

@@ -189,8 +189,8 @@ def _random_shapes(n, seed):
 @pytest.mark.parametrize("N,K,M", _random_shapes(12, 2026))
 @pytest.mark.parametrize("act", ["mx", "token"])
 def test_gemm_random_shapes(N, K, M, act):
-    """Seeded random shapes through the default planner (every tile size, ring, XCD split and the
-    grouped scale copies where K % 512 == 0), against the oracle."""
+    """Seeded random shapes through the default planner, against the oracle: small enough that most take the
+    K-splitting kernel (test_default_plans covers the others)."""
     if act == "token":
         c, rc, rs = _token_case(N, K, M, seed=N + K + M)
         out = ops.h4a8_gemm_token(torch.from_numpy(rc).to(DEV), torch.from_numpy(rs).to(DEV), c["W"].to(DEV),
@@ -202,6 +202,31 @@ def test_gemm_random_shapes(N, K, M, act):
                             c["St"].to(DEV))
         ref = w4a8.gemm(c["W"].numpy(), c["St"].numpy(), rc, rs)
     torch.cuda.synchronize()
+    assert matvec.bf16_excess_error(out.float().cpu().numpy(), ref) < 1e-4
+
+
+@pytest.mark.parametrize("act", ["mx", "token"])
+@pytest.mark.parametrize("N,K,M,order,plan", [
+    (3584, 1536, 1100, 0, 5), (3584, 1536, 1100, 1, 5), (3588, 2048, 1090, 2, 5), (3584, 1152, 1000, 0, 5),
+    (8196, 1536, 1030, 0, 6), (8192, 1152, 1100, 1, 6), (3584, 1536, 1000, 0, 19), (3588, 2560, 900, 1, 19)])
+def test_default_plans(N, K, M, order, plan, act):
+    """The kernels that the planner picks past the K-splitting one, each at a shape of its own: 128 x 128 tiles over
+    more than one round (grouped scale copies over 3 and 4 scale groups, which wrap their ring, and per-step
+    ones), 256 x 128 tiles, K groups of unequal halves (5 scale groups: 3 and 2), partial tiles, the three XCD
+    splits, and the repeat of a call bit for bit."""
+    lib = _lib.load()
+    c, rc, rs = (_token_case if act == "token" else _gemm_case)(N, K, M, seed=N + M)
+    ref = (w4a8.gemm_token if act == "token" else w4a8.gemm)(c["W"].numpy(), c["St"].numpy(), rc, rs)
+    args = [torch.from_numpy(rc).to(DEV), torch.from_numpy(rs).to(DEV), c["W"].to(DEV), c["St"].to(DEV)]
+    gemm = ops.h4a8_gemm_token if act == "token" else ops.h4a8_gemm
+    try:
+        lib.fp8kv_gemm_tune(-1, order)
+        assert lib.fp8kv_gemm_plan(N, K, M, int(act == "token")) == plan
+        out, again = gemm(*args).clone(), gemm(*args)
+        torch.cuda.synchronize()
+    finally:
+        lib.fp8kv_gemm_tune(-1, 0)
+    assert torch.equal(out, again)
     assert matvec.bf16_excess_error(out.float().cpu().numpy(), ref) < 1e-4
 
 
