@@ -95,7 +95,8 @@ void fp8kv_prefill_bf16_tune(int heads_per_wave);
 int fp8kv_prefill_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len,
                        int ctx_hint, int* out);
 
-/* The same for bf16 caches, as far as it has a choice: 1 where the key-split kernel takes the call. */
+/* The same for bf16 caches, as far as it has a choice: 1 where the key-split kernel takes the call (0 for a
+ * shape that the entry points refuse). */
 int fp8kv_prefill_bf16_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len, int ctx_hint);
 
 /* Tuning hook for the MXFP4 x MXFP8 GEMM: kernel variant (0..19; any other value selects the

@@ -1427,6 +1427,8 @@ bool fp8kv::prefill_split_takes_bf16(int hkv, int gqa, int num_seqs, int max_que
 
 extern "C" int fp8kv_prefill_bf16_plan(int num_q_heads, int num_kv_heads, int num_seqs, int max_query_len, int ctx_hint)
 {
+    if (num_q_heads < 1 || num_kv_heads < 1 || num_seqs < 1 || max_query_len < 0) return 0;
+    if (num_q_heads % num_kv_heads != 0 || num_q_heads / num_kv_heads > kMaxGqa) return 0;
     return prefill_split_takes_bf16(num_kv_heads, num_q_heads / num_kv_heads, num_seqs, max_query_len, ctx_hint) ? 1 : 0;
 }
 

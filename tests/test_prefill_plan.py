@@ -157,3 +157,9 @@ def test_bf16_plan_lines(lib, hq, hkv, num_seqs, max_q, ctx, split):
     """The lines of the key-split kernel over bf16 caches, and the single prompts whose pairs overflow one
     round by an eighth or less."""
     assert lib.fp8kv_prefill_bf16_plan(hq, hkv, num_seqs, max_q, ctx) == split
+
+
+@pytest.mark.parametrize("hq,hkv,num_seqs,max_q", [(24, 0, 1, 300), (0, 4, 1, 300), (4, 8, 1, 300), (10, 4, 1, 300),
+                                                   (68, 4, 1, 300), (24, 4, 0, 300), (24, 4, 1, -1)])
+def test_bf16_plan_of_a_refused_shape(lib, hq, hkv, num_seqs, max_q):
+    assert lib.fp8kv_prefill_bf16_plan(hq, hkv, num_seqs, max_q, 4096) == 0
