@@ -522,8 +522,9 @@ inline int worth_splits(int len)
 // pay (24 / 4 heads, one sequence, us: 129 tokens 5.1 in one split and 5.3 in four, 256 6.2 and 5.2; 400 6.2 in
 // four, 5.8 in eight; 777 and 1024 6.5 and 6.7 in eight, 6.5 in 16; 5000 10.5 in 16 and in 32, 6144 11.2 and 11.1,
 // 8192 12.8 and 12.3, 12000 17.3 and 13.8; three sequences, whose 12 pairs leave room for 21, 6144: 11.9 in 16, 13.7
-// in 21; six, of 1024: 7.4 in eight, 8.0 in ten).  Counts that do not divide the CUs are rounded down up to 512 tokens a split (unequal contexts, 1 to 8: 0.67-1.0
-// of the time there, to 1.15 above; 10 of 512..4096, 4 kv heads: 16.8 in six, 14.3 in seven).
+// in 21; six, of 1024: 7.4 in eight, 8.0 in ten).  Counts that do not divide the CUs are rounded down up to 512
+// tokens a split (unequal contexts, 1 to 8: 0.67-1.0 of the time there, to 1.15 above; 10 of 512..4096, 4 kv
+// heads: 16.8 in six, 14.3 in seven).
 inline int worth_splits_bf16(int len)
 {
     return len <= 176 ? 1 : len <= 352 ? 4 : len <= 768 ? 8 : len <= 5632 ? 16 : kMaxPlannedSplits;

@@ -430,14 +430,16 @@ prefill_kernel(Params P)
 }
 
 // ---- key-split kernel ---------------------------------------------------------------------------
-// For a GQA that splits into NG groups of RS heads (gqa = NG * RS, RS row-sets per wave): a
-// workgroup of 8 waves owns the pair of 16-token blocks (r, n16 - 1 - r) of one kv head and
-// processes them one after the other, the longer first.  For one block, wave w takes head group
+// NG groups of RS row-sets, the smallest of kSplitShapes that holds the heads of the GQA: where they do not
+// fill it (GQA 3, 5, 7, 9-11, 13-15) the last one is repeated and not stored, and at GQA 1 and 2 the
+// row-sets are those of 4 and 2 consecutive token blocks (MB).  A workgroup of 8 waves owns one such block of
+// one kv head, or the pair (r, n - 1 - r) of them where single ones overflow a round of workgroups; it takes
+// the longer of a pair first.  For one block, wave w takes row-set group
 // w / NR and, of every window of NR x TPW key tiles (NR = 8 / NG), the TPW tiles of residue
 // w % NR: every wave converts each of its tiles once for RS row-sets, and two waves share each
 // SIMD.  The ring holds two windows; window i + 1 is copied (each wave issuing one 1 KB copy of
-// every tile) while window i is consumed, and one barrier per window publishes it.  At the end
-// of a block the NR partial (m, l, o) states of each head group merge in LDS in a fixed order:
+// every e4m3 tile, two of a bf16 one) while window i is consumed, and one barrier per window publishes it.
+// At the end of a block the NR partial (m, l, o) states of each group merge in LDS in a fixed order:
 // the common max first, then row-set j in the wave of residue j % NR, which normalises and writes it.
 constexpr int kSplitWaves = 8;
 
@@ -456,7 +458,7 @@ constexpr float kMinFactor = 1e-37f, kMinFactor16 = 1.4e-45f;
 constexpr float kMaxFactor = 1073741824.f / (256.f * 448.f * 128.f);
 
 // max without the NaN-quieting canonicalisation the compiler adds to fmaxf of values that come
-// from MFMA results or lane swaps (the scores are never NaN: finite fp8 and bf16 inputs).
+// from MFMA results or lane swaps (finite K and Q give no NaN score; that of a scale joins at the output).
 __device__ __forceinline__ float max_raw(float a, float b)
 {
     float r;
@@ -724,11 +726,11 @@ prefill_split_kernel(Params P)
         // row n).  e4m3 caches: split into e4m3 hi + lo parts (q_fp8_split has the bound), the row's scale
         // folded into this lane's softmax factor qkr.  The split is about 270 VALU a row-set, and the
         // NR residues of a head group need the same ones, so each row-set is split by one wave and
-        // handed over through the LDS (the ring's second window is free until the key loop's first barrier)
-        // (with the merge by row-sets, 24 / 4 heads: 2048 tokens
-        // after 2048 102.1 -> 95.3 us, 1000 after 500 31.5 -> 27.7, 8 of 600 95 -> 72).  bf16 caches: the
-        // four bf16 fragments, loaded by each wave.  Window 0's block ids and the query rows are
-        // requested together, ahead of the window's copies (the asm takes the rows, so the compiler waits there and not behind the copies).
+        // handed over through the LDS (the ring's second window is free until the key loop's first
+        // barrier).  With the merge by row-sets, 24 / 4 heads: 2048 tokens after 2048 102.1 -> 95.3 us, 1000
+        // after 500 31.5 -> 27.7, 8 of 600 95 -> 72.  bf16 caches: the four bf16 fragments, loaded by each
+        // wave.  Window 0's block ids and the query rows are requested together, ahead of the window's
+        // copies (the asm takes the rows, so the compiler waits there and not behind the copies).
         static_assert(RW == 2, "one window is copied ahead");
         auto load_query = [&](u32x4_t (&qf)[4], int tok, int head) {
             const u32x4_t zero = {0u, 0u, 0u, 0u};
@@ -1124,7 +1126,10 @@ constexpr int kSplitMinContextFewParts = 768;
 // per wave): up to two rounds from 640 and 768 keys (16 / 16 heads, 4 of 100..700 0.71 / 0.49, 5 of 768 0.92 /
 // 0.62; 12 / 4, 3 of 120..900 0.58 / 0.54, 5 of 768 1.13 / 1.05), except where a round overflows by an eighth or less
 // (3 of 768: 1.27 / 0.89 and 1.44 / 0.93); past two, GQA 1 from 1024 (6 of 200..1400 0.95 / 0.75) and GQA 3 not at
-// all (8 of 600 1.53, 6 of 1400 1.14, 3 of 1500 1.27).  GQA 2 from 512 (8 of 600 1.04 / 0.58).
+// all (8 of 600 1.53, 6 of 1400 1.14, 3 of 1500 1.27).  GQA 2 from 512 (8 of 600 1.04 / 0.58).  The price is the
+// unequal prompts after long contexts below the lines, which the split kernel would run in half the time (5 of
+// 100..512 after 1500: 49 against 93 us at 16 / 16 heads, 83 at 12 / 4); the host cannot tell them from equal fresh
+// ones, and their tokens do not either.
 constexpr int kSplitMinContextGqa1 = 640, kSplitMinContextGqa1Long = 1024, kSplitMinContextGqa2 = 512;
 constexpr int kSplitMinContextGqa3 = 768;
 // GQAs without a shape of their own repeat row-sets or pack blocks (us, split against per wave; 2048 tokens after

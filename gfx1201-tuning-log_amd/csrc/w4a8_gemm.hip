@@ -46,8 +46,9 @@ constexpr int kBN = 128, kBM = 128;
 // the configs[4] linears at M = 2048: 6 ~1.22-1.69 PFLOP/s, 5 ~1.27-1.41, 8 ~0.88-1.67 (only
 // gate/up fills the GPU), 7 ~1.05-1.27, 4 ~1.33, 0 ~1.01, 1 ~0.40.
 // Default (-1): the K-splitting kernel where its tiles fit one round (slice_shape); else variant 6 (the
-// 8 x 4 wave tile, 256 x 128 per workgroup) when its grid has more tiles than the GPU has CUs, else
-// variant 5 (128 x 128, twice the workgroups).  With one workgroup per CU, variant 6 has one wave per SIMD and nothing hides its waits.  Measured at
+// 8 x 4 wave tile, 256 x 128 per workgroup) when its grid has more tiles than the GPU has CUs, else 128 x 128
+// tiles, twice the workgroups: with two K groups of waves (19) where every tile has a CU of its own, else
+// variant 5.  With one workgroup per CU, variant 6 has one wave per SIMD and nothing hides its waits.  Measured at
 // M = 2048 (MXFP8, us per launch, variant 5 against 6): 224 tiles of 256 x 128 (down, K = 18944)
 // 150 against 184, 256 tiles (qkv) 36 against 45, 384 tiles 58-59 against 56-57, 512 tiles 68
 // against 60, 1024 tiles 131 against 116, gate/up (2368 tiles) 323 against 285.
